@@ -37,10 +37,10 @@ int mvmc_abi_version(void);
  * (lib.rs:12-15).  The results are BatchedEngine::run_f64's BatchOutput<f64>
  * = (pf, inv, status).  All pointers are device pointers; `stream` is a
  * hipStream_t (NULL = default stream).  Asynchronous on `stream`.
- * n <= 64 and 152 <= n <= 224: one plane per workgroup held in registers
- * (256 threads for n <= 64, 1024 above); other n: the panel-delayed kernel
- * (several planes per workgroup through a global work buffer), whichever
- * measured faster at that size; MVMC_PFINV_RR=0 selects the latter for
+ * n <= 104: one plane per wave, held in LDS; n <= 224: one plane per four
+ * waves, held in registers; larger n: the panel-delayed kernel (several
+ * planes per workgroup through a global work buffer).  MVMC_PFINV_RR=0
+ * selects the latter for
  * every n.  Both give the same bits. */
 int mvmc_pfinv_f64(const double* planes, int n, int count, double* pf, double* inv, int* status, void* stream);
 
@@ -72,9 +72,10 @@ int mvmc_pfinv_f64_noalloc(const double* planes, int n, int count, double* pf, d
  * order 1: zsktf2_c_compat (ltl.rs:54-59, the order of the production
  * calc_m_all_complex, crates/mvmc-core/src/pfaffian.rs:383-398).
  * inv == planes factorises in place.  Device pointers; asynchronous on
- * `stream` (NULL = default stream).  n <= 160: one plane per workgroup held
- * in registers; larger n: one plane per 256-lane workgroup through a global
- * work plane (MVMC_PFINV_RR=0 selects the latter for every n); same bits. */
+ * `stream` (NULL = default stream).  n <= 64: one plane per wave, held in
+ * LDS; n <= 160: one plane per four waves, held in registers; larger n: one
+ * plane per 256-lane workgroup through a global work plane (MVMC_PFINV_RR=0
+ * selects the latter for every n); same bits. */
 int mvmc_pfinv_c128(const double* planes, int n, int count, int order, double* pf, double* inv, int* status,
                     void* stream);
 
@@ -222,10 +223,10 @@ int mvmc_ens_get_cg(mvmc_ens* e, double* solution, int* n_active);
  * and of its measurement launches, samples it measured; device ms of the
  * last SR call's CG solve, its iterations, active parameters, sample rows
  * (HIP events on the library's stream); the rebuild-kernel variant in use
- * (-1 while it is being measured; 0: three workgroups per CU, 8-column
- * panel-close batches; 1: two per CU, 16 columns; 2: register-resident,
- * one 1024-thread workgroup per CU, 64 < n <= 224) and the device ms per
- * rebuilt walker measured for variants 0, 1 and 2; device ms of the last
+ * (2: plane by plane with the kernels of mvmc_pfinv_f64, n <= 224; larger n:
+ * -1 while it is being measured, 0: three workgroups per CU, 8-column
+ * panel-close batches, 1: two per CU, 16 columns) and the device ms per
+ * rebuilt walker measured for variants 0 and 1, one reserved; device ms of the last
  * mvmc_ens_vjp_adjoint call and of its plane rebuilds; device ms of the
  * last direct SR's Gram kernel; passes of the last sampling call's k_block
  * launches that wrote a walker's inverse planes back (every second accepted

@@ -27,19 +27,47 @@ def _run(cmd):
     subprocess.run(cmd, check=True)
 
 
+# Translation units of the library: (source, macros).  The Pfaffian kernels
+# come in parts (ranges of plane sizes) so that their instances compile side
+# by side; the longest object sets the build's time.
+UNITS = [("csrc/capi.hip", ()), ("host/model.cpp", ())] + \
+    [("csrc/rr_planes.hip", (f"RR_PART={k}",)) for k in range(4)] + \
+    [("csrc/rr_planes_c128.hip", (f"RR_PART={k}",)) for k in range(2)]
+
+
+def object_command(src, macros, obj):
+    return [HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++20", "-fPIC", "-ffp-contract=off",
+            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+            "-Wno-unused-result"] + [f"-D{d}" for d in macros] + ["-c", "-o", obj, os.path.join(HERE, src)]
+
+
+def link_command(objs, out):
+    return [HIPCC, f"--offload-arch={ARCH}", "-fPIC", "-shared", "-o", out] + objs + \
+        ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
+
+
 def build_library(defines=(), out=None):
     """defines: extra -D macros (MVMC_PHASE_CLOCKS adds the sampling kernel's
     phase clocks); out: output path (default mvmc-rs_amd/_build/libmvmc_hip.so)."""
     out = out or LIB
     os.makedirs(os.path.dirname(out), exist_ok=True)
-    srcs = [os.path.join(HERE, "csrc", "capi.hip"), os.path.join(HERE, "host", "model.cpp")]
+    jobs = []
+    for k, (src, macros) in enumerate(UNITS):
+        obj = f"{out}.{k}.o"
+        cmd = object_command(src, tuple(macros) + tuple(defines), obj)
+        print("+", " ".join(cmd), flush=True)
+        jobs.append((obj, cmd, subprocess.Popen(cmd)))
+    for _, cmd, p in jobs:
+        if p.wait() != 0:
+            for _, _, other in jobs:
+                other.wait()
+            raise subprocess.CalledProcessError(p.returncode, cmd)
+    objs = [obj for obj, _, _ in jobs]
     tmp = out + ".tmp"
-    cmd = [HIPCC, f"--offload-arch={ARCH}", "-O3", "-std=c++20", "-fPIC", "-shared", "-ffp-contract=off",
-           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-           "-Wno-unused-result"] + [f"-D{d}" for d in defines] + ["-o", tmp] + srcs + \
-          ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
-    _run(cmd)
+    _run(link_command(objs, tmp))
     os.replace(tmp, out)
+    for obj in objs:
+        os.remove(obj)
     return out
 
 

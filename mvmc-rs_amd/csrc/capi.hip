@@ -7,6 +7,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -24,7 +25,8 @@
 #include "../host/model.h"
 #include "ensemble.hip"
 #include "pfinv_c128_dev.h"
-#include "pfinv_rr_c128.h"
+#include "pfinv_lds.h"
+#include "rr_planes.h"
 #include "sr_stages.h"
 
 using namespace mvmc_hip;
@@ -298,84 +300,76 @@ double* noalloc_scratch() {
   return (double*)p;
 }
 
-// The register-resident Pfaffian + inverse (full form n <= 64, panel form
-// 64 < n <= RR_NMAX) is a rebuild variant of the sampler (chosen by
-// measurement) and serves the batched entry points where it measured faster
-// than the panel-delayed kernel: n <= 64 and RR_BATCHED_MIN <= n <= RR_NMAX
-// (MI355X, random planes: 1.46-1.65x at n = 16..64; 0.81x at n = 96, 0.97x
-// at 144, 1.10x at 160, 1.18x at 176, 1.29x at 192 and 208, 1.36x at 224).  MVMC_PFINV_RR=0 selects the
-// panel-delayed kernels throughout, MVMC_PFINV_RR=2 the register-resident
-// ones for every 2 <= n <= RR_NMAX (same results either way).
-constexpr int RR_BATCHED_MIN = 152;
-int rr_mode() {
+// Pfaffian + inverse, one plane per workgroup (rr_planes.hip): serves the
+// batched entry points and every rebuild of the sampler for 2 <= n <=
+// RR_PLANE_MAX (complex batches RR_PLANE_MAX_C128); larger planes take the
+// panel-delayed kernels, and so does everything with MVMC_PFINV_RR=0 (same
+// results either way).
+constexpr int RR_PLANE_MAX = 224, RR_PLANE_MAX_C128 = 160;
+bool rr_enabled() {
   const char* e = std::getenv("MVMC_PFINV_RR");
-  return e ? std::atoi(e) : 1;
-}
-bool rr_enabled() { return rr_mode() != 0; }
-bool rr_batched(int n) {
-  if (!rr_enabled() || n < 2 || n > RR_NMAX) return false;
-  return rr_mode() == 2 || n <= RR_NFULL || n >= RR_BATCHED_MIN;
+  return !(e && std::atoi(e) == 0);
 }
 
-// Shape of the register-resident kernels for order n: the full form (16 x 16
-// threads, R = ceil(n / 16) <= 4) for n <= 64, the panel form (32 x 32,
-// R = ceil(n / 32) <= 7) above.
-struct RrCfg {
-  int t = 0, r = 0;
-  bool full = false;
-};
-RrCfg rr_cfg(int n) {
-  RrCfg c;
-  c.full = n <= RR_NFULL;
-  c.t = c.full ? RR_TS : RR_T;
-  c.r = (n + c.t - 1) / c.t;
-  return c;
-}
-
-// Calls f.template operator()<T, R, FULL>() for the configuration's
-// compiled instance.
-template <class F>
-void rr_dispatch(const RrCfg& c, F&& f) {
-  if (c.full) {
-    switch (c.r) {
-      case 1: f.template operator()<RR_TS, 1, true>(); return;
-      case 2: f.template operator()<RR_TS, 2, true>(); return;
-      case 3: f.template operator()<RR_TS, 3, true>(); return;
-      case 4: f.template operator()<RR_TS, 4, true>(); return;
-    }
+// Kernel instance, launch shape and resident workgroups for planes of order
+// n; the device is asked once per order, kind and device.
+RrPlan rr_plan(int n, bool cplx) {
+  if (n < 2 || n > (cplx ? RR_PLANE_MAX_C128 : RR_PLANE_MAX)) return RrPlan{};
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  static std::mutex mu;
+  static std::map<std::array<int, 3>, RrPlan> plans;
+  std::lock_guard<std::mutex> lk(mu);
+  RrPlan& p = plans[{dev, n, cplx ? 1 : 0}];
+  if (p.kernel) return p;
+  RrPlan q;
+  const int r8 = (n + 7) / 8, r16 = (n + 15) / 16;
+  if (n <= (cplx ? RR_NFULL : LP_NMAX)) {
+    q.threads = 64;
+    q.kernel = cplx ? rr_kernel_c128_small(r8) : n <= RR_NFULL ? rr_kernel_small(r8) : rr_kernel_mid(r8);
+    q.lds = rnd16((size_t)n * 4) + (cplx ? lp_lds_bytes<cz>(r8, true) : lp_lds_bytes<double>(r8, false));
+    q.scratch = lp_scratch_len(n) * (cplx ? sizeof(cz) : sizeof(double));
   } else {
-    switch (c.r) {
-      case 3: f.template operator()<RR_T, 3, false>(); return;
-      case 4: f.template operator()<RR_T, 4, false>(); return;
-      case 5: f.template operator()<RR_T, 5, false>(); return;
-      case 6: f.template operator()<RR_T, 6, false>(); return;
-      case 7: f.template operator()<RR_T, 7, false>(); return;
-    }
+    q.threads = 256;
+    q.kernel = cplx ? rr_kernel_c128_large(r16) : r16 <= 10 ? rr_kernel_large(r16) : rr_kernel_huge(r16);
+    q.lds = rnd16((size_t)n * 4) +
+            (cplx ? rr_lds_bytes<cz, true>(16, r16, false, n) : rr_lds_bytes<double, false>(16, r16, false, n));
+    q.scratch = rr_scratch_len(false, n) * (cplx ? sizeof(cz) : sizeof(double));
   }
-  throw Fail(MVMC_E_INVALID_SHAPE, "register-resident path covers 2 <= n <= 224");
+  if (!q.kernel) throw Fail(MVMC_E_INVALID_SHAPE, "no Pfaffian kernel for n = " + std::to_string(n));
+  int ncu = 0, occ = 0;
+  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  raise_lds_limit(q.kernel, q.lds);
+  HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, q.kernel, q.threads, q.lds));
+  q.resident = std::max(occ, 1) * std::max(ncu, 1);
+  return p = q;
 }
 
-// LDS limits of the rebuild kernels and their resident workgroups per CU.
-int rr_rebuild_prepare(const RrCfg& c, size_t lds) {
-  int occ = 1;
-  rr_dispatch(c, [&]<int T, int R, bool FULL>() {
-    raise_lds_limit((const void*)k_rebuild_rr<T, R, FULL>, lds);
-    raise_lds_limit((const void*)k_meas_rebuild_rr<T, R, FULL>, lds);
-    raise_lds_limit((const void*)k_begin_rr<T, R, FULL>, lds);
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_rebuild_rr<T, R, FULL>, T * T, lds));
-  });
-  return std::max(occ, 1);
+void rr_launch(const RrPlan& p, const RrJob& job, int grid, hipStream_t st) {
+  RrJob j = job;
+  void* args[] = {&j};
+  HIPCHK(hipLaunchKernel(p.kernel, dim3(grid), dim3(p.threads), args, p.lds, st));
 }
 
-// Periodic rebuild (s < 0) or measurement rebuild of saved sample s with the
-// register-resident kernels, one T x T workgroup per slot.
-void rr_launch_rebuild(const RrCfg& c, int grid, size_t lds, hipStream_t st, const EnsView& v, int s) {
-  rr_dispatch(c, [&]<int T, int R, bool FULL>() {
-    if (s < 0)
-      hipLaunchKernelGGL((k_rebuild_rr<T, R, FULL>), dim3(grid), dim3(T * T), lds, st, v);
-    else
-      hipLaunchKernelGGL((k_meas_rebuild_rr<T, R, FULL>), dim3(grid), dim3(T * T), lds, st, v, s);
-  });
+// Batched planes; gs: the caller's scratch of `slots` workgroups, or null to
+// take it from the stream's pool.
+void rr_batched(bool cplx, const void* in, void* out, int n, int count, int order, void* pf, int* status, void* gs,
+                int slots, hipStream_t st) {
+  const RrPlan p = rr_plan(n, cplx);
+  RrJob job{};
+  job.mode = RR_BATCHED;
+  job.n = n;
+  job.count = count;
+  job.in = in;
+  job.out = out;
+  job.pf = pf;
+  job.status = status;
+  job.order = order;
+  const int grid = std::min({count, p.resident, slots});
+  job.gs = gs;
+  if (!gs) HIPCHK(hipMallocAsync(&job.gs, p.scratch * grid, st));
+  rr_launch(p, job, grid, st);
+  if (!gs) HIPCHK(hipFreeAsync(job.gs, st));
 }
 
 template <class T>
@@ -415,16 +409,19 @@ struct mvmc_ens {
   std::vector<void*> allocs;
   hipStream_t st = nullptr;
   int grid_samp = 0, grid_meas = 0, grid_rebuild = 0, slots = 0;
-  // rebuild-kernel variants (0: 3 workgroups per CU, 8-column close batches;
-  // 1: 2 per CU, 16 columns; 2: register-resident, one 1024-thread workgroup
-  // per CU, for 64 < n <= RR_NMAX), tuned on the first well-filled launches:
-  // rb_variant -1 while measuring, then the fastest one
-  int grid_rb[3] = {0, 0, 0};
-  int rb_nvar = 2;
+  // rebuild-kernel variants: 2, plane by plane (rr_planes.hip), wherever it
+  // covers n (it measured 2-4 times faster than the others); beyond, walker
+  // by walker (0: 3 workgroups per CU, 8-column close batches; 1: 2 per CU,
+  // 16 columns), tuned on the first well-filled launches: rb_variant -1
+  // while measuring, then the faster one
+  int grid_rb[2] = {0, 0};
+  RrPlan rr;          // variant 2: kernel, workgroups, their scratch
+  int rr_grid = 0;
+  void* rr_gs = nullptr;
   int rb_variant = -1;
-  double rb_ms[3] = {0, 0, 0}, rb_walkers[3] = {0, 0, 0};
-  int rb_samples[3] = {0, 0, 0};
-  size_t lds_rebuild = 0, lds_rr = 0;
+  double rb_ms[2] = {0, 0}, rb_walkers[2] = {0, 0};
+  int rb_samples[2] = {0, 0};
+  size_t lds_rebuild = 0;
   double rebuild_ms = 0, rebuild_launches = 0;
   size_t lds_samp = 0, lds_meas = 0;
   double* d_slater = nullptr;
@@ -704,24 +701,22 @@ void create_impl(mvmc_ens* E, const char* namelist, const char* initial_def, int
   E->grid_rebuild = (int)std::min<long long>(walkers, (long long)occ_r * ncu);
   E->grid_rb[0] = E->grid_rebuild;
   E->grid_rb[1] = (int)std::min<long long>(walkers, (long long)occ_r1 * ncu);
-  size_t work_per_slot = pfinv_work_doubles(v.n, v.nqp);
-  if (rr_enabled() && v.n >= 2 && v.n <= RR_NMAX) {
-    // ei, rs, pfn, then the register-resident carve; 2 n^2 doubles of work
-    E->lds_rr = 2 * rnd16((size_t)v.n * 4) + rnd16((size_t)v.nqp * 8) + rr_lds_bytes(v.n);
-    if (E->lds_rr <= (size_t)maxlds) {
-      const int occ = rr_rebuild_prepare(rr_cfg(v.n), E->lds_rr);
-      E->rb_nvar = 3;
-      E->grid_rb[2] = (int)std::min<long long>(walkers, (long long)occ * ncu);
-      work_per_slot = std::max(work_per_slot, (size_t)2 * v.n * v.n);
-    }
+  const size_t work_per_slot = pfinv_work_doubles(v.n, v.nqp);
+  if (rr_enabled()) E->rr = rr_plan(v.n, false);
+  if (E->rr.kernel) {
+    E->rb_variant = 2;
+    E->rr_grid = (int)std::min<long long>((long long)walkers * v.nqp, E->rr.resident);
+    E->rr_gs = dalloc<char>(A, E->rr.scratch * E->rr_grid);
   }
-  // MVMC_RB_VARIANT=k fixes the rebuild variant instead of tuning it
+  v.pf_new = dalloc<double>(A, W * v.nqp);
+  v.pinfo = dalloc<int>(A, W * v.nqp);
+  // MVMC_RB_VARIANT=k fixes the rebuild variant
   if (const char* f = std::getenv("MVMC_RB_VARIANT")) {
     const int k = std::atoi(f);
-    if (k >= 0 && k < E->rb_nvar) E->rb_variant = k;
+    if (k >= 0 && (k < 2 || (k == 2 && E->rr.kernel))) E->rb_variant = k;
   }
-  E->slots = std::max(std::max(E->grid_samp, E->grid_meas),
-                      std::max(std::max(E->grid_rb[0], E->grid_rb[1]), E->grid_rb[2]));
+  v.by_plane = E->rb_variant == 2 ? 1 : 0;
+  E->slots = std::max(std::max(E->grid_samp, E->grid_meas), std::max(E->grid_rb[0], E->grid_rb[1]));
   v.work = dalloc<double>(A, (size_t)E->slots * work_per_slot);
   v.qorb = dalloc<double>(A, (size_t)E->slots * v.nqp * std::max(v.nslater, 1));
   v.pend = dalloc<double>(A, (size_t)E->slots * 2 * PEND_MAX * v.nqp * v.n);
@@ -751,47 +746,55 @@ void create_impl(mvmc_ens* E, const char* namelist, const char* initial_def, int
   HIPCHK(hipStreamSynchronize(E->st));
 }
 
+// Plane-wise rebuild of a run (mode, saved sample s) on stream st; its
+// walkers' outcomes follow from k_rr_finish.
+void launch_planes(mvmc_ens* E, int mode, int s, hipStream_t st) {
+  RrJob job{};
+  job.mode = mode;
+  job.n = E->v.n;
+  job.gs = E->rr_gs;
+  job.s = s;
+  job.v = E->v;
+  rr_launch(E->rr, job, E->rr_grid, st);
+}
+
 void launch_rebuild(mvmc_ens* E, int var) {
-  if (var == 2)
-    rr_launch_rebuild(rr_cfg(E->v.n), E->grid_rb[2], E->lds_rr, E->st, E->v, -1);
-  else if (var == 1)
+  if (var == 2) {
+    launch_planes(E, RR_REBUILD, 0, E->st);
+    hipLaunchKernelGGL(k_rr_finish, dim3(nblk(E->v.W, 64)), dim3(64), 0, E->st, E->v, (int)RR_REBUILD, 0);
+  } else if (var == 1) {
     hipLaunchKernelGGL((k_rebuild<2, 16>), dim3(E->grid_rb[1]), dim3(256), E->lds_rebuild, E->st, E->v);
-  else
+  } else {
     hipLaunchKernelGGL((k_rebuild<3, 8>), dim3(E->grid_rb[0]), dim3(256), E->lds_rebuild, E->st, E->v);
+  }
   HIPCHK(hipGetLastError());
 }
 
-// Start of a sampling call: with the register-resident rebuild chosen, the
-// walkers resuming from their burn configuration are rebuilt by k_begin_rr
-// and k_begin serves the rest (placement, failed or non-finite rebuilds);
-// otherwise k_begin serves every walker.
+// Start of a sampling call: with the plane-wise rebuild the walkers resuming
+// from their burn configuration are rebuilt by it and k_begin serves the
+// rest (placement, failed or non-finite rebuilds); otherwise k_begin serves
+// every walker.
 void launch_begin(mvmc_ens* E) {
   EnsView& v = E->v;
-  int marked = v.W;
-  if (E->rb_variant == 2) {
-    HIPCHK(hipMemsetAsync(v.nflag + 5, 0, sizeof(int), E->st));
-    rr_dispatch(rr_cfg(v.n), [&]<int T, int R, bool FULL>() {
-      hipLaunchKernelGGL((k_begin_rr<T, R, FULL>), dim3(E->grid_rb[2]), dim3(T * T), E->lds_rr, E->st, v);
-    });
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(&marked, v.nflag + 5, sizeof(int), hipMemcpyDeviceToHost, E->st));
-    HIPCHK(hipStreamSynchronize(E->st));
-    if (marked == 0) return;
+  if (v.by_plane) {
+    launch_planes(E, RR_BEGIN, 0, E->st);
+    hipLaunchKernelGGL(k_rr_finish, dim3(nblk(v.W, 64)), dim3(64), 0, E->st, v, (int)RR_BEGIN, 0);
   }
-  hipLaunchKernelGGL(k_begin<false>, dim3(E->grid_samp), dim3(256), E->lds_samp, E->st, v, GroupArgs{},
-                     E->rb_variant == 2 ? 1 : 0);
+  hipLaunchKernelGGL(k_begin<false>, dim3(E->grid_samp), dim3(256), E->lds_samp, E->st, v, GroupArgs{}, v.by_plane);
   HIPCHK(hipGetLastError());
 }
 
 void launch_meas_rebuild(mvmc_ens* E, int s) {
-  if (E->rb_variant == 2)
-    rr_launch_rebuild(rr_cfg(E->v.n), E->grid_rb[2], E->lds_rr, E->st, E->v, s);
-  else if (E->rb_variant == 1)
+  if (E->rb_variant == 2) {
+    launch_planes(E, RR_MEASURE, s, E->st);
+    hipLaunchKernelGGL(k_rr_finish, dim3(nblk(E->v.W, 64)), dim3(64), 0, E->st, E->v, (int)RR_MEASURE, s);
+  } else if (E->rb_variant == 1) {
     hipLaunchKernelGGL((k_meas_rebuild<2, 16, false>), dim3(E->grid_rb[1]), dim3(256), E->lds_rebuild, E->st, E->v,
                        GroupArgs{}, s);
-  else
+  } else {
     hipLaunchKernelGGL((k_meas_rebuild<3, 8, false>), dim3(E->grid_rb[0]), dim3(256), E->lds_rebuild, E->st, E->v,
                        GroupArgs{}, s);
+  }
   HIPCHK(hipGetLastError());
 }
 
@@ -862,7 +865,7 @@ void sample_impl(mvmc_ens* E) {
       rebuilt += nf;
       // variant: the tuned one, else alternate on launches that fill every
       // slot twice over (smaller ones run variant 0 and are not counted)
-      const int nvar = E->rb_nvar;
+      constexpr int nvar = 2;
       int gmax = 0, least = 0;
       for (int k = 0; k < nvar; ++k) {
         gmax = std::max(gmax, E->grid_rb[k]);
@@ -1416,68 +1419,6 @@ struct GroupPart {
   std::vector<double> weight; // per-run work estimate the ranges are cut by
 };
 
-// Complex planes: the same shapes, full form n <= 64, panel form n <= 160
-// (two doubles per slot), each in both LTL orders.
-template <int ORDER, class F>
-void rr_dispatch_c(const RrCfg& c, F&& f) {
-  if (c.full) {
-    switch (c.r) {
-      case 1: f.template operator()<RR_TS, 1, true, ORDER>(); return;
-      case 2: f.template operator()<RR_TS, 2, true, ORDER>(); return;
-      case 3: f.template operator()<RR_TS, 3, true, ORDER>(); return;
-      case 4: f.template operator()<RR_TS, 4, true, ORDER>(); return;
-    }
-  } else {
-    switch (c.r) {
-      case 3: f.template operator()<RR_T, 3, false, ORDER>(); return;
-      case 4: f.template operator()<RR_T, 4, false, ORDER>(); return;
-      case 5: f.template operator()<RR_T, 5, false, ORDER>(); return;
-    }
-  }
-  throw Fail(MVMC_E_INVALID_SHAPE, "complex register-resident path covers 2 <= n <= 160");
-}
-
-void launch_pfinv_rr_c128(const cz* in, cz* out, int n, int count, int order, cz* pf, int* status, hipStream_t st) {
-  int dev = 0, ncu = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const RrCfg c = rr_cfg(n);
-  const size_t lds = rr_lds_bytes<cz>(n);
-  auto go = [&]<int T, int R, bool FULL, int ORDER>() {
-    raise_lds_limit((const void*)k_pfinv_rr_c128<T, R, FULL, ORDER>, lds);
-    int occ = 1;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pfinv_rr_c128<T, R, FULL, ORDER>, T * T, lds));
-    const int grid = (int)std::min<long long>(count, (long long)std::max(occ, 1) * std::max(ncu, 1));
-    cz* gs = nullptr;
-    HIPCHK(hipMallocAsync((void**)&gs, sizeof(cz) * 2 * (size_t)n * n * grid, st));
-    hipLaunchKernelGGL((k_pfinv_rr_c128<T, R, FULL, ORDER>), dim3(grid), dim3(T * T), lds, st, in, out, n, count, gs,
-                       pf, status);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipFreeAsync(gs, st));
-  };
-  if (order == 0) rr_dispatch_c<0>(c, go);
-  else rr_dispatch_c<1>(c, go);
-}
-
-void launch_pfinv_rr(const double* in, double* out, int n, int count, double* pf, int* status, hipStream_t st) {
-  int dev = 0, ncu = 0;
-  HIPCHK(hipGetDevice(&dev));
-  HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  const RrCfg c = rr_cfg(n);
-  const size_t lds = rr_lds_bytes(n);
-  rr_dispatch(c, [&]<int T, int R, bool FULL>() {
-    raise_lds_limit((const void*)k_pfinv_rr<T, R, FULL>, lds);
-    int occ = 1;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pfinv_rr<T, R, FULL>, T * T, lds));
-    const int grid = (int)std::min<long long>(count, (long long)std::max(occ, 1) * std::max(ncu, 1));
-    double* gs = nullptr;
-    HIPCHK(hipMallocAsync((void**)&gs, sizeof(double) * 2 * (size_t)n * n * grid, st));
-    hipLaunchKernelGGL((k_pfinv_rr<T, R, FULL>), dim3(grid), dim3(T * T), lds, st, in, out, n, count, gs, pf, status);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipFreeAsync(gs, st));
-  });
-}
-
 }  // namespace
 
 struct mvmc_group {
@@ -1496,6 +1437,8 @@ struct mvmc_group {
   double* d_work = nullptr;
   double* d_pend = nullptr;
   long long work_stride = 0, pend_stride = 0;
+  int entries = 0;           // walkers of all runs
+  bool walkerwise = false;   // some run is rebuilt walker by walker
   int graph_rounds = 0;      // k_block + k_rebuild rounds per captured graph (0: direct launches)
   int autotune = 1;          // re-cut the slot ranges from measured busy times after every step
   // timings of the last group step
@@ -1606,6 +1549,8 @@ void group_create_impl(mvmc_group* G, int nruns, const char* const* namelists, c
   for (int r = 0; r < nruns; ++r) order[r] = r;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return G->runs[a]->v.n > G->runs[b]->v.n; });
   for (int k = 0; k < nruns; ++k) qstart[k + 1] = qstart[k] + G->runs[order[k]]->v.W;
+  G->entries = qstart[nruns];
+  for (mvmc_ens* E : G->runs) G->walkerwise = G->walkerwise || !E->v.by_plane;
   G->d_qstart = dalloc<int>(G->allocs, nruns + 1);
   G->d_qrun = dalloc<int>(G->allocs, nruns);
   G->d_gq = dalloc<int>(G->allocs, 4);
@@ -1666,14 +1611,32 @@ void group_clear_times(mvmc_group* G) {
     HIPCHK(hipMemsetAsync(P->time, 0, sizeof(long long) * P->capacity, G->st));
 }
 
+// Plane-wise rebuilds of the group's runs, a launch per run (the kernel
+// instance follows the run's Nsize) and one for the outcomes of all.
+void group_planes(mvmc_group* G, int mode, int s) {
+  bool any = false;
+  for (mvmc_ens* E : G->runs)
+    if (E->v.by_plane) {
+      launch_planes(E, mode, s, G->st);
+      any = true;
+    }
+  if (any)
+    hipLaunchKernelGGL(k_rr_finish_q, dim3(nblk(G->entries, 64)), dim3(64), 0, G->st, group_args(G, G->rb, false),
+                       mode, s);
+}
+
 // One round: clear the walker counters, run every walker until its step ends
 // or its rebuild is due, rebuild the walkers handed over.
 void group_round(mvmc_group* G, int out, int n_in_max) {
+  const int R = (int)G->runs.size();
   hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, G->st, G->d_gq, 4, 0);
+  hipLaunchKernelGGL(k_fill_int, dim3(nblk(NFLAGS * R)), dim3(256), 0, G->st, G->d_flags, NFLAGS * R, 0);
   hipLaunchKernelGGL((k_block<double, true>), dim3(G->samp.capacity), dim3(256), G->lds_samp, G->st, EnsView{},
                      group_args(G, G->samp, false), out, n_in_max);
-  hipLaunchKernelGGL((k_rebuild_q<3, 8>), dim3(G->rb.capacity), dim3(256), G->lds_rebuild, G->st,
-                     group_args(G, G->rb, false));
+  group_planes(G, RR_REBUILD, 0);
+  if (G->walkerwise)
+    hipLaunchKernelGGL((k_rebuild_q<3, 8>), dim3(G->rb.capacity), dim3(256), G->lds_rebuild, G->st,
+                       group_args(G, G->rb, false));
 }
 
 void group_sample(mvmc_group* G) {
@@ -1684,8 +1647,11 @@ void group_sample(mvmc_group* G) {
     E->upload_tables();
   }
   group_clear_times(G);
+  // k_begin serves the walkers that the plane-wise begin leaves (wstate[7])
+  // and, in runs rebuilt walker by walker, every walker
+  group_planes(G, RR_BEGIN, 0);
   hipLaunchKernelGGL(k_begin<true>, dim3(G->samp.start[R]), dim3(256), G->lds_samp, G->st, EnsView{},
-                     group_args(G, G->samp), 0);
+                     group_args(G, G->samp), 1);
   HIPCHK(hipGetLastError());
   int n_out = 0;
   for (mvmc_ens* E : G->runs) {
@@ -1750,8 +1716,10 @@ void group_measure(mvmc_group* G) {
   const double t0 = now_s();
   const int nsample = G->runs[0]->v.nsample;
   for (int s = 0; s < nsample; ++s) {
-    hipLaunchKernelGGL((k_meas_rebuild<3, 8, true>), dim3(G->rb.start[R]), dim3(256), G->lds_rebuild, G->st,
-                       EnsView{}, group_args(G, G->rb), s);
+    group_planes(G, RR_MEASURE, s);
+    if (G->walkerwise)
+      hipLaunchKernelGGL((k_meas_rebuild<3, 8, true>), dim3(G->rb.start[R]), dim3(256), G->lds_rebuild, G->st,
+                         EnsView{}, group_args(G, G->rb), s);
     hipLaunchKernelGGL(k_measure<true>, dim3(G->meas.start[R]), dim3(256), G->lds_meas, G->st, EnsView{},
                        group_args(G, G->meas), 1, s);
     HIPCHK(hipGetLastError());
@@ -1775,8 +1743,8 @@ int mvmc_pfinv_f64(const double* planes, int n, int count, double* pf, double* i
     if (count == 0) return;
     if (!planes || !pf || !inv || !status) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
     hipStream_t st = (hipStream_t)stream;
-    if (rr_batched(n)) {
-      launch_pfinv_rr(planes, inv, n, count, pf, status, st);
+    if (n <= RR_PLANE_MAX && rr_enabled()) {
+      rr_batched(false, planes, inv, n, count, 0, pf, status, nullptr, INT32_MAX, st);
       return;
     }
     if ((const double*)inv != planes)
@@ -1810,6 +1778,11 @@ int mvmc_pfinv_f64_noalloc(const double* planes, int n, int count, double* pf, d
     if (!planes || !pf || !inv || !status) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
     double* work = noalloc_scratch();
     hipStream_t st = (hipStream_t)stream;
+    if (n <= RR_PLANE_MAX && rr_enabled()) {
+      const size_t slots = NOALLOC_SCRATCH_DOUBLES * sizeof(double) / rr_plan(n, false).scratch;
+      rr_batched(false, planes, inv, n, count, 0, pf, status, work, (int)std::min<size_t>(slots, INT32_MAX), st);
+      return;
+    }
     if ((const double*)inv != planes)
       HIPCHK(hipMemcpyAsync(inv, planes, sizeof(double) * n * n * count, hipMemcpyDeviceToDevice, st));
     const int np = n <= 32 ? 8 : 4;
@@ -1840,8 +1813,8 @@ int mvmc_pfinv_c128(const double* planes, int n, int count, int order, double* p
       throw Fail(MVMC_E_INVALID_SHAPE, "complex buffers must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
     const size_t nn = (size_t)n * n;
-    if (rr_enabled() && n <= RR_C_NMAX) {
-      launch_pfinv_rr_c128((const cz*)planes, (cz*)inv, n, count, order, (cz*)pf, status, st);
+    if (n <= RR_PLANE_MAX_C128 && rr_enabled()) {
+      rr_batched(true, planes, inv, n, count, order, pf, status, nullptr, INT32_MAX, st);
       return;
     }
     if ((const double*)inv != planes)
@@ -2243,7 +2216,7 @@ int mvmc_ens_timings(mvmc_ens* e, double* t) {
   t[16] = e->rb_variant;
   t[17] = e->rb_walkers[0] > 0 ? e->rb_ms[0] / e->rb_walkers[0] : 0.0;
   t[18] = e->rb_walkers[1] > 0 ? e->rb_ms[1] / e->rb_walkers[1] : 0.0;
-  t[19] = e->rb_walkers[2] > 0 ? e->rb_ms[2] / e->rb_walkers[2] : 0.0;
+  t[19] = 0.0;  // variant 2 is not tuned
   t[20] = e->adj_ms; t[21] = e->adj_rebuild_ms; t[22] = e->gram_ms; t[23] = e->block_write_passes;
   t[24] = e->block_flush_passes; t[25] = 0.0;
   return MVMC_OK;

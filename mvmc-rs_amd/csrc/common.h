@@ -18,6 +18,21 @@ enum Status : int {
 };
 
 // ---------------------------------------------------------------------------
+// LDS carving (the host computes the same total through lds_bytes_*)
+// ---------------------------------------------------------------------------
+struct Carver {
+  char* p;
+  template <class T>
+  __device__ T* take(size_t count) {
+    T* r = (T*)p;
+    size_t bytes = (count * sizeof(T) + 15) & ~(size_t)15;
+    p += bytes;
+    return r;
+  }
+};
+
+__host__ __device__ inline size_t rnd16(size_t b) { return (b + 15) & ~(size_t)15; }
+// ---------------------------------------------------------------------------
 // SFMT19937 on the device.  State lives in LDS (624 words + cursor) while a
 // walker is active and in HBM between launches; refills are done by one lane.
 // Algorithm: Saito & Matsumoto, SFMT-19937:122-18-1-11-1 (parameters

@@ -7,6 +7,9 @@ namespace mvmc_hip {
 
 constexpr int NFLAGS = 8;  // ints of an ensemble's walker counters (EnsView::nflag)
 
+// Outcomes of a plane's rebuild besides the PlaneStatus codes (pinfo).
+constexpr int RR_ALL_ZERO = -2, RR_BAD_SITE = -3, RR_SKIPPED = -4;
+
 struct EnsView {
   // dimensions
   int W;          // walkers
@@ -46,15 +49,16 @@ struct EnsView {
   double* inv;        // [W][nqp][n*n]
   float* inv32;       // [W][nqp][n*n] the sampler's inverse in the mixed-precision form, else null
   double* pf;         // [W][nqp]
+  double* pf_new;     // [W][nqp] Pfaffians of the planes of a rebuild in progress
+  int* pinfo;         // [W][nqp] their outcome: 0 ok, > 0 zero pivot, -1 non-finite, RR_*
   double* log_ip;     // [W]
   int* wstate;        // [W][8]: 0 burn flag, 1 n_accept window, 2 n_out, 3 status,
                       //   4 next proposal of the outer step, 5 rebuild pending, 6 outer step done,
-                      //   7 left by k_begin_rr to k_begin
+                      //   7 left by the plane-wise begin to k_begin
   int* nflag;         // [NFLAGS]: 0 walkers handed to the rebuild kernel by the last k_block launch,
                       //   1 next walker taken by a k_block slot, 2 next hand-over entry taken by k_rebuild,
                       //   3 passes of the last k_block launch that wrote a walker's planes back,
-                      //   4 those of them that accepted no move (pending updates flushed),
-                      //   5 walkers k_begin_rr left to k_begin
+                      //   4 those of them that accepted no move (pending updates flushed)
   int* rlist;         // [W] walkers handed to the rebuild kernel, in hand-over order
   long long* counter; // [W][4]
   // saved samples
@@ -72,6 +76,7 @@ struct EnsView {
   long long* clk;     // [slots][32] phase clocks (MVMC_PHASE_CLOCKS builds), else null
   double* gscr;       // [slots][gstride] per-term Green ratios of the measurement
   int gstride;
+  int by_plane;       // rebuilds run plane by plane (rr_planes.hip), else walker by walker
 };
 
 // One launch over several ensembles (runs of different models): run r owns
@@ -87,8 +92,10 @@ struct GroupArgs {
   // in [qstart[k], qstart[k+1]) for run qrun[k], walker g - qstart[k]; any
   // workgroup takes any run's walker, with scratch slot blockIdx.x of the
   // group's own buffers (strides for the largest run).
-  int* gq;                // [4]: 0 entries handed to the rebuild, 1 next entry, 2 next hand-over taken
-  int* glist;             // [total] queue entries handed to the rebuild
+  int* gq;                // [4]: 0 walkers handed to the rebuild, 1 next entry, 2 next hand-over taken,
+                          //   3 of the handed-over ones those in glist
+  int* glist;             // [total] queue entries of runs rebuilt walker by walker; the others' walkers are in
+                          //   their runs' own lists (nflag, rlist)
   const int* qstart;      // [nruns + 1]
   const int* qrun;        // [nruns]
   double* work;           // [grid][work_stride]

@@ -22,26 +22,8 @@
 #include "common.h"
 #include "ensemble.h"
 #include "pfinv_dev.h"
+#include "rr_planes.h"
 
-namespace mvmc_hip {
-
-// ---------------------------------------------------------------------------
-// LDS carving (the host computes the same total through lds_bytes_*)
-// ---------------------------------------------------------------------------
-struct Carver {
-  char* p;
-  template <class T>
-  __device__ T* take(size_t count) {
-    T* r = (T*)p;
-    size_t bytes = (count * sizeof(T) + 15) & ~(size_t)15;
-    p += bytes;
-    return r;
-  }
-};
-
-__host__ __device__ inline size_t rnd16(size_t b) { return (b + 15) & ~(size_t)15; }
-}  // namespace mvmc_hip
-#include "pfinv_rr.h"
 namespace mvmc_hip {
 
 // Run of this workgroup in a group launch (slot_start is small and uniform).
@@ -457,7 +439,7 @@ __device__ inline void copy_inv32(const EnsView& v, int w) {
   }
 }
 
-// only_marked: serve only the walkers k_begin_rr left to it (wstate[7] set).
+// only_marked: serve only the walkers k_rr_finish left to it (wstate[7] set).
 template <bool GROUP>
 __global__ void __launch_bounds__(256) k_begin(EnsView v_arg, GroupArgs ga, int only_marked) {
   ENS_SLOT(v_arg, ga)
@@ -468,7 +450,7 @@ __global__ void __launch_bounds__(256) k_begin(EnsView v_arg, GroupArgs ga, int 
   char* pfscr = (char*)L.uni;
   for (int w = slot; w < v.W; w += nslots) {
     int* ws = v.wstate + (size_t)w * 8;
-    if (only_marked && ws[7] == 0) continue;
+    if (only_marked && v.by_plane && ws[7] == 0) continue;
     double* planes = v.inv + (size_t)w * v.nqp * v.n * v.n;
     int* cnt = v.proj_cnt + (size_t)w * v.nproj;
     load_walker(v, w, L, true);
@@ -1343,7 +1325,8 @@ __global__ void __launch_bounds__(256, 2) k_block(EnsView v_arg, GroupArgs ga, i
         ws[1] = L.misc[M_NACC];
         ws[4] = stop_at;
         ws[5] = 1;
-        if (GROUP) ga.glist[atomicAdd(ga.gq, 1)] = qe;
+        if (GROUP) atomicAdd(ga.gq, 1);
+        if (GROUP && !v.by_plane) ga.glist[atomicAdd(ga.gq + 3, 1)] = qe;
         else v.rlist[atomicAdd(v.nflag, 1)] = w;
       }
       __syncthreads();
@@ -1450,7 +1433,7 @@ __global__ void __launch_bounds__(256, MINB) k_rebuild_q(GroupArgs ga) {
   extern __shared__ __align__(16) char lds[];
   const int tid = threadIdx.x;
   double* work = ga.work + (size_t)blockIdx.x * ga.work_stride;
-  const int nhand = *ga.gq;  // entries handed over by the k_block launch before
+  const int nhand = ga.gq[3];  // entries handed over by the k_block launch before
   __shared__ int next_i;
   for (;;) {
     if (tid == 0) next_i = atomicAdd(ga.gq + 2, 1);
@@ -1511,6 +1494,7 @@ __device__ double direct_proj_ratio_moved(const EnsView& v, int source, int dest
 template <int MINB, int JB, bool GROUP>
 __global__ void __launch_bounds__(256, MINB) k_meas_rebuild(EnsView v_arg, GroupArgs ga, int s) {
   ENS_SLOT(v_arg, ga)
+  if (GROUP && v.by_plane) return;
   extern __shared__ __align__(16) char lds[];
   Carver c{lds};
   int* ei = c.take<int>(v.n);
@@ -2291,198 +2275,61 @@ __global__ void k_cg_dir(int na, const double* sc, const int* ctl, const double*
 // Batched Pfaffian + inverse (BatchedEngine): planes [count][n][n]
 // column-major; one workgroup per plane batch of np planes.
 // ---------------------------------------------------------------------------
-// Batched Pfaffian + inverse of n <= RR_NMAX planes, one plane per T x T
-// workgroup at a time (planes blockIdx.x, + gridDim.x, ...), register-
-// resident (pfinv_rr.h: the panel form, T = 32, for n > 64; the full form,
-// T = 16, for n <= 64); gs: 2 n^2 doubles of scratch per workgroup.
-// Results and statuses as k_pfinv_batched; in == out works in place (the
-// plane is read whole before it is written).
-template <int T, int R, bool FULL>
-__global__ void __launch_bounds__(T * T) k_pfinv_rr(const double* in, double* out, int n, int count, double* gs_base,
-                                                   double* pf, int* status) {
-  extern __shared__ __align__(16) char lds[];
-  Carver c{lds};
-  RrLds L = carve_rr(c, n);
-  double* gs = gs_base + (size_t)blockIdx.x * 2 * n * n;
-  for (int p = blockIdx.x; p < count; p += gridDim.x) {
-    const double* A = in + (size_t)p * n * n;
-    double* O = out + (size_t)p * n * n;
-    double pfv = 0.0;
-    int info = 0;
-    bool az = false;
-    rr_pfinv<T, R, FULL>([&](int i, int j) { return A[i + (size_t)j * n]; }, n, O, 1.0, gs, L, pfv, info, false, az);
-    if (threadIdx.x == 0) {
-      status[p] = info;
-      pf[p] = info > 0 ? 0.0 : pfv;
-    }
-    if (info != 0)
-      for (int e = threadIdx.x; e < n * n; e += blockDim.x) O[e] = 0.0;
-    __syncthreads();
-  }
-}
-
-// Periodic rebuild (engine.rs:454-473) of the handed-over walkers with the
-// register-resident Pfaffian + inverse, one walker per T x T workgroup, its
-// NQP planes in turn, gathered straight from the Slater table
-// (A(r, c) = -S[rs_c][rs_r], pfaffian.rs:1107-1188).  A plane that is all
-// zero or fails stops the walker's rebuild (its Pfaffians are then not
-// replaced; the accept window restarts either way).
-template <int T, int R, bool FULL>
-__device__ __forceinline__ int rr_calc_m_all(const EnsView& v, const int* ei, int* rs, double* planes, double* gs,
-                                             RrLds& L, double* pfn) {
-  const int tid = threadIdx.x;
-  __shared__ int bad_site;
-  if (tid == 0) bad_site = 0;
-  __syncthreads();
-  for (int i = tid; i < v.n; i += blockDim.x) {
-    const int r = ei[i];
-    rs[i] = r + (i / v.ne) * v.ns;
-    if (r < 0 || r >= v.ns) bad_site = 1;
-  }
-  __syncthreads();
-  if (bad_site) {
-    if (tid == 0) set_status(v.status, ST_BAD_INPUT);
-    __syncthreads();
-    return 1;
-  }
-  const int n = v.n, n2 = v.n2;
-  for (int q = 0; q < v.nqp; ++q) {
-    const double* S = v.slater + (size_t)q * n2 * n2;
-    double pfv = 0.0;
-    int info = 0;
-    bool az = false;
-    rr_pfinv<T, R, FULL>([&](int i, int j) { return -S[(size_t)rs[j] * n2 + rs[i]]; }, n,
-                         planes + (size_t)q * n * n, -1.0, gs, L, pfv, info, true, az);
-    if (az || info != 0) return 1;
-    if (tid == 0) pfn[q] = pfv;
-  }
-  __syncthreads();
-  return 0;
-}
-
-template <int T, int R, bool FULL>
-__global__ void __launch_bounds__(T * T) k_rebuild_rr(EnsView v) {
-  extern __shared__ __align__(16) char lds[];
-  Carver c{lds};
-  int* ei = c.take<int>(v.n);
-  int* rs = c.take<int>(v.n);
-  double* pfn = c.take<double>(v.nqp);
-  RrLds L = carve_rr(c, v.n);
-  const int tid = threadIdx.x;
-  double* gs = v.work + (size_t)blockIdx.x * 2 * v.n * v.n;
-  const int nhand = *v.nflag;
-  __shared__ int next_i;
-  for (;;) {
-    if (tid == 0) next_i = atomicAdd(v.nflag + 2, 1);
-    __syncthreads();
-    const int li = next_i;
-    __syncthreads();
-    if (li >= nhand) break;
-    const int w = v.rlist[li];
-    int* ws = v.wstate + (size_t)w * 8;
-    for (int i = tid; i < v.n; i += blockDim.x) ei[i] = v.ele_idx[(size_t)w * v.n + i];
-    __syncthreads();
-    double* planes = v.inv + (size_t)w * v.nqp * v.n * v.n;
-    const int bad = rr_calc_m_all<T, R, FULL>(v, ei, rs, planes, gs, L, pfn);
-    copy_inv32(v, w);
-    if (tid == 0) {
-      if (!bad) {
-        for (int q = 0; q < v.nqp; ++q) v.pf[(size_t)w * v.nqp + q] = pfn[q];
-        v.log_ip[w] = ddm::cr_log(fabs(ip_of(v, pfn)));
-      }
-      ws[1] = 0;
-      ws[5] = 0;
-    }
-    __syncthreads();
-  }
-}
-
-// Start of a sampling call (k_begin) for the walkers that resume from their
-// burn configuration, the case of every call after the first: its rebuild
-// through the register-resident Pfaffian + inverse, walkers blockIdx.x,
-// + gridDim.x, ...  That phase draws no random numbers and keeps the
-// configuration, so a walker is done here when every plane factorises (no
-// AllZero plane, info 0: the planes and Pfaffians then equal k_begin's bit
-// for bit) and log|<x|psi>| is finite.  Any other walker is marked
-// (wstate[7] = 1, counted in nflag[5]) and left to k_begin, which repeats
-// the same rebuild and goes on from there.
-template <int T, int R, bool FULL>
-__global__ void __launch_bounds__(T * T) k_begin_rr(EnsView v) {
-  extern __shared__ __align__(16) char lds[];
-  Carver c{lds};
-  int* ei = c.take<int>(v.n);
-  int* rs = c.take<int>(v.n);
-  double* pfn = c.take<double>(v.nqp);
-  RrLds L = carve_rr(c, v.n);
-  const int tid = threadIdx.x;
-  double* gs = v.work + (size_t)blockIdx.x * 2 * v.n * v.n;
-  __shared__ double lip;
-  for (int w = blockIdx.x; w < v.W; w += gridDim.x) {
-    int* ws = v.wstate + (size_t)w * 8;
-    bool done = false;
-    if (ws[0]) {
-      for (int i = tid; i < v.n; i += blockDim.x) ei[i] = v.ele_idx[(size_t)w * v.n + i];
-      __syncthreads();
-      double* planes = v.inv + (size_t)w * v.nqp * v.n * v.n;
-      const int bad = rr_calc_m_all<T, R, FULL>(v, ei, rs, planes, gs, L, pfn);
-      if (tid == 0) lip = bad ? 0.0 : ddm::cr_log(fabs(ip_of(v, pfn)));
-      __syncthreads();
-      done = !bad && lip - lip == 0.0;
-    }
+// Outcome of a plane-wise rebuild (rr_planes.hip) of one walker, from its
+// planes' Pfaffians (pf_new) and outcomes (pinfo).
+//   RR_REBUILD (engine.rs:454-473): with every plane factorised the Pfaffians
+//     and log|<x|psi>| are replaced; the accept window restarts either way.
+//   RR_BEGIN: the walkers that resume from their burn configuration.  That
+//     phase draws no random numbers and keeps the configuration, so a walker
+//     is done when every plane factorised (planes and Pfaffians then equal
+//     k_begin's bit for bit) and log|<x|psi>| is finite.  Any other walker
+//     is marked (wstate[7] = 1) and left to k_begin, which repeats the same
+//     rebuild and goes on from there.
+//   RR_MEASURE: the Pfaffians and s_valid[w][s] of the saved sample.
+__device__ inline void rr_finish_walker(const EnsView& v, int mode, int s, int w) {
+  const size_t off = (size_t)w * v.nqp;
+  bool ok = true;
+  for (int q = 0; q < v.nqp; ++q) ok = ok && v.pinfo[off + q] == 0;
+  int* ws = v.wstate + (size_t)w * 8;
+  if (mode == RR_BEGIN) {
+    double lip = 0.0;
+    bool done = ws[0] != 0 && ok;
     if (done) {
-      copy_inv32(v, w);
-      if (tid == 0) {
-        for (int q = 0; q < v.nqp; ++q) v.pf[(size_t)w * v.nqp + q] = pfn[q];
-        v.log_ip[w] = lip;
-        ws[1] = 0;
-        ws[2] = v.nsample + 1;
-        ws[7] = 0;
-        for (int k = 0; k < 4; ++k) v.counter[(size_t)w * 4 + k] = 0;
-      }
-    } else if (tid == 0) {
-      ws[7] = 1;
-      atomicAdd(v.nflag + 5, 1);
+      lip = ddm::cr_log(fabs(ip_of(v, v.pf_new + off)));
+      done = lip - lip == 0.0;
     }
-    __syncthreads();
+    ws[7] = done ? 0 : 1;
+    if (!done) return;
+    v.log_ip[w] = lip;
+    ws[1] = 0;
+    ws[2] = v.nsample + 1;
+    for (int k = 0; k < 4; ++k) v.counter[(size_t)w * 4 + k] = 0;
+  } else if (mode == RR_REBUILD) {
+    if (ok) v.log_ip[w] = ddm::cr_log(fabs(ip_of(v, v.pf_new + off)));
+    ws[1] = 0;
+    ws[5] = 0;
+  } else {
+    v.s_valid[(size_t)w * v.nsample + s] = ok ? 1 : 0;
   }
+  if (ok)
+    for (int q = 0; q < v.nqp; ++q) v.pf[off + q] = v.pf_new[off + q];
 }
 
-// Measurement rebuild of saved sample s (as k_meas_rebuild) with the
-// register-resident Pfaffian + inverse, walkers blockIdx.x, + gridDim.x, ...
-// (T x T workgroups)
-template <int T, int R, bool FULL>
-__global__ void __launch_bounds__(T * T) k_meas_rebuild_rr(EnsView v, int s) {
-  extern __shared__ __align__(16) char lds[];
-  Carver c{lds};
-  int* ei = c.take<int>(v.n);
-  int* rs = c.take<int>(v.n);
-  double* pfn = c.take<double>(v.nqp);
-  RrLds L = carve_rr(c, v.n);
-  const int tid = threadIdx.x;
-  double* gs = v.work + (size_t)blockIdx.x * 2 * v.n * v.n;
-  __shared__ int flag;
-  for (int w = blockIdx.x; w < v.W; w += gridDim.x) {
-    const size_t ws = (size_t)w * v.nsample + s;
-    for (int i = tid; i < v.n; i += blockDim.x) ei[i] = v.s_idx[ws * v.n + i];
-    __syncthreads();
-    if (tid == 0) {
-      int all0 = 1, allneg = 1;
-      for (int k = 0; k < v.n; ++k) { all0 &= (ei[k] == 0); allneg &= (ei[k] < 0); }
-      flag = (all0 || allneg) ? 0 : 1;
-    }
-    __syncthreads();
-    int valid = flag;
-    if (valid) {
-      double* planes = v.inv + (size_t)w * v.nqp * v.n * v.n;
-      valid = !rr_calc_m_all<T, R, FULL>(v, ei, rs, planes, gs, L, pfn);
-    }
-    if (tid == 0) {
-      v.s_valid[ws] = valid;
-      if (valid)
-        for (int q = 0; q < v.nqp; ++q) v.pf[(size_t)w * v.nqp + q] = pfn[q];
-    }
-    __syncthreads();
-  }
+__global__ void k_rr_finish(EnsView v, int mode, int s) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= (mode == RR_REBUILD ? *v.nflag : v.W)) return;
+  rr_finish_walker(v, mode, s, mode == RR_REBUILD ? v.rlist[k] : k);
+}
+
+// The same over a group's queue entries (a rebuild takes those whose walker
+// waits for one).
+__global__ void k_rr_finish_q(GroupArgs ga, int mode, int s) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= ga.qstart[ga.nruns]) return;
+  int w = 0;
+  const EnsView& v = ga.views[queue_run(ga, e, w)];
+  if (!v.by_plane || (mode == RR_REBUILD && !v.wstate[(size_t)w * 8 + 5])) return;
+  rr_finish_walker(v, mode, s, w);
 }
 
 // Batched Pfaffian + inverse: plane group g = np consecutive planes; the

@@ -6,71 +6,153 @@
 // sequence of that order (bit-identical to the sequential loops; built with
 // -ffp-contract=off).
 //
-// Layout: T x T threads, thread (a, b) = (tid % T, tid / T) owns the
-// elements (i, j) = (a + T ri, b + T cj) of the plane.  Panel form (n > 64,
-// T = 32): only the strict upper triangle is ever needed (the elimination
-// reads it, the inverse's panel path forms the upper triangle and fills the
-// lower by skew symmetry), and (i, j) with cj > ri is always upper, cj < ri
-// never, cj == ri iff b > a: a thread keeps the R(R+1)/2 slots cj >= ri in
-// registers.  Full form (n <= 64, T = 16, the whole plane held on chip):
-// utu2inv's small-matrix path multiplies the whole solved matrix, so a
-// thread keeps all R^2 slots (the elimination still uses the upper ones).
-// Steps exchange rows and columns through LDS vectors; the trtri result M
-// and the solved C go to a per-workgroup global scratch (row-major) from
-// which the product reads one row of each per step.  The matrix is read once
-// (gathered from the source) and the inverse written once.
+// For the sizes whose triangle does not fit a CU's LDS several times
+// (pfinv_lds.h serves the smaller ones): T x T threads, thread (a, b) =
+// (tid % T, tid / T) owns the elements (i, j) = (a + T ri, b + T cj) of the
+// plane's upper triangle and keeps them in registers.
+//
+// What bounds it is the dependent chain of n elimination steps, so the
+// design cuts what a step waits for:
+//   - one exchange through LDS and one barrier per step.  The pivot column
+//     of a step is the y column of the step before, so its search, the
+//     pivot's reciprocal and the x column come from the copy already in LDS,
+//     the swapped column is staged straight into y, and every wave searches
+//     the pivot by itself (16 waves per plane searching cost more than they
+//     save: n = 224 0.6x; 4 waves, T = 16, it is);
+//   - the block of the step's column picks one of R code bodies whose slots
+//     and bounds are compile-time constants (no per-element tests inside).
+// Measured: 2048 planes of n = 144 7470 -> 4000 us, 1024 of n = 224
+// 8580 -> 7200 us (before: 1024 threads a plane, two barriers a step),
+// complex 768 of n = 144 4080 -> 3190 us.
 #pragma once
 #include "common.h"
 
-// needs Carver and rnd16 (ensemble.hip) before inclusion
+// on the kernel's lambdas: a call would put the register slots into memory
+#define RR_INLINE __attribute__((always_inline))
 
 namespace mvmc_hip {
 
-constexpr int RR_T = 32;      // threads per side of the panel form (1024 per workgroup)
-constexpr int RR_TS = 16;     // threads per side of the full form (256 per workgroup)
-constexpr int RR_NMAX = 224;  // largest n (R = 7 slots per side)
+constexpr int RR_NMAX = 224;  // largest n
 constexpr int RR_NFULL = 64;  // largest n of the full form (utu2inv's small-matrix path)
 
-// LDS of one plane: 11 vectors of n scalars (real or complex), 2 of n
-// ints, scalars.
+// Orders the LDS traffic of the T x T workgroup: a barrier, or for the
+// single wave of T = 8, whose LDS operations complete in order, only a fence
+// for the compiler.
+template <int T>
+__device__ __forceinline__ void rr_sync() {
+  if constexpr (T == 8) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// Keeps the compiler from merging the tails of sibling branches: merged code
+// would index the register slots by a run-time choice, i.e. through memory.
+#define RR_APART(tag) asm volatile("; branch %0" ::"n"(tag))
+
+// Calls f.template operator()<k>() for the run-time k of [LO, HI).
+template <int LO, int HI, class F>
+__device__ __forceinline__ void rr_case(int k, F&& f) {
+  if constexpr (LO + 1 == HI) {
+    f.template operator()<LO>();
+    RR_APART(LO);
+  } else {
+    constexpr int M = (LO + HI) / 2;
+    if (k < M) rr_case<LO, M>(k, f);
+    else rr_case<M, HI>(k, f);
+  }
+}
+
+// for (X = LO; X < HI; ++X) with X a compile-time constant in the body:
+// RR_FOR(X, LO, HI) { ... };  The register slots are indexed only by such
+// constants from the start: left to the loop unroller, they end in memory.
+template <int LO, int HI>
+struct RrRange {
+  template <class F>
+  __device__ __forceinline__ void operator<<(F&& f) const {
+    if constexpr (LO < HI) {
+      f.template operator()<LO>();
+      RrRange<LO + 1, HI>{} << f;
+    }
+  }
+};
+#define RR_FOR(X, LO, HI) RrRange<(LO), (HI)>{} << [&]<int X>() RR_INLINE
+
+// Maximum over the wave's lanes (no NaN), in every lane.
+__device__ __forceinline__ double rr_wave_max(double x) {
+#define RR_DPP_MAX(ctrl)                                                                             \
+  do {                                                                                               \
+    const int lo_ = __double2loint(x), hi_ = __double2hiint(x);                                      \
+    const double y_ = __hiloint2double(__builtin_amdgcn_update_dpp(hi_, hi_, ctrl, 0xf, 0xf, false), \
+                                       __builtin_amdgcn_update_dpp(lo_, lo_, ctrl, 0xf, 0xf, false)); \
+    x = y_ > x ? y_ : x;                                                                             \
+  } while (0)
+  RR_DPP_MAX(0x111);  // row_shr:1, 2, 4, 8: lane 15 of each row of 16 has the row's maximum
+  RR_DPP_MAX(0x112);
+  RR_DPP_MAX(0x114);
+  RR_DPP_MAX(0x118);
+  RR_DPP_MAX(0x142);  // row_bcast:15, row_bcast:31: lane 63 has the wave's
+  RR_DPP_MAX(0x143);
+#undef RR_DPP_MAX
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                          __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+
+// LDS of one plane.  `vec`: the step vectors (two sets by step parity when
+// several waves share the plane: a fast wave may write the next step's while
+// a slow one still reads this step's), reused as the row blocks of the solve
+// (full form), of the product and of the output.
+constexpr int rr_vl(int T, int R) { return (T * R + 63) / 64 * 64; }  // padded vector length
+constexpr int rr_sets(int T) { return T == 8 ? 1 : 2; }
+// row stride of the T-row blocks: T lanes of a row beside the next row's
+constexpr int rr_ldb(int T, int R) { return rr_vl(T, R) + T; }
+// scalars of `vec`: 2 y columns, then per set x, u, r1, r2
+constexpr int rr_vec_len(int T, int R, bool FULL) {
+  const int step = (2 + 4 * rr_sets(T)) * rr_vl(T, R);
+  const int blocks = (FULL ? 1 : 2) * T * rr_ldb(T, R);
+  return step > blocks ? step : blocks;
+}
+// packed strict upper triangle of M, columns up to n - 2 (full form)
+__host__ __device__ constexpr int rr_m_len(int n) { return n > 2 ? (n - 1) * (n - 2) / 2 : 0; }
+
 template <class S>
 struct RrLdsT {
-  S *v0, *v1, *v2, *v3, *buf0, *buf1, *buf2, *buf3;
+  S* vec;
   S* sup;          // the superdiagonal A(i, i+1) after the LTL
   S *rneg, *rpos;  // complex solve: reciprocals of -vt[i] and vt[i]
-  int *piv, *perm;
-  int* si;     // [16] ints: 2 info, 4..7 pivot results by step parity
-  S* sa;       // [4] scalars: 0, 1 alpha by step parity, 2 the Pfaffian
-  double* sd;  // [32] doubles: 16.. max |a|^2 per wave
+  S* m;            // full form: M packed
+  S* sa;           // [1] the Pfaffian
+  int* finv;       // inverse of the output permutation
+  double* sd;      // [16] max |a|^2 per wave
 };
 using RrLds = RrLdsT<double>;
 
-template <class S = double>
-__host__ __device__ inline size_t rr_lds_bytes(int n) {
-  return 11 * rnd16((size_t)n * sizeof(S)) + 2 * rnd16((size_t)n * 4) + 16 * 4 + rnd16(4 * sizeof(S)) + 32 * 8;
+template <class S, bool RECIP>
+__host__ __device__ inline size_t rr_lds_bytes(int T, int R, bool full, int n) {
+  const int nw = T * T / 64;
+  return rnd16((size_t)rr_vec_len(T, R, full) * sizeof(S)) + rnd16((size_t)n * sizeof(S)) * (RECIP ? 3 : 1) +
+         (full ? rnd16((size_t)rr_m_len(n) * sizeof(S)) : 0) + 16 + rnd16((size_t)n * 4) + rnd16((size_t)nw * 8);
 }
 
-template <class S = double, class Carver>
+template <class S, bool RECIP, int T, int R, bool FULL, class Carver>
 __device__ inline RrLdsT<S> carve_rr(Carver& c, int n) {
   RrLdsT<S> L;
-  L.v0 = c.template take<S>(n);
-  L.v1 = c.template take<S>(n);
-  L.v2 = c.template take<S>(n);
-  L.v3 = c.template take<S>(n);
-  L.buf0 = c.template take<S>(n);
-  L.buf1 = c.template take<S>(n);
-  L.buf2 = c.template take<S>(n);
-  L.buf3 = c.template take<S>(n);
+  L.vec = c.template take<S>(rr_vec_len(T, R, FULL));
   L.sup = c.template take<S>(n);
-  L.rneg = c.template take<S>(n);
-  L.rpos = c.template take<S>(n);
-  L.piv = c.template take<int>(n);
-  L.perm = c.template take<int>(n);
-  L.si = c.template take<int>(16);
-  L.sa = c.template take<S>(4);
-  L.sd = c.template take<double>(32);
+  L.rneg = RECIP ? c.template take<S>(n) : nullptr;
+  L.rpos = RECIP ? c.template take<S>(n) : nullptr;
+  L.m = FULL ? c.template take<S>(rr_m_len(n)) : nullptr;
+  L.sa = c.template take<S>(1);
+  L.finv = c.template take<int>(n);
+  L.sd = c.template take<double>(T * T / 64);
   return L;
 }
+
+// Scratch in global memory per workgroup, in scalars: M and C of the panel
+// form; the full form needs none.
+__host__ __device__ inline size_t rr_scratch_len(bool full, int n) { return full ? 0 : (size_t)2 * n * n; }
 
 // Slot of block (ri, cj): packed upper block triangle (cj >= ri) in the
 // panel form, row-major R x R in the full form.
@@ -99,285 +181,314 @@ struct RrReal {
   static __device__ __forceinline__ S mul(S x, S y) { return x * y; }
   static __device__ __forceinline__ double mag2(S x) { return x * x; }
   static __device__ __forceinline__ double key(S x, int i) { return rr_key(fabs(x), i); }
-  static __device__ __forceinline__ S alpha(S pivot) { return 1.0 / pivot; }
+  __device__ __forceinline__ S alpha(S pivot) const { return 1.0 / pivot; }
   // rank-2 update of one element: (c + x_i t1) - y_i t2
   static __device__ __forceinline__ S update(S c, S xi, S yi, S t1, S t2) { return (c + xi * t1) - yi * t2; }
-  static __device__ __forceinline__ S scale(S x, S alpha) { return x * alpha; }
+  __device__ __forceinline__ S scale(S x, S alpha) const { return x * alpha; }
   static __device__ __forceinline__ S sign(bool neg) { return neg ? (0.0 - 1.0) : 1.0; }
   static __device__ __forceinline__ bool finite(S x) { return isfinite(x); }
   // solve: num / -vt (forward), num / vt (backward)
   static __device__ __forceinline__ S div_negvt(S num, S vt, S) { return num / -vt; }
   static __device__ __forceinline__ S div_vt(S num, S vt, S) { return num / vt; }
   static __device__ __forceinline__ S recip(S x) { return 1.0 / x; }
+  static __device__ __forceinline__ S readlane(S x, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                            __builtin_amdgcn_readlane(__double2loint(x), l));
+  }
 };
 
 // One plane.  src(i, j) gives A(i, j) (any i, j < n).  On exit: info (0 ok,
 // k > 0 zero pivot at 1-based row k, -1 non-finite Pfaffian), pf (the
 // Pfaffian; on a zero pivot not formed), and for info == 0 the plane `out`
-// (column-major, element (r, c) at r + c n) holds sign * A^{-1}.  allzero
-// (when check_zero) reports max |a|^2 < 1e-28 over the whole plane, in which
-// case nothing else is done.  gs: 2 n^2 doubles of global scratch.  Every
-// thread of the T x T workgroup (blockDim.x == T * T) calls it.  FULL: the
-// full form (n <= 64), else the panel form (n > 64).
-template <int T, int R, bool FULL, class Ar = RrReal, class Src>
-__device__ __forceinline__ void rr_pfinv(Src src, int n, typename Ar::S* out, double sign, typename Ar::S* gs,
-                                         RrLdsT<typename Ar::S>& L, typename Ar::S& pf, int& info, bool check_zero,
-                                         bool& allzero) {
+// (column-major, element (r, c) at r + c n) holds sign * A^{-1} (and out32,
+// if set, the same rounded to FP32).  allzero (when check_zero) reports
+// max |a|^2 < 1e-28 over the whole plane, in which case nothing else is
+// done.  gs: rr_scratch_len scalars of global scratch.  Every thread of the
+// T x T workgroup (blockDim.x == T * T) calls it; the results are uniform.
+// FULL: the full form (n <= 64), else the panel form (n > 64).
+// T (R - 1) < n <= T R.
+template <int T, int R, bool FULL, class Ar, class Src>
+__device__ __forceinline__ void rr_pfinv(const Ar& ar, Src src, int n, typename Ar::S* out, float* out32, double sign,
+                                         typename Ar::S* gs, RrLdsT<typename Ar::S>& L, typename Ar::S& pf, int& info,
+                                         bool check_zero, bool& allzero) {
   using S = typename Ar::S;
   constexpr int NS = FULL ? R * R : R * (R + 1) / 2;
-  const int tid = threadIdx.x, NT = T * T;
+  constexpr int NT = T * T, VL = rr_vl(T, R), LDB = rr_ldb(T, R), SETS = rr_sets(T), Q = VL / 64;
+  constexpr int JC = (T * R + NT - 1) / NT;  // columns per thread where a thread owns whole columns
+  const int tid = threadIdx.x, lane = tid & 63;
   const int a0 = tid % T, b0 = tid / T;
-  // per-step copies of (a, b) the compiler cannot prove loop-invariant: the
-  // per-slot row/column indices are recomputed in each step instead of being
-  // kept live across the whole elimination (registers hold the slots)
+  // copies of (a, b) the compiler cannot prove loop-invariant: the index
+  // arithmetic of a step is formed in the step instead of being kept live
+  // across the elimination (the registers hold the slots)
   int a = a0, b = b0;
-#define RR_FRESH() \
-  do {             \
-    a = a0;        \
-    b = b0;        \
+#define RR_FRESH()                       \
+  do {                                   \
+    a = a0;                              \
+    b = b0;                              \
     asm volatile("" : "+v"(a), "+v"(b)); \
   } while (0)
   S c[NS];
+#define RC(ri, cj) c[rr_slot<R, FULL>(ri, cj)]
 #ifdef MVMC_PHASE_CLOCKS
-  long long rr_t0 = wall_clock64(), rr_ph[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  long long rr_s0 = 0, rr_sub[4] = {0, 0, 0, 0};
-#define RR_SUB(k)                        \
-  do {                                   \
-    const long long t_ = wall_clock64(); \
-    rr_sub[k] += t_ - rr_s0;             \
-    rr_s0 = t_;                          \
-  } while (0)
-#define RR_PHASE(k)                           \
-  do {                                        \
-    const long long t_ = wall_clock64();      \
-    rr_ph[k] += t_ - rr_t0;                   \
-    rr_t0 = t_;                               \
+  long long rr_t0 = __builtin_readcyclecounter(), rr_ph[12] = {};
+#define RR_PHASE(k)                                         \
+  do {                                                      \
+    const long long t_ = __builtin_readcyclecounter();      \
+    rr_ph[k] += t_ - rr_t0;                                 \
+    rr_t0 = t_;                                             \
   } while (0)
 #else
 #define RR_PHASE(k) \
   do {              \
   } while (0)
-#define RR_SUB(k) \
-  do {            \
-  } while (0)
 #endif
-  // ---- gather (and the all-zero guard over every element, pfaffian.rs:884-890) ----
+  // ---- gather (and the all-zero guard, pfaffian.rs:884-890: the plane is skew, so the upper half decides) ----
   double mx = 0.0;
-#pragma unroll
-  for (int ri = 0; ri < R; ++ri)
-#pragma unroll
-    for (int cj = ri; cj < R; ++cj) {
+RR_FOR(ri, 0, R) {
+RR_FOR(cj, FULL ? 0 : ri, R) {
       const int i = a + T * ri, j = b + T * cj;
       S x = Ar::zero();
-      if (i < n && j < n && i <= j) {
+      if (cj >= ri && i < n && j < n && i <= j) {
         x = src(i, j);
-        if (check_zero) {
-          const S y = src(j, i);
-          mx = fmax(mx, fmax(Ar::mag2(x), Ar::mag2(y)));
-        }
+        mx = fmax(mx, Ar::mag2(x));
       }
-      c[rr_slot<R, FULL>(ri, cj)] = x;
-    }
-  if (FULL) {
-#pragma unroll
-    for (int ri = 1; ri < R; ++ri)
-#pragma unroll
-      for (int cj = 0; cj < ri; ++cj) c[rr_slot<R, FULL>(ri, cj)] = Ar::zero();
-  }
-  for (int i = tid; i < n; i += NT) L.piv[i] = i + 1;
-  if (tid == 0) L.si[2] = 0;
+      RC(ri, cj) = x;
+    };
+  };
   if (check_zero) {
-    for (int off = 32; off >= 1; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-    if ((tid & 63) == 0) L.sd[16 + (tid >> 6)] = mx;
+    mx = rr_wave_max(mx);
+    if (lane == 0) L.sd[tid >> 6] = mx;
     __syncthreads();
     double m = 0.0;
-    for (int k = 0; k < NT / 64; ++k) m = fmax(m, L.sd[16 + k]);
+    for (int k = 0; k < NT / 64; ++k) m = fmax(m, L.sd[k]);
     allzero = m < 1.0e-28;
     __syncthreads();
     if (allzero) return;
   } else {
     allzero = false;
-    __syncthreads();
   }
-
-  // Slots of one block column / block row: f(global row or column index,
-  // slot) for the lanes that own that column (b == col % T) or row; the block
-  // index is uniform, so the other blocks' code is branched over.
-  auto for_col = [&](int col, auto f) {
-    if (b != col % T) return;
-    const int kc = col / T;
-#pragma unroll
-    for (int cj = 0; cj < R; ++cj)
-      if (cj == kc) {
-#pragma unroll
-        for (int ri = 0; ri <= cj; ++ri) f(a + T * ri, c[rr_slot<R, FULL>(ri, cj)]);
-      }
-  };
-  auto for_row = [&](int row, auto f) {
-    if (a != row % T) return;
-    const int kr = row / T;
-#pragma unroll
-    for (int ri = 0; ri < R; ++ri)
-      if (ri == kr) {
-#pragma unroll
-        for (int cj = ri; cj < R; ++cj) f(b + T * cj, c[rr_slot<R, FULL>(ri, cj)]);
-      }
-  };
+  S* const y0 = L.vec;
+  auto setv = [&](int par, int k) { return L.vec + (2 + (SETS == 2 ? 4 * par : 0) + k) * VL; };
 
   RR_PHASE(0);
   // ---- dsktf2: k0 = n-1 .. 1 ----
-  // The pivot column of step k0 - 1 is column kk0 as swapped in step k0,
-  // which the rank-2 update of step k0 does not touch: its search runs
-  // before that update (look-ahead), so a step is swap staging | swap
-  // write-back + staging of x, y, alpha + next pivot | update.  Pivot
-  // results, x / y and alpha alternate between two LDS sets by step parity.
-  auto pivot_search = [&](int col, int par) {
-    if (b != col % T) return;
-    const int kk = col - 1;
-    double best = -2.0;
-    int bi = 0x7fffffff;
-    const int kc = col / T;
+  // first largest key of yv[0 .. m), each wave by itself
+  auto pivot = [&](const S* yv, int m, int& kp, bool& zero) RR_INLINE {
+    double key[Q], best = -2.0;
 #pragma unroll
-    for (int cj = 0; cj < R; ++cj)
-      if (cj == kc) {
-#pragma unroll
-        for (int ri = 0; ri <= cj; ++ri) {
-          const int i = a + T * ri;
-          if (i <= kk) {
-            const double key = Ar::key(c[rr_slot<R, FULL>(ri, cj)], i);
-            if (key > best) { best = key; bi = i; }
-          }
-        }
-      }
-#pragma unroll
-    for (int off = T / 2; off >= 1; off >>= 1) {
-      const double ob = __shfl_xor(best, off, 64);
-      const int oi = __shfl_xor(bi, off, 64);
-      if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+    for (int q = 0; q < Q; ++q) {
+      const int i = lane + 64 * q;
+      key[q] = i < m ? Ar::key(yv[i], i) : -2.0;
+      best = key[q] > best ? key[q] : best;
     }
-    if (a == 0) {
-      L.si[4 + 2 * par] = bi;
-      L.si[5 + 2 * par] = best == 0.0 ? 1 : 0;
+    best = rr_wave_max(best);
+    kp = 0;
+#pragma unroll
+    for (int q = Q - 1; q >= 0; --q) {
+      const unsigned long long hit = __ballot(key[q] == best);
+      if (hit) kp = 64 * q + (int)__builtin_ctzll(hit);
     }
+    zero = best == 0.0;
   };
-  pivot_search(n - 1, (n - 1) & 1);
-  __syncthreads();
-  for (int k0 = n - 1; k0 >= 1; --k0) {
-    const int kk0 = k0 - 1;
-    const int par = k0 & 1;
-    RR_FRESH();
-#ifdef MVMC_PHASE_CLOCKS
-    rr_s0 = wall_clock64();
-#endif
-    const int kp = L.si[4 + 2 * par];
-    if (L.si[5 + 2 * par]) {
-      // zero column: INFO records the first, the step is skipped
-      if (tid == 0) {
-        if (L.si[2] == 0) L.si[2] = kk0 + 1;
-        L.piv[kk0] = kk0 + 1;
-      }
-      if (kk0 >= 1) pivot_search(kk0, par ^ 1);
-      __syncthreads();
-      continue;
-    }
-    if (kp != kk0) {
-      // interchange rows/columns kk0 and kp in the upper triangle with the
-      // sign twiddles: stage column kk0 (rows < kk0), column kp (rows < kp),
-      // row kp (columns > kp), row kk0 (columns >= k0)
-      for_col(kk0, [&](int i, S& x) { if (i < kk0) L.v0[i] = x; });
-      for_col(kp, [&](int i, S& x) { if (i < kp) L.v1[i] = x; });
-      for_row(kp, [&](int j, S& x) { if (j > kp && j < n) L.v2[j] = x; });
-      for_row(kk0, [&](int j, S& x) { if (j >= k0 && j < n) L.v3[j] = x; });
-      __syncthreads();
-      RR_SUB(1);
-      // write-back; the four groups target disjoint elements
-      for_col(kk0, [&](int i, S& x) {
-        if (i < kp) x = L.v1[i];
-        else if (i == kp) x = Ar::neg(L.v0[kp]);
-        else if (i < kk0) x = Ar::neg(L.v2[i]);
+  info = 0;
+  // the last column, the first pivot column
+  {
+    const int k = n - 1;
+    if (b == k % T)
+      rr_case<0, R>(k / T, [&]<int K>() RR_INLINE {
+RR_FOR(ri, 0, K + 1) { y0[a + T * ri] = RC(ri, K);
+        };
       });
-      for_col(kp, [&](int i, S& x) { if (i < kp) x = L.v0[i]; });
-      for_row(kp, [&](int j, S& x) {
-        if (j > kp && j < kk0) x = Ar::neg(L.v0[j]);
-        else if (j >= k0 && j < n) x = L.v3[j];
-      });
-      for_row(kk0, [&](int j, S& x) { if (j >= k0 && j < n) x = L.v2[j]; });
-    }
-    if (tid == 0) L.piv[kk0] = kp + 1;
-    if (kk0 >= 1) {
-      // rank-2 update of the leading kk0 x kk0 block with x = column k0,
-      // y = column kk0 (as swapped), alpha = 1 / A(kk0, k0)
-      S* xs = par ? L.buf0 : L.buf2;
-      S* ys = par ? L.buf1 : L.buf3;
-      for_col(k0, [&](int i, S& x) {
-        if (i < kk0) xs[i] = x;
-        else if (i == kk0) L.sa[par] = Ar::alpha(x);
-      });
-      for_col(kk0, [&](int i, S& x) { if (i < kk0) ys[i] = x; });
-      pivot_search(kk0, par ^ 1);
-      __syncthreads();
-      RR_SUB(2);
-      const S alpha = L.sa[par];
-#pragma unroll
-      for (int cj = 0; cj < R; ++cj)
-        if (T * cj < kk0) {
-          const int j = b + T * cj;
-          if (j < kk0) {
-            const S t1 = Ar::mul(alpha, ys[j]);
-            const S t2 = Ar::mul(alpha, xs[j]);
-#pragma unroll
-            for (int ri = 0; ri <= cj; ++ri) {
-              const int i = a + T * ri;
-              S& x = c[rr_slot<R, FULL>(ri, cj)];
-              if (i < j) x = Ar::update(x, xs[i], ys[i], t1, t2);
-              else if (i == j) x = Ar::zero();
-            }
-          }
-        }
-      // scale column k0 (its pre-scale values were staged in xs)
-      for_col(k0, [&](int i, S& x) { if (i < kk0) x = Ar::scale(x, alpha); });
-      RR_SUB(3);
-    }
   }
-  __syncthreads();
-  RR_PHASE(1);
-  info = L.si[2];
+  rr_sync<T>();
+  int f[JC];  // the output permutation: position r holds index f(r); the swaps composed as they come
+#pragma unroll
+  for (int u = 0; u < JC; ++u) f[u] = tid + NT * u;
+  bool neg = false;  // parity of the interchanges
+  int kp = 0;
+  bool zero = false;
+  pivot(y0, n - 1, kp, zero);
+  S xk = y0[kp];
+  for (int k0 = n - 1; k0 >= 1; --k0) {
+    const int kk0 = k0 - 1, par = k0 & 1;  // n is even: k0 = n - 1 reads y0, writes y1
+    RR_FRESH();
+    if (zero) {  // zero pivot column: the plane has no Pfaffian form to go on with
+      info = kk0 + 1;
+      break;
+    }
+    if (tid == 0) L.sup[kk0] = xk;
+    if (kp != kk0) {
+      neg = !neg;
+#pragma unroll
+      for (int u = 0; u < JC; ++u) f[u] = f[u] == kk0 ? kp : f[u] == kp ? kk0 : f[u];
+    }
+    if (kk0 == 0) break;
+    const S* yp = L.vec + (par ? 0 : VL);
+    S* yn = L.vec + (par ? VL : 0);
+    S* xs = setv(par, 0);
+    S* us = setv(par, 1);
+    S* r1 = setv(par, 2);
+    S* r2 = setv(par, 3);
+    const int K0 = kk0 / T, kb = kk0 % T;
+    // stage: x = column k0 with its rows kk0 and kp interchanged (column k0
+    // is y of the step before), u = column kk0, y = column kk0 after the
+    // interchange of rows/columns kk0 and kp in the upper triangle (with the
+    // sign twiddles), r1 / r2 = rows kp / kk0 in the columns >= k0
+#pragma unroll
+    for (int q = 0; q < (VL + NT - 1) / NT; ++q) {
+      const int i = tid + NT * q;
+      if (i < kk0) xs[i] = yp[i == kp ? kk0 : i];
+    }
+    if (kp == kk0) {
+      rr_case<0, R>(K0, [&]<int K>() RR_INLINE {
+        if (b == kb) {
+RR_FOR(ri, 0, K + 1) { yn[a + T * ri] = RC(ri, K);
+          };
+        }
+      });
+    } else {
+      rr_case<0, R>(K0, [&]<int K>() RR_INLINE {
+        if (b == kb) {
+RR_FOR(ri, 0, K + 1) {
+            const int i = a + T * ri;
+            us[i] = RC(ri, K);
+            if (i == kp) yn[i] = Ar::neg(RC(ri, K));
+          };
+        }
+        if (a == kb) {
+RR_FOR(cj, K, R) { r2[b + T * cj] = RC(K, cj);
+          };
+        }
+      });
+      const int kpb = kp % T;
+      rr_case<0, R>(kp / T, [&]<int P>() RR_INLINE {
+        if (b == kpb) {
+RR_FOR(ri, 0, P + 1) {
+            if (ri < P || a < kpb) yn[a + T * ri] = RC(ri, P);
+          };
+        }
+        if (a == kpb) {
+RR_FOR(cj, P, R) {
+            const int j = b + T * cj;
+            if (cj > P || b > kpb) {
+              if (j < kk0) yn[j] = Ar::neg(RC(P, cj));
+              else r1[j] = RC(P, cj);
+            }
+          };
+        }
+      });
+    }
+    RR_PHASE(1);  // stage
+    rr_sync<T>();
+    const S alpha = ar.alpha(xk);
+    // the next step's pivot column is y, which this step's update leaves alone
+    const int kpc = kp;
+    pivot(yn, kk0, kp, zero);
+    xk = yn[kp];
+    RR_PHASE(2);
+    if (kpc != kk0) {
+      const int kpb = kpc % T;
+      rr_case<0, R>(kpc / T, [&]<int P>() RR_INLINE {
+        if (b == kpb) {
+RR_FOR(ri, 0, P + 1) {
+            if (ri < P || a < kpb) RC(ri, P) = us[a + T * ri];
+          };
+        }
+        if (a == kpb) {
+RR_FOR(cj, P, R) {
+            const int j = b + T * cj;
+            const S w = j < kk0 ? Ar::neg(us[j]) : r2[j];
+            if (cj > P || b > kpb) RC(P, cj) = w;  // column kk0 follows below
+          };
+        }
+      });
+    }
+    RR_PHASE(3);
+    rr_case<0, R>(K0, [&]<int K>() RR_INLINE {
+      S xi[K + 1], yi[K + 1];
+RR_FOR(ri, 0, K + 1) {
+        xi[ri] = xs[a + T * ri];
+        yi[ri] = yn[a + T * ri];
+      };
+      if (kpc != kk0) {
+        if (b == kb) {
+RR_FOR(ri, 0, K + 1) {
+            if (ri < K || a < kb) RC(ri, K) = yi[ri];
+          };
+        }
+        if (a == kb) {
+RR_FOR(cj, K, R) {
+            if (cj > K || b > kb) RC(K, cj) = r1[b + T * cj];
+          };
+        }
+      }
+      // rank-2 update of the leading kk0 x kk0 block (elements on and below
+      // the diagonal of a diagonal block are never read)
+RR_FOR(cj, 0, K + 1) {
+        const S yj = yn[b + T * cj], xj = xs[b + T * cj];
+        const S t1 = Ar::mul(alpha, yj), t2 = Ar::mul(alpha, xj);
+        if (cj < K || b < kb) {
+RR_FOR(ri, 0, cj + 1) { RC(ri, cj) = Ar::update(RC(ri, cj), xi[ri], yi[ri], t1, t2);
+          };
+        }
+      };
+      // column k0 scaled (its rows are x)
+      if (kb + 1 < T) {
+        if (b == kb + 1) {
+RR_FOR(ri, 0, K + 1) {
+            if (ri < K || a < kb) RC(ri, K) = ar.scale(xi[ri], alpha);
+          };
+        }
+        RR_APART(K + 100);
+      } else if constexpr (K + 1 < R) {
+        if (b == 0) {
+RR_FOR(ri, 0, K + 1) {
+            if (ri < K || a < kb) RC(ri, K + 1) = ar.scale(xi[ri], alpha);
+          };
+        }
+      }
+    });
+    RR_PHASE(4);
+  }
   if (info != 0) {
     pf = Ar::zero();
+    __syncthreads();
     return;
   }
-  // ---- utu2pfa: product of A(i, i+1), i even, sign by the count of moves ----
-  // (the superdiagonal also gives vt = -A(i, i+1) of the solve: sup)
-#pragma unroll
-  for (int ri = 0; ri < R; ++ri)
-#pragma unroll
-    for (int cj = ri; cj < R; ++cj) {
-      const int i = a + T * ri, j = b + T * cj;
-      if (j == i + 1 && j < n) L.sup[i] = c[rr_slot<R, FULL>(ri, cj)];
-    }
   __syncthreads();
+  RR_PHASE(4);
+  // ---- utu2pfa: product of A(i, i+1), i even, sign by the count of moves ----
   if (tid == 0) {
     S p = Ar::one();
-    for (int i = 0; i + 1 < n; i += 2) p = Ar::mul(p, L.sup[i]);
-    bool neg = false;
-    for (int k = 0; k < n; ++k)
-      if (L.piv[k] != k + 1) neg = !neg;
-    L.sa[2] = Ar::mul(Ar::sign(neg), p);
+    int i = 0;
+    for (; i + 16 <= n; i += 16) {
+      S v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = L.sup[i + 2 * u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) p = Ar::mul(p, v[u]);
+    }
+    for (; i + 1 < n; i += 2) p = Ar::mul(p, L.sup[i]);
+    L.sa[0] = Ar::mul(Ar::sign(neg), p);
   }
-  if (Ar::kRecip)
+  if constexpr (Ar::kRecip)
     for (int i = tid; i + 1 < n; i += NT) {
       const S vt = Ar::neg(L.sup[i]);
       L.rneg[i] = Ar::recip(Ar::neg(vt));
       L.rpos[i] = Ar::recip(vt);
     }
   __syncthreads();
-  pf = L.sa[2];
+  pf = L.sa[0];
   if (!Ar::finite(pf)) {
     info = -1;
+    __syncthreads();
     return;
   }
+#pragma unroll
+  for (int u = 0; u < JC; ++u)
+    if (tid + NT * u < n) L.finv[f[u]] = tid + NT * u;
 
-  RR_PHASE(2);
+  RR_PHASE(5);
   // ---- utu2inv (panel path for n > 64; the full form differs from the
   // solve on) ----
   // trtri('U','U') on B(i, j) = A(i, j+1), 0 <= i < j <= n-2: at step k the
@@ -387,212 +498,318 @@ __device__ __forceinline__ void rr_pfinv(Src src, int n, typename Ar::S* out, do
   // ascending order, as the row-chain loops do.
   for (int k = 1; k <= n - 2; ++k) {
     RR_FRESH();
-    S* U = (k & 1) ? L.v0 : L.v2;   // column k of the inverse, rows < k
-    S* Bk = (k & 1) ? L.v1 : L.v3;  // row k of B (columns > k)
-    for_col(k + 1, [&](int i, S& x) {
-      if (i < k) {
-        x = Ar::neg(x);
-        U[i] = x;
+    S* U = setv(k & 1, 0);   // column k of the inverse, rows < k
+    S* Bk = setv(k & 1, 1);  // row k of B by plane column (> k + 1)
+    const int kb = k % T;
+    rr_case<0, R>(k / T, [&]<int K>() RR_INLINE {
+      if (kb + 1 < T) {
+        if (b == kb + 1) {
+RR_FOR(ri, 0, K + 1) {
+            const S x = Ar::neg(RC(ri, K));
+            U[a + T * ri] = x;
+            if (ri < K || a < kb) RC(ri, K) = x;
+          };
+        }
+        RR_APART(K + 200);
+      } else if constexpr (K + 1 < R) {
+        if (b == 0) {
+RR_FOR(ri, 0, K + 1) {
+            const S x = Ar::neg(RC(ri, K + 1));
+            U[a + T * ri] = x;
+            if (ri < K || a < kb) RC(ri, K + 1) = x;
+          };
+        }
+      }
+      if (a == kb) {
+RR_FOR(cj, K, R) { Bk[b + T * cj] = RC(K, cj);
+        };
       }
     });
-    for_row(k, [&](int jj, S& x) { if (jj >= k + 2 && jj < n) Bk[jj - 1] = x; });
-    __syncthreads();
-    if (k <= n - 3) {
-#pragma unroll
-      for (int ri = 0; ri < R; ++ri)
-        if (T * ri < k) {
-#pragma unroll
-          for (int cj = ri; cj < R; ++cj)
-            if (T * cj + T > k + 2) {
-              const int i = a + T * ri, jj = b + T * cj;
-              if (i < k && jj >= k + 2 && jj < n) {
-                S& x = c[rr_slot<R, FULL>(ri, cj)];
-                x = Ar::add(x, Ar::mul(U[i], Bk[jj - 1]));
-              }
-            }
-        }
-    }
+    rr_sync<T>();
+    if (k <= n - 3)
+      rr_case<0, R>(k / T, [&]<int K>() RR_INLINE {
+        S ui[K + 1];
+RR_FOR(ri, 0, K + 1) { ui[ri] = U[a + T * ri];
+        };
+RR_FOR(cj, K, R) {
+          const S bj = Bk[b + T * cj];
+          if (cj > K + 1 || b + T * cj >= k + 2) {
+RR_FOR(ri, 0, K) { RC(ri, cj) = Ar::add(RC(ri, cj), Ar::mul(ui[ri], bj));
+            };
+            if (a < kb) RC(K, cj) = Ar::add(RC(K, cj), Ar::mul(ui[K], bj));
+          }
+        };
+      });
   }
-  __syncthreads();
-  RR_PHASE(3);
+  RR_PHASE(6);
   // M (unit upper, M(i, j) = Bn(i, j) for i < j <= n-2, M(i, n-1) = 0 for
-  // i < n-1) to gs row-major: gm[i * n + j]
+  // i < n-1): packed in LDS (full form) or row-major in gs
+  auto mrow = [&](int i) { return i * (n - 2) - i * (i - 1) / 2 - i - 1; };  // packed: element (i, m) at mrow(i) + m
   S* gm = gs;
   S* gc = gs + (size_t)n * n;
-  for (int e = tid; e < n * n; e += NT) gm[e] = (e / n == e % n) ? Ar::one() : Ar::zero();
-  __syncthreads();
-#pragma unroll
-  for (int ri = 0; ri < R; ++ri)
-#pragma unroll
-    for (int cj = ri; cj < R; ++cj) {
+  RR_FRESH();
+RR_FOR(ri, 0, R) {
+RR_FOR(cj, ri, R) {
       const int i = a + T * ri, jj = b + T * cj;
-      if (i + 1 < jj && jj < n) gm[(size_t)i * n + (jj - 1)] = c[rr_slot<R, FULL>(ri, cj)];
-    }
-  __syncthreads();
-  RR_PHASE(4);
-  // skew-tridiagonal solve T C = M, all columns at once, row by row through
-  // LDS (vt[i] = -A(i, i+1) = -sup[i]); every row of C goes to gc row-major
-  // and into the registers (panel form: the strict upper part).
-  auto keep_row = [&](int r, const S* row) {
-#pragma unroll
-    for (int ri = 0; ri < R; ++ri)
-      if (a + T * ri == r) {
-#pragma unroll
-        for (int cj = FULL ? 0 : ri; cj < R; ++cj) {
-          const int j = b + T * cj;
-          if ((FULL || r < j) && j < n) c[rr_slot<R, FULL>(ri, cj)] = row[j];
-        }
+      if (i + 1 < jj && jj < n) {
+        if constexpr (FULL) L.m[mrow(i) + jj - 1] = RC(ri, cj);
+        else gm[(size_t)i * n + (jj - 1)] = RC(ri, cj);
       }
+    };
   };
-  {
-    // thread j < n carries column j; the rows of M it reads do not depend on
-    // the chain, so they are loaded two steps ahead
-    const int j = tid;
-    const bool col = j < n;
-    // forward: c[1] = b[0] / -vt[0]; c[i+1] = (b[i] - c[i-1] vt[i-1]) / -vt[i]
-    S m0 = col ? gm[j] : Ar::zero();
-    S m1 = (col && 2 < n) ? gm[(size_t)2 * n + j] : Ar::zero();
-    S m2 = (col && 4 < n) ? gm[(size_t)4 * n + j] : Ar::zero();
-    if (col) {
-      const S vt0 = Ar::neg(L.sup[0]);
-      const S x = Ar::div_negvt(m0, vt0, L.rneg[0]);
-      L.buf0[j] = x;
-      gc[(size_t)1 * n + j] = x;
-    }
-    __syncthreads();
-    keep_row(1, L.buf0);
-    S* prev = L.buf0;
-    S* next = L.buf1;
-    for (int i = 2; i < n; i += 2) {
-      const S mi = m1;
-      m1 = m2;
-      m2 = (col && i + 4 < n) ? gm[(size_t)(i + 4) * n + j] : Ar::zero();
-      const S vtm = Ar::neg(L.sup[i - 1]), vti = Ar::neg(L.sup[i]);
-      if (col) {
-        const S x = Ar::div_negvt(Ar::sub(mi, Ar::mul(prev[j], vtm)), vti, L.rneg[i]);
-        next[j] = x;
-        gc[(size_t)(i + 1) * n + j] = x;
-      }
-      __syncthreads();
-      RR_FRESH();
-      keep_row(i + 1, next);
-      S* t = prev; prev = next; next = t;
-    }
-    __syncthreads();
-    // backward: c[n-2] = b[n-1] / vt[n-2]; c[i-1] = (b[i] + c[i+1] vt[i]) / vt[i-1]
-    m0 = col ? gm[(size_t)(n - 1) * n + j] : Ar::zero();
-    m1 = (col && n - 3 >= 1) ? gm[(size_t)(n - 3) * n + j] : Ar::zero();
-    m2 = (col && n - 5 >= 1) ? gm[(size_t)(n - 5) * n + j] : Ar::zero();
-    if (col) {
-      const S vtl = Ar::neg(L.sup[n - 2]);
-      const S x = Ar::div_vt(m0, vtl, L.rpos[n - 2]);
-      prev[j] = x;
-      gc[(size_t)(n - 2) * n + j] = x;
-    }
-    __syncthreads();
-    keep_row(n - 2, prev);
-    for (int i = n - 3; i >= 1; i -= 2) {
-      const S mi = m1;
-      m1 = m2;
-      m2 = (col && i - 4 >= 1) ? gm[(size_t)(i - 4) * n + j] : Ar::zero();
-      const S vti = Ar::neg(L.sup[i]), vtm = Ar::neg(L.sup[i - 1]);
-      if (col) {
-        const S x = Ar::div_vt(Ar::add(mi, Ar::mul(prev[j], vti)), vtm, L.rpos[i - 1]);
-        next[j] = x;
-        gc[(size_t)(i - 1) * n + j] = x;
-      }
-      __syncthreads();
-      RR_FRESH();
-      keep_row(i - 1, next);
-      S* t = prev; prev = next; next = t;
-    }
-  }
   __syncthreads();
-  RR_PHASE(5);
-  // product C'(i, j) = C(i, j) + sum_{k < i} M(k, i) C(k, j) (k ascending,
-  // C as solved): right-looking over k with rows k of M and C from the
-  // scratch.  Panel form: the upper part (the lower follows by skew
-  // symmetry).  Full form: every element (the small-matrix path multiplies
-  // the column-permuted C; a column's result depends on that column alone,
-  // so the permutation moves to the output gather).
-  {
-    // rows k of M and C, loaded two steps ahead by thread j < n
+  auto mval = [&](int i, int j) RR_INLINE -> S {  // M(i, j), j < n
+    if (j <= i) return j == i ? Ar::one() : Ar::zero();
+    if (j == n - 1) return Ar::zero();
+    if constexpr (FULL) return L.m[mrow(i) + j];
+    else return gm[(size_t)i * n + j];
+  };
+  RR_PHASE(7);
+  // skew-tridiagonal solve T C = M (vt[i] = -A(i, i+1) = -sup[i]), a thread
+  // per column, its two chains side by side:
+  //   forward   C(1) = M(0) / -vt[0]; C(i+1) = (M(i) - C(i-1) vt[i-1]) / -vt[i], i even
+  //   backward  C(n-2) = M(n-1) / vt[n-2]; C(i-1) = (M(i) + C(i+1) vt[i]) / vt[i-1], i odd descending
+  // The forward chain fills the odd rows of C, the backward one the even
+  // rows.  Full form: through a T-row LDS block into the registers (M is in
+  // LDS).  Panel form: the upper part to gc row-major, M read ahead.
+  if constexpr (FULL) {
+    S* cb = L.vec;
     const int j = tid;
-    const bool col = j < n;
-    S pm0 = col ? gm[j] : Ar::zero(), pc0 = col ? gc[j] : Ar::zero();
-    S pm1 = (col && 1 < n) ? gm[(size_t)n + j] : Ar::zero(), pc1 = (col && 1 < n) ? gc[(size_t)n + j] : Ar::zero();
-    for (int k = 0; k + 2 < n; ++k) {
+    S prev = Ar::zero();
+#pragma unroll 1
+    for (int blk = 0; blk < R; ++blk) {
+      if (j < n) {
+#pragma unroll 4
+        for (int i = T * blk; i < T * blk + T; i += 2)
+          if (i < n) {
+            const S vti = Ar::neg(L.sup[i]);
+            S num = mval(i, j);
+            if (i > 0) num = Ar::sub(num, Ar::mul(prev, Ar::neg(L.sup[i - 1])));
+            prev = Ar::div_negvt(num, vti, Ar::kRecip ? L.rneg[i] : vti);
+            cb[(i + 1 - T * blk) * LDB + j] = prev;
+          }
+      }
+      rr_sync<T>();
       RR_FRESH();
-      S* Mr = (k & 1) ? L.v0 : L.v2;
-      S* Cr = (k & 1) ? L.v1 : L.v3;
-      if (col) {
-        Mr[j] = pm0;
-        Cr[j] = pc0;
+      if (a & 1)
+        rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
+RR_FOR(cj, 0, R) { RC(K, cj) = cb[a * LDB + b + T * cj];
+          };
+        });
+      rr_sync<T>();
+    }
+#pragma unroll 1
+    for (int blk = R - 1; blk >= 0; --blk) {
+      if (j < n) {
+#pragma unroll 4
+        for (int i = T * blk + T - 1; i > T * blk; i -= 2)
+          if (i < n) {
+            const S vtm = Ar::neg(L.sup[i - 1]);
+            S num = mval(i, j);
+            if (i < n - 1) num = Ar::add(num, Ar::mul(prev, Ar::neg(L.sup[i])));
+            prev = Ar::div_vt(num, vtm, Ar::kRecip ? L.rpos[i - 1] : vtm);
+            cb[(i - 1 - T * blk) * LDB + j] = prev;
+          }
       }
-      pm0 = pm1;
-      pc0 = pc1;
-      if (col && k + 2 < n) {
-        pm1 = gm[(size_t)(k + 2) * n + j];
-        pc1 = gc[(size_t)(k + 2) * n + j];
-      }
-      __syncthreads();
+      rr_sync<T>();
+      RR_FRESH();
+      if (!(a & 1))
+        rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
+RR_FOR(cj, 0, R) { RC(K, cj) = cb[a * LDB + b + T * cj];
+          };
+        });
+      rr_sync<T>();
+    }
+  } else {
+#pragma unroll 1
+    for (int u = 0; u < JC; ++u) {
+      const int j = tid + NT * u;
+      if (j < n) {
+        // step s of the chains: forward row 2 s + 1 from M row 2 s,
+        // backward row n - 2 - 2 s from M row n - 1 - 2 s; M of MB steps
+        // loaded together, a batch ahead
+        constexpr int MB = 4;
+        const int steps = n / 2;
+        S mf[MB], mb[MB], pfw = Ar::zero(), pbw = Ar::zero();
+        auto fetch = [&](int s0, S (&vf)[MB], S (&vb)[MB]) RR_INLINE {
 #pragma unroll
-      for (int ri = 0; ri < R; ++ri)
-        if (T * ri + T > k + 1) {
+          for (int t = 0; t < MB; ++t) {
+            vf[t] = s0 + t < steps ? mval(2 * (s0 + t), j) : Ar::zero();
+            vb[t] = s0 + t < steps ? mval(n - 1 - 2 * (s0 + t), j) : Ar::zero();
+          }
+        };
+        fetch(0, mf, mb);
+#pragma unroll 1
+        for (int s0 = 0; s0 < steps; s0 += MB) {
+          S nf[MB], nb[MB];
+          fetch(s0 + MB, nf, nb);
 #pragma unroll
-          for (int cj = FULL ? 0 : ri; cj < R; ++cj) {
-            const int i = a + T * ri, jj = b + T * cj;
-            if (k < i && (FULL || i < jj) && jj < n && i < n) {
-              S& x = c[rr_slot<R, FULL>(ri, cj)];
-              x = Ar::add(x, Ar::mul(Mr[i], Cr[jj]));
+          for (int t = 0; t < MB; ++t) {
+            const int s = s0 + t;
+            if (s < steps) {
+              const int i = 2 * s, k = n - 1 - 2 * s;
+              const S vti = Ar::neg(L.sup[i]), vtm = Ar::neg(L.sup[k - 1]);
+              S nu = mf[t], nv = mb[t];
+              if (s > 0) {
+                nu = Ar::sub(nu, Ar::mul(pfw, Ar::neg(L.sup[i - 1])));
+                nv = Ar::add(nv, Ar::mul(pbw, Ar::neg(L.sup[k])));
+              }
+              pfw = Ar::div_negvt(nu, vti, Ar::kRecip ? L.rneg[i] : vti);
+              pbw = Ar::div_vt(nv, vtm, Ar::kRecip ? L.rpos[k - 1] : vtm);
+              if (i + 1 < j) gc[(size_t)(i + 1) * n + j] = pfw;
+              if (k - 1 < j) gc[(size_t)(k - 1) * n + j] = pbw;
             }
           }
+#pragma unroll
+          for (int t = 0; t < MB; ++t) {
+            mf[t] = nf[t];
+            mb[t] = nb[t];
+          }
         }
+      }
+    }
+    __syncthreads();
+    RR_FRESH();
+RR_FOR(ri, 0, R) {
+RR_FOR(cj, ri, R) {
+        const int i = a + T * ri, j = b + T * cj;
+        RC(ri, cj) = (i < j && j < n) ? gc[(size_t)i * n + j] : Ar::zero();
+      };
+    };
+  }
+  RR_PHASE(8);
+  // product C'(i, j) = C(i, j) + sum_{k < i} M(k, i) C(k, j), k ascending,
+  // C as solved.  Full form, every element (the small-matrix path multiplies
+  // the column-permuted C; a column's result depends on that column alone,
+  // so the permutation moves to the output): row block by row block from the
+  // last, its sums beside the registers' C, the row blocks of C broadcast
+  // through LDS.  Panel form, the upper part (the lower follows by skew
+  // symmetry): k block by k block, T rows of M and C from gs through LDS.
+  if constexpr (FULL) {
+    S* cb = L.vec;
+#pragma unroll 1
+    for (int ib = R - 1; ib >= 0; --ib) {
+      RR_FRESH();
+      S acc[R];
+      rr_case<0, R>(ib, [&]<int K>() RR_INLINE {
+RR_FOR(cj, 0, R) { acc[cj] = RC(K, cj);
+        };
+      });
+      const int i = a + T * ib;
+#pragma unroll 1
+      for (int kb = 0; kb <= ib; ++kb) {
+        rr_case<0, R>(kb, [&]<int K>() RR_INLINE {
+RR_FOR(cj, 0, R) { cb[a * LDB + b + T * cj] = RC(K, cj);
+          };
+        });
+        rr_sync<T>();
+#pragma unroll 4
+        for (int kk = 0; kk < T; ++kk) {
+          const int k = kb * T + kk;
+          if (k < i && i < n) {
+            const S m = mval(k, i);
+RR_FOR(cj, 0, R) { acc[cj] = Ar::add(acc[cj], Ar::mul(m, cb[kk * LDB + b + T * cj]));
+            };
+          }
+        }
+        rr_sync<T>();
+      }
+      rr_case<0, R>(ib, [&]<int K>() RR_INLINE {
+RR_FOR(cj, 0, R) { RC(K, cj) = acc[cj];
+        };
+      });
+    }
+  } else {
+    S* mb = L.vec;
+    S* cb = L.vec + T * LDB;
+#pragma unroll 1
+    for (int kb = 0; kb < R; ++kb) {
+      RR_FRESH();
+      // rows kb T + b of M and C, columns a + T cj
+      const int k = kb * T + b;
+#pragma unroll 1
+      for (int cj = kb; cj < R; ++cj) {
+        const int j = a + T * cj;
+        const bool in = k < j && j < n;
+        mb[b * LDB + j] = in ? mval(k, j) : Ar::zero();
+        cb[b * LDB + j] = in ? gc[(size_t)k * n + j] : Ar::zero();
+      }
+      __syncthreads();
+      rr_case<0, R>(kb, [&]<int K>() RR_INLINE {
+#pragma unroll 1
+        for (int kk = 0; kk < T; ++kk) {
+          S mi[R], cjv[R];
+RR_FOR(r, K, R) {
+            mi[r] = mb[kk * LDB + a + T * r];
+            cjv[r] = cb[kk * LDB + b + T * r];
+          };
+RR_FOR(cj, K, R) {
+RR_FOR(ri, K + 1, cj + 1) { RC(ri, cj) = Ar::add(RC(ri, cj), Ar::mul(mi[ri], cjv[cj]));
+            };
+            if (kk < a) RC(K, cj) = Ar::add(RC(K, cj), Ar::mul(mi[K], cjv[cj]));
+          };
+        }
+      });
+      __syncthreads();
     }
   }
-  __syncthreads();
-  RR_PHASE(6);
-  // permutation of the column swaps (and the same row swaps): position r
-  // holds index perm[r] after the swap sequence of utu2inv
-  if (tid == 0) {
-    for (int r = 0; r < n; ++r) L.perm[r] = r;
-    for (int j = 0; j < n; ++j) {
-      const int t = L.piv[j] - 1;
-      if (t != j) { const int x = L.perm[j]; L.perm[j] = L.perm[t]; L.perm[t] = x; }
-    }
-  }
-  // C' to the scratch (row-major: panel form the upper part, full form
-  // all), then the output gather: out(r, c) = sign * F(perm[r], perm[c]),
-  // F = C' (full form) or the skew completion of C' (panel form, 0 on the
-  // diagonal)
+  RR_PHASE(9);
+  // output: out(r, c) = sign * F(f(r), f(c)), F = C' (full form) or the skew
+  // completion of C' (panel form, 0 on the diagonal).  T columns of F at a
+  // time through LDS, each written as one permuted column of out.
+  {
+    S* ob = L.vec;
+#pragma unroll 1
+    for (int blk = 0; blk < R; ++blk) {
+      RR_FRESH();
+      rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
+        if constexpr (FULL) {
+RR_FOR(ri, 0, R) { ob[b * LDB + a + T * ri] = RC(ri, K);
+          };
+        } else {
+RR_FOR(ri, 0, K) { ob[b * LDB + a + T * ri] = RC(ri, K);
+          };
+          if (a < b) {
+            ob[b * LDB + a + T * K] = RC(K, K);
+            ob[a * LDB + b + T * K] = Ar::neg(RC(K, K));
+          } else if (a == b) {
+            ob[a * LDB + a + T * K] = Ar::zero();
+          }
+RR_FOR(cj, K + 1, R) { ob[a * LDB + b + T * cj] = Ar::neg(RC(K, cj));
+          };
+        }
+      });
+      rr_sync<T>();
+      const int v1 = min(T, n - T * blk);
+#pragma unroll 1
+      for (int v = 0; v < v1; ++v) {
+        const size_t col = (size_t)L.finv[T * blk + v] * n;
 #pragma unroll
-  for (int ri = 0; ri < R; ++ri)
-#pragma unroll
-    for (int cj = FULL ? 0 : ri; cj < R; ++cj) {
-      const int i = a + T * ri, j = b + T * cj;
-      if ((FULL || i < j) && i < n && j < n) gc[(size_t)i * n + j] = c[rr_slot<R, FULL>(ri, cj)];
+        for (int u = 0; u < JC; ++u) {
+          const int r = tid + NT * u;
+          if (r < n) {
+            S x = ob[v * LDB + f[u]];
+            if (sign != 1.0) x = Ar::neg(x);
+            out[col + r] = x;
+            if constexpr (sizeof(S) == sizeof(double))
+              if (out32) out32[col + r] = (float)x;
+          }
+        }
+      }
+      rr_sync<T>();
     }
-  __syncthreads();
-  for (int e = tid; e < n * n; e += NT) {
-    const int r = e % n, cc = e / n;
-    const int u = L.perm[r], v = L.perm[cc];
-    S x = Ar::zero();
-    if (FULL) x = gc[(size_t)u * n + v];
-    else if (u < v) x = gc[(size_t)u * n + v];
-    else if (u > v) x = Ar::neg(gc[(size_t)v * n + u]);
-    out[e] = sign != 1.0 ? Ar::neg(x) : x;
   }
   __syncthreads();
-  RR_PHASE(7);
+  RR_PHASE(10);
 #ifdef MVMC_PHASE_CLOCKS
   if (tid == 0 && blockIdx.x == 0)
-    printf("rr n=%d phases(10ns): gather %lld ltl %lld pf %lld trtri %lld mwrite %lld solve %lld product %lld out %lld"
-           " | ltl: pivot %lld swapstage %lld wb+stage %lld update %lld\n",
-           n, rr_ph[0], rr_ph[1], rr_ph[2], rr_ph[3], rr_ph[4], rr_ph[5], rr_ph[6], rr_ph[7], rr_sub[0], rr_sub[1],
-           rr_sub[2], rr_sub[3]);
+    printf("rr n=%d cycles: gather %lld ltl stage %lld pivot %lld swap %lld update %lld pf %lld trtri %lld mwrite %lld "
+           "solve %lld product %lld out %lld\n",
+           n, rr_ph[0], rr_ph[1], rr_ph[2], rr_ph[3], rr_ph[4], rr_ph[5], rr_ph[6], rr_ph[7], rr_ph[8], rr_ph[9],
+           rr_ph[10]);
 #endif
 #undef RR_PHASE
-#undef RR_SUB
+#undef RC
 #undef RR_FRESH
 }
 
