@@ -27,6 +27,7 @@
 #include "pfinv_c128_dev.h"
 #include "pfinv_lds.h"
 #include "rr_planes.h"
+#include "sr_cg.h"
 #include "sr_stages.h"
 
 using namespace mvmc_hip;
@@ -82,7 +83,8 @@ void require_gpu() {
 struct CgWork {
   double *x = nullptr, *r = nullptr, *d = nullptr, *q = nullptr, *g = nullptr;
   double *cpart = nullptr, *spart = nullptr;  // chunk / superchunk partials of S x
-  double* sc = nullptr;  // scalars: 0 delta, 2 alpha, 4 beta, 5 coef
+  double* prod = nullptr;  // products of a dot (na > CGT_NMAX)
+  double* sc = nullptr;  // scalars: 0 delta, 5 coef
   int* ctl = nullptr;    // 0 done, 1..2 status (int64)
   int cap_n = 0, cap_rows = 0;
   void ensure(int na, int rows) {
@@ -99,14 +101,15 @@ struct CgWork {
     HIPCHK(hipMalloc(&g, sizeof(double) * cap_n));
     HIPCHK(hipMalloc(&cpart, sizeof(double) * cap_n * nch));
     HIPCHK(hipMalloc(&spart, sizeof(double) * cap_n * nsup));
+    HIPCHK(hipMalloc(&prod, sizeof(double) * cap_n));
     HIPCHK(hipMalloc(&sc, sizeof(double) * 8));
     HIPCHK(hipMalloc(&ctl, sizeof(int) * 4));
   }
   void release() {
-    for (void* p : {(void*)x, (void*)r, (void*)d, (void*)q, (void*)g, (void*)cpart, (void*)spart, (void*)sc,
-                    (void*)ctl})
+    for (void* p : {(void*)x, (void*)r, (void*)d, (void*)q, (void*)g, (void*)cpart, (void*)spart, (void*)prod,
+                    (void*)sc, (void*)ctl})
       if (p) (void)hipFree(p);
-    x = r = d = q = g = cpart = spart = sc = nullptr;
+    x = r = d = q = g = cpart = spart = prod = sc = nullptr;
     ctl = nullptr;
     cap_n = cap_rows = 0;
   }
@@ -127,138 +130,6 @@ namespace {
 
 inline int nblk(long long n, int b = 256) { return (int)((n + b - 1) / b); }
 
-// out = S x (or g - S x when g is given) with the sampled operator
-// (sr_cg.rs:952-1004) in the blocked reduction order.
-template <class P>
-void cg_apply_dev(int na, int rows, const P* pack, const double* mean, const double* diag, const double* xv,
-                  const double* g, double* out, double inv_w, double shift, CgWork& wk, hipStream_t st) {
-  const int nch = (rows + CG_RCH - 1) / CG_RCH;
-  const int nsup = (nch + CG_SCH - 1) / CG_SCH;
-  const int cols = (na + 255) / 256;
-  const dim3 grid(nch + 1), blk(256);
-  double* coef = wk.sc + 5;
-  if (cols <= 4)
-    hipLaunchKernelGGL((k_cg_chunk<4, P>), grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
-  else if (cols <= 8)
-    hipLaunchKernelGGL((k_cg_chunk<8, P>), grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
-  else if (cols <= 16)
-    hipLaunchKernelGGL((k_cg_chunk<16, P>), grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
-  else if (cols <= CG_CMAX)
-    hipLaunchKernelGGL((k_cg_chunk<CG_CMAX, P>), grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef,
-                       wk.ctl);
-  else
-    hipLaunchKernelGGL(k_cg_chunk_wide<P>, grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
-  if (nsup > 0)
-    hipLaunchKernelGGL(k_cg_fold1, dim3(nblk(na), nsup), blk, 0, st, wk.cpart, nch, na, wk.spart, wk.ctl);
-  hipLaunchKernelGGL(k_cg_fold2, dim3(nblk(na)), blk, 0, st, wk.spart, nsup, na, xv, mean, diag, coef, inv_w, shift,
-                     g, out, wk.ctl);
-}
-
-// The same product from the explicit Gram G = O^T O (FP32, full symmetric
-// na x na; the precision form).
-void cg_apply_gram(int na, const float* G, const double* mean, const double* diag, const double* xv,
-                   const double* g, double* out, double inv_w, double shift, CgWork& wk, hipStream_t st) {
-  double* coef = wk.sc + 5;
-  hipLaunchKernelGGL(k_gram_coef, dim3(1), dim3(256), 0, st, mean, xv, na, coef, wk.ctl);
-  hipLaunchKernelGGL(k_gram_apply, dim3((na + 3) / 4), dim3(256), 0, st, G, na, xv, mean, diag, coef, inv_w, shift,
-                     g, out, wk.ctl);
-}
-
-// C 1.4.0 StochasticOptCG_Main / PreconCG_DiagScale (sr_cg.rs:700-880).
-// Iterations run on the device as a HIP graph of one residual-refresh period
-// (CG_PERIOD iterations, the refresh S x at its last one), captured once per
-// solve and replayed: the kernels read the period's first iteration from
-// ctl[CTL_ITER] (k_cg_advance moves it on), and a done flag set by the head /
-// guard kernels turns the rest into no-ops.  The host reads the flag once per
-// period.  The graph holds kernel nodes only.
-constexpr int CG_PERIOD = 20;
-
-template <class P>
-long long cg_solve_dev(int na, int W, int NS, const P* pack, const double* mean, const double* diag,
-                       const double* g, double inv_w, double shift, double tol, int max_it, bool diag_scale,
-                       double* x_out, CgWork& wk, hipStream_t st_in, const float* gram = nullptr) {
-  const int rows = W * NS;
-  wk.ensure(na, rows);
-  // graph capture needs a created stream: the null stream's work is ordered
-  // with a default-flag stream by the runtime
-  hipStream_t own = nullptr;
-  if (!st_in) HIPCHK(hipStreamCreate(&own));
-  hipStream_t st = st_in ? st_in : own;
-  const double threshold = tol * tol * (double)na * (double)na;
-  const double pfac = 1.0 + shift;
-  const dim3 blk(256);
-  // S x: one pass over the packed samples, or (gram set) one over their Gram
-  auto apply = [&](const double* xv, const double* gv, double* out) {
-    if (gram) cg_apply_gram(na, gram, mean, diag, xv, gv, out, inv_w, shift, wk, st);
-    else cg_apply_dev(na, rows, pack, mean, diag, xv, gv, out, inv_w, shift, wk, st);
-  };
-  HIPCHK(hipMemsetAsync(wk.ctl, 0, sizeof(int) * 4, st));
-  HIPCHK(hipMemcpyAsync(wk.g, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-  hipLaunchKernelGGL(k_fill, dim3(nblk(na)), blk, 0, st, wk.x, na, 0.0);
-  HIPCHK(hipMemcpyAsync(wk.r, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-  if (diag_scale)
-    apply(wk.x, wk.g, wk.r);
-  else
-    HIPCHK(hipMemcpyAsync(wk.d, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-  hipLaunchKernelGGL(k_cg_init, dim3(1), blk, 0, st, na, wk.r, wk.d, diag, pfac, diag_scale ? 1 : 0, wk.sc, wk.ctl);
-  HIPCHK(hipGetLastError());
-  // one refresh period of iterations (kernel launches only)
-  auto issue_period = [&]() {
-    for (int j = 0; j < CG_PERIOD; ++j) {
-      hipLaunchKernelGGL(k_cg_head, dim3(1), dim3(64), 0, st, j, max_it, threshold, wk.sc, wk.ctl);
-      apply(wk.d, nullptr, wk.q);
-      hipLaunchKernelGGL(k_cg_alpha, dim3(1), blk, 0, st, j, na, wk.d, wk.q, wk.sc, wk.ctl);
-      const int refresh = (j == CG_PERIOD - 1);  // (iter + 1) % 20 == 0 with periods starting at multiples of 20
-      hipLaunchKernelGGL(k_cg_update, dim3(nblk(na)), blk, 0, st, na, wk.sc, wk.ctl, wk.d, wk.x, wk.q, wk.r,
-                         refresh);
-      if (refresh) apply(wk.x, wk.g, wk.r);
-      hipLaunchKernelGGL(k_cg_beta, dim3(1), blk, 0, st, j, na, wk.r, wk.q, diag, pfac, diag_scale ? 1 : 0, wk.sc,
-                         wk.ctl);
-      hipLaunchKernelGGL(k_cg_dir, dim3(nblk(na)), blk, 0, st, na, wk.sc, wk.ctl, diag_scale ? wk.q : wk.r, wk.d);
-    }
-    hipLaunchKernelGGL(k_cg_advance, dim3(1), dim3(64), 0, st, wk.ctl, CG_PERIOD);
-  };
-  // MVMC_CG_GRAPH=0 issues the same launches without a graph (for tools that
-  // do not follow graph launches)
-  static const bool use_graph = [] {
-    const char* e = std::getenv("MVMC_CG_GRAPH");
-    return !(e && e[0] == '0');
-  }();
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
-  if (use_graph) {
-    HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    issue_period();
-    HIPCHK(hipStreamEndCapture(st, &graph));
-    HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-  }
-  long long status = 0;
-  bool done = false;
-  for (int it0 = 0; it0 <= max_it; it0 += CG_PERIOD) {
-    if (use_graph) HIPCHK(hipGraphLaunch(exec, st));
-    else issue_period();
-    HIPCHK(hipGetLastError());
-    int ctl[4];
-    HIPCHK(hipMemcpyAsync(ctl, wk.ctl, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    if (ctl[0]) {
-      status = (long long)(((unsigned long long)(unsigned)ctl[2] << 32) | (unsigned)ctl[1]);
-      done = true;
-      break;
-    }
-  }
-  if (exec) (void)hipGraphExecDestroy(exec);
-  if (graph) (void)hipGraphDestroy(graph);
-  if (!done) {
-    if (own) (void)hipStreamDestroy(own);
-    throw Fail(MVMC_E_BACKEND, "SR-CG control flag not set at the iteration limit");
-  }
-  HIPCHK(hipMemcpyAsync(x_out, wk.x, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-  HIPCHK(hipStreamSynchronize(st));
-  if (own) HIPCHK(hipStreamDestroy(own));
-  return status;
-}
-
 // A kernel's dynamic-LDS limit is a process-wide attribute while every
 // ensemble (and batched call) needs its own size: the limit only grows, so
 // handles of different models can live and run side by side.
@@ -270,6 +141,143 @@ void raise_lds_limit(const void* fn, size_t bytes) {
   if (bytes <= c) return;
   HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
   c = bytes;
+}
+
+// Superchunk partials of the sampled operator's product with xv (wk.spart,
+// the return value their number) and coef = mean . xv, in the blocked
+// reduction order (sr_cg.rs:952-1004).
+template <class P>
+int cg_product(int na, int rows, const P* pack, const double* mean, const double* xv, CgWork& wk, hipStream_t st) {
+  const int nch = (rows + CG_RCH - 1) / CG_RCH;
+  const int nsup = (nch + CG_SCH - 1) / CG_SCH;
+  const int cols = (na + 255) / 256;
+  const dim3 grid(nch + 1), blk(256);
+  double* coef = wk.sc + 5;
+  auto chunk = [&]<int C>() {
+    hipLaunchKernelGGL((k_cg_chunk<C, P>), grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
+  };
+  if (cols <= 2) chunk.template operator()<2>();
+  else if (cols <= 4) chunk.template operator()<4>();
+  else if (cols <= 6) chunk.template operator()<6>();
+  else if (cols <= 9) chunk.template operator()<9>();
+  else if (cols <= 12) chunk.template operator()<12>();
+  else if (cols <= 16) chunk.template operator()<16>();
+  else if (cols <= 24) chunk.template operator()<24>();
+  else if (cols <= CG_CMAX) chunk.template operator()<CG_CMAX>();
+  else
+    hipLaunchKernelGGL(k_cg_chunk_wide<P>, grid, blk, 0, st, pack, rows, na, xv, mean, wk.cpart, coef, wk.ctl);
+  if (nsup > 0)
+    hipLaunchKernelGGL(k_cg_fold1, dim3(nblk(na), nsup), blk, 0, st, wk.cpart, nch, na, wk.spart, wk.ctl);
+  return nsup;
+}
+
+// out = S x (or g - S x when g is given).
+template <class P>
+void cg_apply_dev(int na, int rows, const P* pack, const double* mean, const double* diag, const double* xv,
+                  const double* g, double* out, double inv_w, double shift, CgWork& wk, hipStream_t st) {
+  const int nsup = cg_product(na, rows, pack, mean, xv, wk, st);
+  hipLaunchKernelGGL(k_cg_fold2, dim3(nblk(na)), dim3(256), 0, st, wk.spart, nsup, na, xv, mean, diag, wk.sc + 5,
+                     inv_w, shift, g, out, wk.ctl);
+}
+
+// k_cg_small of M = ceil(na / 64) columns per lane (rounded up to an
+// instance).
+template <bool GRAM, class P>
+void cg_small(const P* op, int rows, int na, const double* mean, const double* diag, const double* g, double inv_w,
+              double shift, double threshold, double pfac, int max_it, int diag_scale, double* x, int* ctl,
+              hipStream_t st) {
+  const size_t lds = cgs_lds_doubles(na, rows, GRAM) * sizeof(double);
+  auto go = [&]<int M>() {
+    raise_lds_limit((const void*)k_cg_small<M, GRAM, P>, lds);
+    hipLaunchKernelGGL((k_cg_small<M, GRAM, P>), dim3(1), dim3(CGS_NT), lds, st, op, rows, na, mean, diag, g, inv_w,
+                       shift, threshold, pfac, max_it, diag_scale, x, ctl);
+  };
+  const int m = (na + 63) / 64;
+  if (m <= 1) go.template operator()<1>();
+  else if (m <= 2) go.template operator()<2>();
+  else if (m <= 3) go.template operator()<3>();
+  else if (m <= 5) go.template operator()<5>();
+  else if (m <= 7) go.template operator()<7>();
+  else go.template operator()<CGS_M>();
+  HIPCHK(hipGetLastError());
+}
+
+// C 1.4.0 StochasticOptCG_Main / PreconCG_DiagScale (sr_cg.rs:700-880).
+// Operators that one CU streams fast enough (CGS_ELEMS) are solved by one
+// launch.  Otherwise an iteration is its product (chunk partials and their
+// first fold, or the Gram's rows) and k_cg_tail, issued a residual-refresh
+// period at a time; a done flag set by the guards turns the rest into
+// no-ops, and the host reads it once per period.
+constexpr int CG_PERIOD = 20;
+
+template <class P>
+long long cg_solve_dev(int na, int W, int NS, const P* pack, const double* mean, const double* diag,
+                       const double* g, double inv_w, double shift, double tol, int max_it, bool diag_scale,
+                       double* x_out, CgWork& wk, hipStream_t st, const float* gram = nullptr) {
+  const int rows = W * NS;
+  wk.ensure(na, rows);
+  const double threshold = tol * tol * (double)na * (double)na;
+  const double pfac = 1.0 + shift;
+  const dim3 blk(256);
+  auto read_ctl = [&](int (&ctl)[4]) {
+    HIPCHK(hipMemcpyAsync(ctl, wk.ctl, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return (long long)(((unsigned long long)(unsigned)ctl[2] << 32) | (unsigned)ctl[1]);
+  };
+  int ctl[4];
+  const long long elems = (long long)na * (gram ? na : rows);
+  if (na <= 64 * CGS_M && rows > 0 && elems <= CGS_ELEMS) {
+    if (gram)
+      cg_small<true>(gram, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
+                     wk.ctl, st);
+    else
+      cg_small<false>(pack, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
+                      wk.ctl, st);
+    HIPCHK(hipMemcpyAsync(x_out, wk.x, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+    return read_ctl(ctl);
+  }
+  auto product = [&](const double* xv) {
+    if (!gram) return cg_product(na, rows, pack, mean, xv, wk, st);
+    hipLaunchKernelGGL(k_gram_product, dim3((na + 3) / 4 + 1), blk, 0, st, gram, na, xv, mean, wk.spart, wk.sc + 5,
+                       wk.ctl);
+    return 1;
+  };
+  HIPCHK(hipMemsetAsync(wk.ctl, 0, sizeof(int) * 4, st));
+  HIPCHK(hipMemcpyAsync(wk.g, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+  hipLaunchKernelGGL(k_fill, dim3(nblk(na)), blk, 0, st, wk.x, na, 0.0);
+  HIPCHK(hipMemcpyAsync(wk.r, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+  if (diag_scale) {
+    const int nsup = product(wk.x);
+    hipLaunchKernelGGL(k_cg_fold2, dim3(nblk(na)), blk, 0, st, wk.spart, nsup, na, wk.x, mean, diag, wk.sc + 5, inv_w,
+                       shift, wk.g, wk.r, wk.ctl);
+  } else {
+    HIPCHK(hipMemcpyAsync(wk.d, g, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+  }
+  hipLaunchKernelGGL(k_cg_init, dim3(1), blk, 0, st, na, wk.r, wk.d, diag, pfac, diag_scale ? 1 : 0, max_it,
+                     threshold, wk.sc, wk.ctl);
+  HIPCHK(hipGetLastError());
+  const size_t lds = na <= CGT_NMAX ? sizeof(double) * na : 0;
+  raise_lds_limit((const void*)k_cg_tail, sizeof(double) * CGT_NMAX);
+  auto tail = [&](int stage, int j, int nsup) {
+    hipLaunchKernelGGL(k_cg_tail, dim3(1), dim3(CGT_NT), lds, st, stage, j, na, nsup, wk.spart, mean, diag, wk.g,
+                       wk.sc + 5, inv_w, shift, pfac, diag_scale ? 1 : 0, max_it, threshold, wk.x, wk.r, wk.d, wk.q,
+                       wk.prod, wk.sc, CG_PERIOD, wk.ctl);
+  };
+  for (int it0 = 0; it0 <= max_it; it0 += CG_PERIOD) {
+    for (int j = 0; j < CG_PERIOD; ++j) {
+      const bool refresh = j == CG_PERIOD - 1;  // (iter + 1) % 20 == 0 with periods starting at multiples of 20
+      tail(refresh ? 1 : 0, j, product(wk.d));
+      if (refresh) tail(2, j, product(wk.x));
+    }
+    HIPCHK(hipGetLastError());
+    const long long status = read_ctl(ctl);
+    if (ctl[0]) {
+      HIPCHK(hipMemcpyAsync(x_out, wk.x, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+      HIPCHK(hipStreamSynchronize(st));
+      return status;
+    }
+  }
+  throw Fail(MVMC_E_BACKEND, "SR-CG control flag not set at the iteration limit");
 }
 
 // Work array of mvmc_pfinv_f64_noalloc, in the code object (no allocation

@@ -1996,7 +1996,7 @@ __global__ void k_cg_pack(EnsView v, const int* map, int na, P* pack) {
 }
 
 // ctl: 0 done, 1..2 status (int64), 3 first iteration of the current period
-// of the replayed CG graph (kernels get their offset in the period)
+// of residual refreshes (kernels get their offset in the period)
 enum { CTL_DONE = 0, CTL_STATUS_LO = 1, CTL_STATUS_HI = 2, CTL_ITER = 3 };
 
 __device__ inline void cg_finish(int* ctl, long long status) {
@@ -2056,15 +2056,42 @@ struct RowBuf<float> {
   }
 };
 
+// Two values' pairwise trees over the 256 lane partials at once (the order
+// of block_tree256 for each).
+__device__ inline void block_tree256x2(double& p0, double& p1, double* red) {
+  const int tid = threadIdx.x;
+  red[tid] = p0;
+  red[256 + tid] = p1;
+  __syncthreads();
+  if (tid < 64) {
+    double v0 = (red[tid] + red[tid + 128]) + (red[tid + 64] + red[tid + 192]);
+    double v1 = (red[256 + tid] + red[tid + 384]) + (red[tid + 320] + red[tid + 448]);
+    for (int h = 32; h >= 1; h >>= 1) {
+      v0 += __shfl_down(v0, h, 64);
+      v1 += __shfl_down(v1, h, 64);
+    }
+    if (tid == 0) {
+      red[512] = v0;
+      red[513] = v1;
+    }
+  }
+  __syncthreads();
+  p0 = red[512];
+  p1 = red[513];
+}
+
 // Chunk partials cpart[b][i] = sum_{r in chunk b} O_ri y_r with y_r formed
 // from the same registers; block nch computes coef = bdot(mean, x).
 // C = columns per lane (na <= 256*C).  P: element type of the packed samples
-// (double; float in the precision form, accumulated in FP64).
+// (double; float in the precision form, accumulated in FP64).  Bound by HBM
+// (the samples once per product), if the rows' dot chain does not hold the
+// loads up: two rows share a tree, and the next two rows' loads are in
+// flight meanwhile (8192 rows x 2099: 36 -> 27 us).
 template <int C, class P>
-__global__ void __launch_bounds__(256, 2) k_cg_chunk(const P* pack, int rows, int na, const double* x,
+__global__ void __launch_bounds__(256, C <= 16 ? 2 : 1) k_cg_chunk(const P* pack, int rows, int na, const double* x,
                                                   const double* mean, double* cpart, double* coef, const int* ctl) {
   if (ctl[CTL_DONE]) return;
-  __shared__ double red[256];
+  __shared__ double red[514];
   const int tid = threadIdx.x;
   const int nch = (rows + CG_RCH - 1) / CG_RCH;
   const int b = blockIdx.x;
@@ -2073,6 +2100,19 @@ __global__ void __launch_bounds__(256, 2) k_cg_chunk(const P* pack, int rows, in
     if (tid == 0) *coef = c;
     return;
   }
+  const int r0 = b * CG_RCH, r1 = min(rows, r0 + CG_RCH);
+  // one buffer resource per row: element i >= na reads 0 in hardware, so the
+  // loads carry no branch and are all in flight before the first use
+  P raw[2][C];
+  auto load = [&](int r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const RowBuf<P> row(pack + (size_t)min(r + u, r1 - 1) * na, na);
+#pragma unroll
+      for (int k = 0; k < C; ++k) raw[u][k] = row.load(tid + 256 * k);
+    }
+  };
+  load(r0);
   double xv[C], acc[C];
 #pragma unroll
   for (int k = 0; k < C; ++k) {
@@ -2080,25 +2120,26 @@ __global__ void __launch_bounds__(256, 2) k_cg_chunk(const P* pack, int rows, in
     xv[k] = i < na ? x[i] : 0.0;
     acc[k] = 0.0;
   }
-  const int r1 = min(rows, (b + 1) * CG_RCH);
-  for (int r = b * CG_RCH; r < r1; ++r) {
-    // one buffer resource per row: element i >= na reads 0 in hardware, so
-    // the C loads carry no branch and are all in flight before the first use
-    const RowBuf<P> row(pack + (size_t)r * na, na);
-    P raw[C];
+  for (int r = r0; r < r1; r += 2) {
+    double o[2][C];
 #pragma unroll
-    for (int k = 0; k < C; ++k) raw[k] = row.load(tid + 256 * k);
-    double o[C];
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int k = 0; k < C; ++k) o[k] = (double)raw[k];
-    double p = 0.0;
+      for (int k = 0; k < C; ++k) o[u][k] = (double)raw[u][k];
+    load(min(r + 2, r1 - 1));
+    double p[2] = {0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < C; ++k)
-      if (tid + 256 * k < na) p += o[k] * xv[k];
-    const double y = block_tree256(p, red);
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int k = 0; k < C; ++k)
+        if (tid + 256 * k < na) p[u] += o[u][k] * xv[k];
+    block_tree256x2(p[0], p[1], red);
 #pragma unroll
     for (int k = 0; k < C; ++k)
-      if (tid + 256 * k < na) acc[k] += o[k] * y;
+      if (tid + 256 * k < na) {
+        acc[k] += o[0][k] * p[0];
+        if (r + 1 < r1) acc[k] += o[1][k] * p[1];
+      }
   }
 #pragma unroll
   for (int k = 0; k < C; ++k) {
@@ -2167,11 +2208,18 @@ __device__ inline double cg_precond(double pfac, double dg, double r) {
   return r / dq;
 }
 
-// sc: 0 delta, 2 alpha, 4 beta, 5 coef.  ctl: done flag + 64-bit status.
-// Start of the initial residual: diag-scale d = precond(r), delta = r.d;
+// Head of iteration `iter` (the loop condition of the C solver).
+__device__ inline void cg_head(int iter, int max_it, double threshold, double delta, int* ctl) {
+  if (iter >= max_it) cg_finish(ctl, fabs(delta) >= threshold ? -(long long)(max_it + 1) : (long long)iter);
+  else if (!(delta - delta == 0.0)) cg_finish(ctl, -(long long)(iter + 1));
+  else if (fabs(delta) < threshold) cg_finish(ctl, iter);
+}
+
+// sc: 0 delta, 5 coef.  ctl: done flag + 64-bit status.
+// Start from the initial residual: diag-scale d = precond(r), delta = r.d;
 // plain: delta = r.r.  Non-finite delta ends the solve with status -1.
 __global__ void __launch_bounds__(256) k_cg_init(int na, const double* r, double* d, const double* diag, double pfac,
-                                                 int diag_scale, double* sc, int* ctl) {
+                                                 int diag_scale, int max_it, double threshold, double* sc, int* ctl) {
   __shared__ double red[256];
   double p = 0.0;
   for (int i = threadIdx.x; i < na; i += 256) {
@@ -2188,87 +2236,8 @@ __global__ void __launch_bounds__(256) k_cg_init(int na, const double* r, double
     sc[0] = delta;
     ctl[CTL_DONE] = 0;
     if (!(delta - delta == 0.0)) cg_finish(ctl, -1);
+    else cg_head(0, max_it, threshold, delta, ctl);
   }
-}
-
-// Head of iteration `iter` (the loop condition of the C solver).
-__global__ void k_cg_head(int j, int max_it, double threshold, const double* sc, int* ctl) {
-  if (threadIdx.x || blockIdx.x || ctl[CTL_DONE]) return;
-  const int iter = ctl[CTL_ITER] + j;
-  const double delta = sc[0];
-  if (iter >= max_it) {
-    cg_finish(ctl, fabs(delta) >= threshold ? -(long long)(max_it + 1) : (long long)iter);
-    return;
-  }
-  if (!(delta - delta == 0.0)) cg_finish(ctl, -(long long)(iter + 1));
-  else if (fabs(delta) < threshold) cg_finish(ctl, iter);
-}
-
-// alpha = delta / (d.q) with the C guards
-__global__ void __launch_bounds__(256) k_cg_alpha(int j, int na, const double* d, const double* q, double* sc,
-                                                  int* ctl) {
-  if (ctl[CTL_DONE]) return;
-  const int iter = ctl[CTL_ITER] + j;
-  __shared__ double red[256];
-  const double dq = block_bdot(d, q, na, red);
-  if (threadIdx.x == 0) {
-    if (!(dq - dq == 0.0) || fabs(dq) < 1.0e-20) { cg_finish(ctl, -(long long)(iter + 1)); return; }
-    const double a = sc[0] / dq;
-    if (!(a - a == 0.0)) { cg_finish(ctl, -(long long)(iter + 1)); return; }
-    sc[2] = a;
-  }
-}
-
-// x += alpha d; r -= alpha q (not on refresh iterations)
-__global__ void k_cg_update(int na, const double* sc, const int* ctl, const double* d, double* x, const double* q,
-                            double* r, int refresh) {
-  if (ctl[CTL_DONE]) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= na) return;
-  const double a = sc[2];
-  x[i] += a * d[i];
-  if (!refresh) r[i] -= a * q[i];
-}
-
-// dnew (diag-scale: q = precond(r), dnew = r.q; plain: r.r), beta, delta
-__global__ void __launch_bounds__(256) k_cg_beta(int j, int na, const double* r, double* q, const double* diag,
-                                                 double pfac, int diag_scale, double* sc, int* ctl) {
-  if (ctl[CTL_DONE]) return;
-  const int iter = ctl[CTL_ITER] + j;
-  __shared__ double red[256];
-  double p = 0.0;
-  for (int i = threadIdx.x; i < na; i += 256) {
-    if (diag_scale) {
-      const double qq = cg_precond(pfac, diag[i], r[i]);
-      q[i] = qq;
-      p += r[i] * qq;
-    } else {
-      p += r[i] * r[i];
-    }
-  }
-  const double dn = block_tree256(p, red);
-  if (threadIdx.x == 0) {
-    const double dl = sc[0];
-    if (!(dn - dn == 0.0) || fabs(dl) < 1.0e-20) { cg_finish(ctl, -(long long)(iter + 1)); return; }
-    const double b = dn / dl;
-    if (!(b - b == 0.0)) { cg_finish(ctl, -(long long)(iter + 1)); return; }
-    sc[4] = b;
-    sc[0] = diag_scale ? dn : dl * b;
-  }
-}
-
-// d = src + beta d
-// End of a replayed period of the CG graph: the next period starts `period`
-// iterations later.
-__global__ void k_cg_advance(int* ctl, int period) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && !ctl[CTL_DONE]) ctl[CTL_ITER] += period;
-}
-
-__global__ void k_cg_dir(int na, const double* sc, const int* ctl, const double* src, double* d) {
-  if (ctl[CTL_DONE]) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= na) return;
-  d[i] = src[i] + sc[4] * d[i];
 }
 
 // ---------------------------------------------------------------------------
