@@ -433,6 +433,7 @@ struct mvmc_ens {
   double rebuild_ms = 0, rebuild_launches = 0;
   size_t lds_samp = 0, lds_meas = 0;
   double* d_slater = nullptr;
+  double* d_orb = nullptr;   // orbital parameters
   double* d_proj = nullptr;
   double* d_dg = nullptr;
   double* d_dj = nullptr;
@@ -463,6 +464,9 @@ struct mvmc_ens {
   // FP32 (inv32), everything else FP64
   int precision = 0;
   float* inv32 = nullptr;
+  // caller-supplied configurations: EleIdx of a layer, and its packed rows
+  int* d_cfg = nullptr;
+  char* d_cfg_out = nullptr;
   double* d_rows = nullptr;  // [W*nsample] cotangents / log|psi| of the saved samples
   // direct SR (NSRCG 0): rocBLAS handle on the library's stream, S [na][na], Cholesky info
   rocblas_handle blas = nullptr;
@@ -494,14 +498,15 @@ struct mvmc_ens {
     if (st) (void)hipStreamDestroy(st);
   }
   void upload_tables() {
-    std::vector<double> S, g, j;
-    mvmc::build_slater_table(m, S);
-    mvmc::direct_projection_tables(m, g, j);
-    HIPCHK(hipMemcpyAsync(d_slater, S.data(), sizeof(double) * S.size(), hipMemcpyHostToDevice, st));
+    if (!m.slater.empty())
+      HIPCHK(hipMemcpyAsync(d_orb, m.slater.data(), sizeof(double) * m.slater.size(), hipMemcpyHostToDevice, st));
     if (!m.proj.empty())
       HIPCHK(hipMemcpyAsync(d_proj, m.proj.data(), sizeof(double) * m.proj.size(), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(d_dg, g.data(), sizeof(double) * g.size(), hipMemcpyHostToDevice, st));
-    HIPCHK(hipMemcpyAsync(d_dj, j.data(), sizeof(double) * j.size(), hipMemcpyHostToDevice, st));
+    const long long sites = (long long)v.ns * v.ns;
+    hipLaunchKernelGGL(k_slater_table, dim3((unsigned)((v.nqp * sites + 255) / 256)), dim3(256), 0, st, v, d_orb,
+                       d_slater);
+    hipLaunchKernelGGL(k_proj_tables, dim3((unsigned)((sites + 255) / 256)), dim3(256), 0, st, v, d_dg, d_dj);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
   }
   // Device-to-host copy ordered on the handle's own (non-blocking) stream:
@@ -591,6 +596,7 @@ void create_impl(mvmc_ens* E, const char* namelist, const char* initial_def, int
   v.exp_cr = 1;
   // model tables
   E->d_slater = dalloc<double>(A, (size_t)v.nqp * v.n2 * v.n2);
+  E->d_orb = dalloc<double>(A, m.slater.size());
   v.slater = E->d_slater;
   v.qpw = dupload(A, m.qp_full_weight, E->st);
   E->d_proj = dalloc<double>(A, std::max(v.nproj, 1));
@@ -985,19 +991,31 @@ void measure_finish(mvmc_ens* E) {
 // measure_sample batched over samples (crates/mvmc-core/src/stage_backend.rs:
 // 418-438; per sample the work of run.rs:2937-3616).  Configuration c goes to
 // the saved-sample slot of walker c mod W in layer c / W; every layer is
-// rebuilt (k_meas_rebuild) and measured (k_measure) by the kernels of
-// mvmc_ens_measure with the current parameters.  EleCfg / EleNum and the
-// projection counts are derived here (projection.rs:179-277).  The saved
-// samples and the walkers' inverse tables are overwritten.
+// rebuilt and measured (k_measure) by the kernels of mvmc_ens_measure with
+// the current parameters.  Only EleIdx goes up and whole rows come down, one
+// copy each: EleCfg / EleNum and the projection counts are derived on the
+// device (k_config_slots).  The saved samples and the walkers' inverse
+// tables are overwritten.
 void measure_configs_impl(mvmc_ens* E, int count, const int* ele_idx, double* e_loc, double* o, int* valid) {
   EnsView& v = E->v;
   if (count < 0 || (long long)count > (long long)v.W * v.nsample)
     throw Fail(MVMC_E_INVALID_SHAPE, "count must be between 0 and walkers x NVMCSample");
   if (count == 0) return;
   if (!ele_idx || !e_loc) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
-  const mvmc::Model& m = E->m;
-  const int n = v.n, ne = v.ne, ns = v.ns, n2 = v.n2, np = v.nproj, size = v.size, nsamp = v.nsample;
-  const int npc = np > 0 ? np : 1;
+  const int n = v.n, ne = v.ne, ns = v.ns, size = v.size, nsamp = v.nsample;
+  {
+    std::vector<int> seen(v.n2, -1);
+    for (int c = 0; c < count; ++c)
+      for (int mi = 0; mi < n; ++mi) {
+        const int ri = ele_idx[(size_t)c * n + mi];
+        if (ri < 0 || ri >= ns)
+          throw Fail(MVMC_E_INPUT, "configuration " + std::to_string(c) + ": site index out of range");
+        int& at = seen[ri + (mi / ne) * ns];
+        if (at == c)
+          throw Fail(MVMC_E_INPUT, "configuration " + std::to_string(c) + ": two electrons of one spin on a site");
+        at = c;
+      }
+  }
   E->upload_tables();
   const int W0 = v.W;
   struct RestoreW {
@@ -1006,61 +1024,34 @@ void measure_configs_impl(mvmc_ens* E, int count, const int* ele_idx, double* e_
     ~RestoreW() { view.W = w; }
   } restore{v, W0};
   hipStream_t st = E->st;
+  if (!E->d_cfg) E->d_cfg = dalloc<int>(E->allocs, (size_t)W0 * n);
+  const size_t ob = sizeof(double) * size, row = ob + sizeof(double) + sizeof(int);
+  if (nsamp > 1 && !E->d_cfg_out) E->d_cfg_out = dalloc<char>(E->allocs, (size_t)W0 * row);
+  raise_lds_limit((const void*)k_config_slots, sizeof(int) * std::max(v.nproj, 1));
+  // rows of sample s to the host: in place with one sample per walker, else packed first
+  auto down = [&](auto* dst, auto* src, int width, int s, int wl, size_t off) {
+    using T = std::remove_pointer_t<decltype(dst)>;
+    const T* from = src;
+    if (nsamp > 1) {
+      T* to = reinterpret_cast<T*>(E->d_cfg_out + off);
+      const long long total = (long long)wl * width;
+      hipLaunchKernelGGL(k_pack_sample<T>, dim3(nblk(total)), dim3(256), 0, st, src, nsamp, s, width, total, to);
+      from = to;
+    }
+    HIPCHK(hipMemcpyAsync(dst, from, sizeof(T) * wl * width, hipMemcpyDeviceToHost, st));
+  };
   for (int s = 0; (long long)s * W0 < count; ++s) {
     const int base = s * W0, wl = std::min(W0, count - base);
-    std::vector<int> idx((size_t)wl * n), cfg((size_t)wl * n2, -1), num((size_t)wl * n2, 0), pc((size_t)wl * npc, 0);
-    for (int w = 0; w < wl; ++w) {
-      const int* e = ele_idx + (size_t)(base + w) * n;
-      int* cf = cfg.data() + (size_t)w * n2;
-      int* nm = num.data() + (size_t)w * n2;
-      for (int mi = 0; mi < n; ++mi) {
-        const int ri = e[mi];
-        if (ri < 0 || ri >= ns)
-          throw Fail(MVMC_E_INPUT, "configuration " + std::to_string(base + w) + ": site index out of range");
-        const int slot = ri + (mi / ne) * ns;
-        if (cf[slot] != -1)
-          throw Fail(MVMC_E_INPUT, "configuration " + std::to_string(base + w) + ": two electrons of one spin on a site");
-        cf[slot] = mi % ne;
-        nm[slot] = 1;
-        idx[(size_t)w * n + mi] = ri;
-      }
-      int* cnt = pc.data() + (size_t)w * npc;
-      for (int ri = 0; ri < ns; ++ri) {
-        const int g = m.gutz_idx[ri];
-        if (g >= 0 && g < np) cnt[g] += nm[ri] * nm[ri + ns];
-      }
-      if (np > m.n_gutz)
-        for (int ri = 0; ri < ns; ++ri) {
-          const int xi = nm[ri] + nm[ri + ns] - 1;
-          if (xi == 0) continue;
-          for (int rj = ri + 1; rj < ns; ++rj) {
-            const int j = m.jast_idx[(size_t)ri * ns + rj];
-            if (j < 0) continue;
-            cnt[m.n_gutz + j] += xi * (nm[rj] + nm[rj + ns] - 1);
-          }
-        }
-    }
-    auto put = [&](int* dst, const std::vector<int>& src, int width) {
-      HIPCHK(hipMemcpy2DAsync(dst + (size_t)s * width, sizeof(int) * nsamp * width, src.data(), sizeof(int) * width,
-                              sizeof(int) * width, wl, hipMemcpyHostToDevice, st));
-    };
-    put(v.s_idx, idx, n);
-    put(v.s_cfg, cfg, n2);
-    put(v.s_num, num, n2);
-    if (np > 0) put(v.s_proj, pc, np);
+    HIPCHK(hipMemcpyAsync(E->d_cfg, ele_idx + (size_t)base * n, sizeof(int) * wl * n, hipMemcpyHostToDevice, st));
     v.W = wl;
+    hipLaunchKernelGGL(k_config_slots, dim3(wl), dim3(64), sizeof(int) * std::max(v.nproj, 1), st, v, s, E->d_cfg);
     launch_meas_rebuild(E, s);
     hipLaunchKernelGGL(k_measure<false>, dim3(E->grid_meas), dim3(256), E->lds_meas, st, v, GroupArgs{}, 1, s);
     HIPCHK(hipGetLastError());
     v.W = W0;
-    HIPCHK(hipMemcpy2DAsync(e_loc + base, sizeof(double), v.e_loc + s, sizeof(double) * nsamp, sizeof(double), wl,
-                            hipMemcpyDeviceToHost, st));
-    if (o)
-      HIPCHK(hipMemcpy2DAsync(o + (size_t)base * size, sizeof(double) * size, v.o_store + (size_t)s * size,
-                              sizeof(double) * size * nsamp, sizeof(double) * size, wl, hipMemcpyDeviceToHost, st));
-    if (valid)
-      HIPCHK(hipMemcpy2DAsync(valid + base, sizeof(int), v.s_valid + s, sizeof(int) * nsamp, sizeof(int), wl,
-                              hipMemcpyDeviceToHost, st));
+    down(e_loc + base, v.e_loc, 1, s, wl, (size_t)W0 * ob);
+    if (o) down(o + (size_t)base * size, v.o_store, size, s, wl, 0);
+    if (valid) down(valid + base, v.s_valid, 1, s, wl, (size_t)W0 * (ob + sizeof(double)));
     HIPCHK(hipStreamSynchronize(st));
   }
   E->check_status();

@@ -218,6 +218,103 @@ __device__ inline double ip_of_l(const double* qpw, const double* pf, int nqp) {
 }
 
 // ---------------------------------------------------------------------------
+// Tables of the current parameters, on the device (only the parameters cross
+// the bus: the 16 x 16 lattice's Slater table is 16.8 MB).
+// ---------------------------------------------------------------------------
+// Slater table (update_slater_elm, slater_update.rs:17-126), a thread per
+// (plane, site, site): its four spin blocks.
+__global__ void k_slater_table(EnsView v, const double* orb, double* table) {
+  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int ns = v.ns, n2 = v.n2;
+  if (e >= (long long)v.nqp * ns * ns) return;
+  const int rj = (int)(e % ns), ri = (int)(e / ns % ns), qp = (int)(e / ((long long)ns * ns));
+  const int sp = qp % v.nleg, mp = (qp % (v.nleg * v.nmp)) / v.nleg;
+  const double cs = v.spgl_cs[sp], cc = v.spgl_cc[sp], ss = v.spgl_ss[sp];
+  const int ti = v.tsite[(size_t)mp * ns + ri], tj = v.tsite[(size_t)mp * ns + rj];
+  const int qs = v.tsgn[(size_t)mp * ns + ri] * v.tsgn[(size_t)mp * ns + rj];
+  const int ij = v.orb_idx[(size_t)ti * ns + tj], ji = v.orb_idx[(size_t)tj * ns + ti];
+  double* plane = table + (size_t)qp * n2 * n2;
+  double uu = 0.0, ud = 0.0, du = 0.0, dd = 0.0;
+  if (ij >= 0 && ji >= 0) {
+    const double fij = orb[ij] * (double)(v.orb_sgn[(size_t)ti * ns + tj] * qs);
+    const double fji = orb[ji] * (double)(v.orb_sgn[(size_t)tj * ns + ti] * qs);
+    uu = -(fij - fji) * cs;
+    ud = fij * cc + fji * ss;
+    du = -fij * ss - fji * cc;
+    dd = (fij - fji) * cs;
+  }
+  plane[(size_t)ri * n2 + rj] = uu;
+  plane[(size_t)ri * n2 + rj + ns] = ud;
+  plane[(size_t)(ri + ns) * n2 + rj] = du;
+  plane[(size_t)(ri + ns) * n2 + rj + ns] = dd;
+}
+
+// Projection parameters by site and by pair (the direct ratio of the
+// measurement, observables.rs:1638-1672).
+__global__ void k_proj_tables(EnsView v, double* gutz, double* jast) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ns = v.ns, nj = v.nproj - v.ngutz;
+  if (e >= ns * ns) return;
+  const int a = e / ns, b = e % ns;
+  const int k = a != b ? v.jast_idx[e] : -1;
+  jast[e] = k >= 0 && k < nj ? v.proj[v.ngutz + k] : 0.0;
+  if (b == 0) {
+    const int g = v.gutz_idx[a];
+    gutz[a] = g >= 0 && g < v.ngutz ? v.proj[g] : 0.0;
+  }
+}
+
+// Saved-sample slot s of walkers 0 .. wl-1 from configurations idx [wl][n]
+// (EleIdx; checked by the host): EleIdx, EleCfg, EleNum and the projection
+// counts (projection.rs:179-277), a workgroup per configuration; the counts
+// are integers, so lanes add them in any order.  LDS: nproj ints.
+__global__ void __launch_bounds__(64) k_config_slots(EnsView v, int s, const int* idx) {
+  extern __shared__ __align__(16) int cnt[];
+  const int w = blockIdx.x, tid = threadIdx.x, n = v.n, ns = v.ns, n2 = v.n2, np = v.nproj;
+  const size_t ws = (size_t)w * v.nsample + s;
+  int* cfg = v.s_cfg + ws * n2;
+  int* num = v.s_num + ws * n2;
+  for (int i = tid; i < n2; i += 64) {
+    cfg[i] = -1;
+    num[i] = 0;
+  }
+  for (int i = tid; i < np; i += 64) cnt[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < n; i += 64) {
+    const int r = idx[(size_t)w * n + i], slot = r + (i / v.ne) * ns;
+    v.s_idx[ws * n + i] = r;
+    cfg[slot] = i % v.ne;
+    num[slot] = 1;
+  }
+  __syncthreads();
+  for (int r = tid; r < ns; r += 64) {
+    const int g = v.gutz_idx[r];
+    if (g >= 0 && g < np) atomicAdd(&cnt[g], num[r] * num[r + ns]);
+  }
+  if (np > v.ngutz)
+    for (int ri = 0; ri < ns; ++ri) {
+      const int xi = num[ri] + num[ri + ns] - 1;
+      if (xi == 0) continue;
+      for (int rj = ri + 1 + tid; rj < ns; rj += 64) {
+        const int j = v.jast_idx[(size_t)ri * ns + rj];
+        const int xj = num[rj] + num[rj + ns] - 1;
+        if (j >= 0 && xj != 0) atomicAdd(&cnt[v.ngutz + j], xi * xj);
+      }
+    }
+  __syncthreads();
+  for (int i = tid; i < np; i += 64) v.s_proj[ws * np + i] = cnt[i];
+}
+
+// Rows [W][nsample][width] of sample s, packed [wl][width].
+template <class T>
+__global__ void k_pack_sample(const T* src, int nsample, int s, int width, long long total, T* dst) {
+  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= total) return;
+  const long long w = e / width;
+  dst[e] = src[(w * nsample + s) * width + e % width];
+}
+
+// ---------------------------------------------------------------------------
 // seeding: init_gen_rand(seed + w), then `skip` words (init_parameter draws)
 // ---------------------------------------------------------------------------
 __global__ void k_seed(EnsView v, long long base_seed, int skip) {

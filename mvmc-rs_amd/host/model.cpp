@@ -463,40 +463,6 @@ void translation_maps(const Model& m, std::vector<int>& tsite, std::vector<int>&
     for (int r = 0; r < ns; ++r) translated_site(m, r, t, tsite[(size_t)t * ns + r], tsgn[(size_t)t * ns + r]);
 }
 
-void build_slater_table(const Model& m, std::vector<double>& table) {
-  const int ns = m.nsite(), n2 = m.nsite2(), nleg = m.n_sp_gl(), nqp = m.nqp();
-  table.assign((size_t)nqp * n2 * n2, 0.0);
-  for (int qp = 0; qp < nqp; ++qp) {
-    double* plane = table.data() + (size_t)qp * n2 * n2;
-    const int spidx = qp % nleg;
-    const int mpidx = (qp % (nleg * m.n_mp_trans())) / nleg;
-    const double cs = m.spgl_cos_sin[spidx], cc = m.spgl_cos_cos[spidx], ss = m.spgl_sin_sin[spidx];
-    for (int ri = 0; ri < ns; ++ri) {
-      int tri, sgni;
-      translated_site(m, ri, mpidx, tri, sgni);
-      if (tri < 0 || tri >= ns) continue;
-      for (int rj = 0; rj < ns; ++rj) {
-        int trj, sgnj;
-        translated_site(m, rj, mpidx, trj, sgnj);
-        if (trj < 0 || trj >= ns) continue;
-        const int qpsgn = sgni * sgnj;
-        const int idx_ij = m.orb_idx[(size_t)tri * ns + trj];
-        const int idx_ji = m.orb_idx[(size_t)trj * ns + tri];
-        if (idx_ij < 0 || idx_ji < 0) continue;
-        const int sgn_ij = m.orb_sgn[(size_t)tri * ns + trj] * qpsgn;
-        const int sgn_ji = m.orb_sgn[(size_t)trj * ns + tri] * qpsgn;
-        const double slt_ij = m.slater[idx_ij] * (double)sgn_ij;
-        const double slt_ji = m.slater[idx_ji] * (double)sgn_ji;
-        const int rsi0 = ri, rsi1 = ri + ns, rsj0 = rj, rsj1 = rj + ns;
-        plane[(size_t)rsi0 * n2 + rsj0] = -(slt_ij - slt_ji) * cs;
-        plane[(size_t)rsi0 * n2 + rsj1] = slt_ij * cc + slt_ji * ss;
-        plane[(size_t)rsi1 * n2 + rsj0] = -slt_ij * ss - slt_ji * cc;
-        plane[(size_t)rsi1 * n2 + rsj1] = (slt_ij - slt_ji) * cs;
-      }
-    }
-  }
-}
-
 void sync_modified_parameter(Model& m, bool shift_correlations) {
   const int ng = m.n_gutz, nj = m.n_jast;
   bool all_active = true;
@@ -516,23 +482,6 @@ void sync_modified_parameter(Model& m, bool shift_correlations) {
     const double ratio = 4.0 / xmax;  // D_AMP_MAX
     for (double& v : m.slater) v *= ratio;
   }
-}
-
-void direct_projection_tables(const Model& m, std::vector<double>& gutz, std::vector<double>& jast) {
-  const int n = m.nsite();
-  gutz.assign(n, 0.0);
-  jast.assign((size_t)n * n, 0.0);
-  for (int s = 0; s < n; ++s) {
-    int idx = m.gutz_idx[s];
-    if (m.n_gutz > 0 && idx >= 0 && idx < m.n_gutz) gutz[s] = m.proj[idx];
-  }
-  if (m.n_jast > 0)
-    for (int a = 0; a < n; ++a)
-      for (int b = 0; b < n; ++b) {
-        if (a == b) continue;
-        int idx = m.jast(a, b);
-        if (idx >= 0 && idx < m.n_jast) jast[(size_t)a * n + b] = m.proj[m.n_gutz + idx];
-      }
 }
 
 }  // namespace mvmc

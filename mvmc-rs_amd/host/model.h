@@ -126,10 +126,6 @@ bool load_initial_def(Model& m, const std::string& path);
 // (crates/mvmc-expert-parsers/src/utils/qp_weight.rs:24-146).
 void init_qp_weight(Model& m);
 
-// Slater table S[qp][2Ns][2Ns] from the current orbital parameters
-// (crates/mvmc-core/src/slater_update.rs:17-126, real branch).
-void build_slater_table(const Model& m, std::vector<double>& table);
-
 // Gauge fixing after every parameter change: Gutzwiller/Jastrow mean shift
 // when every projection parameter is optimised, then Slater rescaled to
 // max|f| = 4 (crates/mvmc-expert-parsers/src/utils/parameter_init.rs:168-265,
@@ -139,11 +135,6 @@ void sync_modified_parameter(Model& m, bool shift_correlations);
 // Translated site / sign of `site` under translation `mpidx`
 // (crates/mvmc-core/src/qp.rs:30-70 with no OptTrans).
 void translated_site(const Model& m, int site, int mpidx, int& out_site, int& out_sign);
-
-// Flattened tables of the direct transfer projection ratio
-// (crates/mvmc-core/src/observables.rs:1553-1605).
-void direct_projection_tables(const Model& m, std::vector<double>& gutz,
-                              std::vector<double>& jast);
 
 // Per-translation orbital index/sign of electron pairs are data-dependent;
 // this returns the static translated site map [n_mp_trans][nsite] and sign.
