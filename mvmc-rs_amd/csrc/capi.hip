@@ -962,8 +962,8 @@ void measure_impl(mvmc_ens* E) {
 // (run.rs:1863-1903, average.rs:18-63), on the handle's stream.
 void measure_finish(mvmc_ens* E) {
   EnsView& v = E->v;
-  hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(64), 0, E->st, v, E->d_out5);
-  hipLaunchKernelGGL(k_reduce_ops, dim3(nblk(v.size)), dim3(256), 0, E->st, v, E->d_ho, E->d_mean, E->d_diag);
+  hipLaunchKernelGGL(k_reduce_energy, dim3(1), dim3(RE_NT), 0, E->st, v, E->d_out5);
+  hipLaunchKernelGGL(k_reduce_ops, dim3(nblk(v.size, 64)), dim3(64), 0, E->st, v, E->d_ho, E->d_mean, E->d_diag);
   HIPCHK(hipGetLastError());
   double o5[5];
   std::vector<double> ho(v.size), mean(v.size), diag(v.size);
@@ -2067,7 +2067,7 @@ int mvmc_ens_vjp(mvmc_ens* e, const double* cot, double* grad) {
     if (!e->d_rows) e->d_rows = dalloc<double>(e->allocs, rows);
     if (!e->d_grad) e->d_grad = dalloc<double>(e->allocs, (size_t)v.size);
     HIPCHK(hipMemcpyAsync(e->d_rows, cot, sizeof(double) * rows, hipMemcpyHostToDevice, e->st));
-    hipLaunchKernelGGL(k_vjp, dim3(nblk(v.size)), dim3(256), 0, e->st, v, e->d_rows, e->d_grad);
+    hipLaunchKernelGGL(k_vjp, dim3(nblk(v.size, 64)), dim3(64), 0, e->st, v, e->d_rows, e->d_grad);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(grad, e->d_grad, sizeof(double) * v.size, hipMemcpyDeviceToHost, e->st));
     HIPCHK(hipStreamSynchronize(e->st));
@@ -2172,7 +2172,7 @@ int mvmc_ens_vjp_adjoint(mvmc_ens* e, const double* cot, double* grad) {
                        e->adj_slots, len);
     hipLaunchKernelGGL(k_adj_fold, dim3((unsigned)((glen + 255) / 256)), dim3(256), 0, e->st, e->d_gproj,
                        e->adj_slots, glen);
-    hipLaunchKernelGGL(k_adj_orbital, dim3(nblk(v.size)), dim3(256), 0, e->st, e->d_sbar, e->d_adj_start,
+    hipLaunchKernelGGL(k_adj_orbital, dim3(nblk(v.size, 64)), dim3(64), 0, e->st, e->d_sbar, e->d_adj_start,
                        e->d_adj_ent, e->d_adj_wt, e->d_gproj, v.nproj, v.nslater, e->d_grad);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(ev[1], e->st));

@@ -1928,14 +1928,27 @@ __global__ void k_log_psi(EnsView v, int s, double* out) {
 
 // Vector-Jacobian product over the stored samples: grad[k] = sum_r cot[r] *
 // O[r][k], r ascending (r = walker * NVMCSample + sample), O = [1,
-// d log|psi| / d p] per sample as the measurement stored it.  One thread
-// per component; consecutive threads read consecutive components.
-__global__ void k_vjp(EnsView v, const double* cot, double* grad) {
+// d log|psi| / d p] per sample as the measurement stored it.  One lane per
+// component; consecutive lanes read consecutive components, the rows of
+// VJP_U samples loaded together ahead of their adds.
+constexpr int VJP_U = 16;
+__global__ void __launch_bounds__(64) k_vjp(EnsView v, const double* cot, double* grad) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= v.size) return;
   const size_t rows = (size_t)v.W * v.nsample;
   double acc = 0.0;
-  for (size_t r = 0; r < rows; ++r) acc += cot[r] * v.o_store[r * v.size + k];
+  size_t r = 0;
+  for (; r + VJP_U <= rows; r += VJP_U) {
+    double o[VJP_U], c[VJP_U];
+#pragma unroll
+    for (int u = 0; u < VJP_U; ++u) {
+      o[u] = v.o_store[(r + u) * v.size + k];
+      c[u] = cot[r + u];
+    }
+#pragma unroll
+    for (int u = 0; u < VJP_U; ++u) acc += c[u] * o[u];
+  }
+  for (; r < rows; ++r) acc += cot[r] * v.o_store[r * v.size + k];
   grad[k] = acc;
 }
 
@@ -2008,6 +2021,7 @@ __global__ void k_adj_fold(double* buf, int nslots, long long len) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= len) return;
   double a = buf[e];
+#pragma unroll 16
   for (int sl = 1; sl < nslots; ++sl) a += buf[(size_t)sl * len + e];
   buf[e] = a;
 }
@@ -2026,36 +2040,107 @@ __global__ void k_adj_orbital(const double* sbar, const int* start, const long l
   const int orb = k - 1 - nproj;
   if (orb >= nslater) return;
   double a = 0.0;
-  for (int t = start[orb]; t < start[orb + 1]; ++t) a += sbar[ent[t]] * wt[t];
+  int t = start[orb];
+  const int t1 = start[orb + 1];
+  constexpr int U = 16;  // gathered together ahead of the chain of adds
+  for (; t + U <= t1; t += U) {
+    double b[U], x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      b[u] = sbar[ent[t + u]];
+      x[u] = wt[t + u];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) a += b[u] * x[u];
+  }
+  for (; t < t1; ++t) a += sbar[ent[t]] * wt[t];
   grad[k] = a;
 }
 
-__global__ void k_reduce_energy(EnsView v, double* out5) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  double tot[5] = {0, 0, 0, 0, 0};
-  for (int w = 0; w < v.W; ++w) {
-    double a[5] = {0, 0, 0, 0, 0};
-    for (int s = 0; s < v.nsample; ++s) {
-      const size_t ws = (size_t)w * v.nsample + s;
-      if (!v.s_valid[ws]) continue;
-      const double e = v.e_loc[ws], sz = v.sz[ws], wt = 1.0;
-      a[0] += wt;
-      a[1] += wt * e;
-      a[2] += (wt * e) * e;
-      a[3] += wt * sz;
-      a[4] += wt * sz * sz;
+// Energy sums: five left folds over the walkers.  The walkers' terms are
+// formed by all threads, a tile of RE_TILE walkers at a time into LDS, and
+// five lanes of the first wave fold the tile before (one thread with its
+// loads in the chain took 990 us for 4096 walkers).
+constexpr int RE_TILE = 512, RE_NT = 320;
+__global__ void __launch_bounds__(RE_NT) k_reduce_energy(EnsView v, double* out5) {
+  __shared__ double term[2][5][RE_TILE];
+  const int tid = threadIdx.x;
+  auto fill = [&](int w0, int buf) {
+    for (int k = tid - 64; k < RE_TILE && w0 + k < v.W; k += RE_NT - 64) {
+      if (k < 0) continue;
+      double a[5] = {0, 0, 0, 0, 0};
+      for (int s = 0; s < v.nsample; ++s) {
+        const size_t ws = (size_t)(w0 + k) * v.nsample + s;
+        if (!v.s_valid[ws]) continue;
+        const double e = v.e_loc[ws], sz = v.sz[ws], wt = 1.0;
+        a[0] += wt;
+        a[1] += wt * e;
+        a[2] += (wt * e) * e;
+        a[3] += wt * sz;
+        a[4] += wt * sz * sz;
+      }
+      for (int c = 0; c < 5; ++c) term[buf][c][k] = a[c];
     }
-    for (int k = 0; k < 5; ++k) tot[k] = (w == 0) ? a[k] : tot[k] + a[k];
+  };
+  if (tid >= 64) fill(0, 0);
+  __syncthreads();
+  double tot = 0.0;
+  for (int w0 = 0, buf = 0; w0 < v.W; w0 += RE_TILE, buf ^= 1) {
+    if (tid >= 64) {
+      if (w0 + RE_TILE < v.W) fill(w0 + RE_TILE, buf ^ 1);
+    } else if (tid < 5) {
+      const double* t = term[buf][tid];
+      const int cnt = min(RE_TILE, v.W - w0);
+      int k = 0;
+      if (w0 == 0) tot = t[k++];
+      for (; k + 16 <= cnt; k += 16) {
+        double x[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[u] = t[k + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) tot += x[u];
+      }
+      for (; k < cnt; ++k) tot += t[k];
+    }
+    __syncthreads();
   }
-  for (int k = 0; k < 5; ++k) out5[k] = tot[k];
+  if (tid < 5) out5[tid] = tot;
 }
 
-// ho[i], mean[i], diag[i] (CG mode: finalize_oo_store_real diagonal_only)
-__global__ void k_reduce_ops(EnsView v, double* ho, double* mean, double* diag) {
+// ho[i], mean[i], diag[i] (CG mode: finalize_oo_store_real diagonal_only): a
+// left fold over the walkers per component, a lane per component; RO_U
+// walkers' rows are loaded together ahead of their adds, and the workgroups
+// are single waves so that more CUs stream the O rows.
+constexpr int RO_U = 16;
+__global__ void __launch_bounds__(64) k_reduce_ops(EnsView v, double* ho, double* mean, double* diag) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= v.size) return;
   double th = 0, tm = 0, td = 0;
-  for (int w = 0; w < v.W; ++w) {
+  auto add = [&](int w, double h, double m, double d) {
+    if (w == 0) { th = h; tm = m; td = d; }
+    else { th += h; tm += m; td += d; }
+  };
+  int w = 0;
+  if (v.nsample == 1)
+    for (; w + RO_U <= v.W; w += RO_U) {
+      double o[RO_U], e[RO_U];
+      int ok[RO_U];
+#pragma unroll
+      for (int u = 0; u < RO_U; ++u) {
+        o[u] = v.o_store[(size_t)(w + u) * v.size + i];
+        e[u] = v.e_loc[w + u];
+        ok[u] = v.s_valid[w + u];
+      }
+#pragma unroll
+      for (int u = 0; u < RO_U; ++u) {
+        double h = 0.0, m = 0.0, d = 0.0;
+        if (ok[u]) h += (1.0 * e[u]) * o[u];
+        m += o[u];
+        d += o[u] * o[u];
+        add(w + u, h, m, d);
+      }
+    }
+  for (; w < v.W; ++w) {
     double h = 0.0, m = 0.0, d = 0.0;
     for (int s = 0; s < v.nsample; ++s) {
       const size_t ws = (size_t)w * v.nsample + s;
@@ -2064,8 +2149,7 @@ __global__ void k_reduce_ops(EnsView v, double* ho, double* mean, double* diag) 
       m += o;
       d += o * o;
     }
-    if (w == 0) { th = h; tm = m; td = d; }
-    else { th += h; tm += m; td += d; }
+    add(w, h, m, d);
   }
   ho[i] = th;
   mean[i] = tm;
