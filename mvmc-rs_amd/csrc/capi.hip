@@ -677,7 +677,7 @@ void create_impl(mvmc_ens* E, const char* namelist, const char* initial_def, int
   HIPCHK(hipMemsetAsync(v.ele_num, 0, sizeof(int) * W * v.n2, E->st));
   HIPCHK(hipMemsetAsync(v.proj_cnt, 0, sizeof(int) * W * std::max(v.nproj, 1), E->st));
   // persistent grids sized to the resident capacity
-  E->lds_samp = lds_bytes_sampler(v, 256);
+  E->lds_samp = lds_bytes_sampler(v);
   E->lds_meas = lds_bytes_measure(v, 256);
   int dev = 0, ncu = 0, maxlds = 0;
   HIPCHK(hipGetDevice(&dev));

@@ -86,22 +86,48 @@ __host__ __device__ inline size_t union_doubles_sampler(const EnsView& v) {
   const size_t nq = (size_t)v.nqp * v.n;
   size_t hop = 3 * (size_t)v.nqp * hop_ld(v.n);
   size_t ex = v.ex_path != 0 ? 5 * nq + 16 * (size_t)v.nqp : 0;
+  if (v.ex_path != 0 && ex < 4 * (size_t)v.ns + 16) ex = 4 * (size_t)v.ns + 16;
   size_t m = hop > ex ? hop : ex;
   size_t pfb = (pf_bytes(v.n, v.nqp) + 7) / 8;
   return m > pfb ? m : pfb;
 }
 
-__host__ __device__ inline size_t lds_bytes_sampler(const EnsView& v, int nthreads) {
+// Projection parameters a proposal can change: two per site and hop, and the
+// hopped sites' own.  A hop's terms have an array of their own (rows are
+// staged into the union meanwhile); an exchange's stand in the union, which
+// is free until they are summed.
+__host__ __device__ inline int term_cap(const EnsView& v) { return (v.ex_path != 0 ? 4 : 2) * v.ns + 16; }
+// (40960 parameters' deltas would fill the LDS: the indices fit 16 bits.)
+__host__ __device__ inline int hop_cap(const EnsView& v) { return 2 * v.ns + 16; }
+// The tables below go to LDS only where the rows of the planes leave room for
+// them (2048 doubles a row array: at most 80 KiB of the 160).
+__host__ __device__ inline bool lds_tables(const EnsView& v) { return v.nqp * v.n <= 2048 && v.nproj <= 8192; }
+// Entries of the Jastrow index table (16 bits each) and of the projection
+// parameters that the sampler keeps in LDS: those of the smaller models,
+// whose proposals wait for little else than these loads (L2: 0.3 us each).
+__host__ __device__ inline int jast_lds(const EnsView& v) {
+  return v.ns <= 64 && v.nproj > v.ngutz && lds_tables(v) ? v.ns * v.ns : 0;
+}
+__host__ __device__ inline int proj_lds(const EnsView& v) { return v.nproj <= 256 && lds_tables(v) ? v.nproj : 0; }
+// Words of the bitmap of projection parameters a proposal touches; few
+// parameters are scanned directly instead (0).
+__host__ __device__ inline int touch_words(const EnsView& v) {
+  return v.nproj > 512 && lds_tables(v) ? (v.nproj + 31) / 32 : 0;
+}
+
+__host__ __device__ inline size_t lds_bytes_sampler(const EnsView& v) {
   size_t b = 0;
   b += rnd16(sizeof(SfmtLds));
   b += rnd16((size_t)v.n * 4) + 2 * rnd16((size_t)v.n2 * 4);
   b += rnd16(64 * 4);                      // misc ints
   b += 2 * rnd16((size_t)v.nqp * 8) + rnd16(32 * 8);  // pf, pf_new, dmisc
   b += rnd16((size_t)(v.nproj > 0 ? v.nproj : 1) * 4);  // delta
-  b += rnd16((size_t)(4 * v.ns + 16) * 8);  // compacted terms
-  b += rnd16((size_t)(nthreads + 64) * 4); // scan
+  b += rnd16((size_t)hop_cap(v) * 8);   // terms of the changed projection parameters
+  b += rnd16((size_t)term_cap(v) * 2);  // their indices
   b += rnd16((size_t)v.n * 4);             // rs
   b += 2 * rnd16((size_t)v.ns * 4) + rnd16((size_t)v.nqp * 8);  // loc_spn, gutz_idx, qpw copies
+  b += rnd16((size_t)jast_lds(v) * 2) + rnd16((size_t)proj_lds(v) * 8);  // jast_idx, proj copies
+  b += rnd16((size_t)touch_words(v) * 4);  // touched projection parameters
   b += rnd16(union_doubles_sampler(v) * 8);
   return b;
 }
@@ -123,28 +149,6 @@ __host__ __device__ inline size_t lds_bytes_measure(const EnsView& v, int nthrea
 // small block helpers
 // ---------------------------------------------------------------------------
 __device__ inline void set_status(int* st, int code) { atomicCAS(st, 0, code); }
-
-// Exclusive block scan of one int per thread; returns the total via *total.
-__device__ inline int block_exscan(int v, int* scan, int* total) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = (blockDim.x + 63) >> 6;
-  int x = v;
-  for (int off = 1; off < 64; off <<= 1) {
-    int y = __shfl_up(x, off, 64);
-    if (lane >= off) x += y;
-  }
-  if (lane == 63 || tid == (int)blockDim.x - 1) scan[wave] = x;
-  __syncthreads();
-  if (tid == 0) {
-    int acc = 0;
-    for (int k = 0; k < nw; ++k) { int t = scan[k]; scan[k] = acc; acc += t; }
-    scan[nw] = acc;
-  }
-  __syncthreads();
-  const int ex = scan[wave] + x - v;
-  *total = scan[nw];
-  __syncthreads();
-  return ex;
-}
 
 // calc_m_all for one walker: assemble, LTL, Pfaffian, inverse, negate.
 // native = true skips the all-zero guard (C's separate real setup).
@@ -357,11 +361,15 @@ __global__ void k_seed(EnsView v, long long base_seed, int skip) {
 // ---------------------------------------------------------------------------
 struct SampLds {
   SfmtLds* rng;
-  int *ele_idx, *ele_cfg, *ele_num, *misc, *delta, *scan, *rs;
+  int *ele_idx, *ele_cfg, *ele_num, *misc, *delta, *rs;
+  unsigned short* tidx;
   double *pf, *pf_new, *dmisc, *terms, *uni;
   // copies of small model tables read on the serial lane-0 path
   int *loc_spn, *gutz_idx;
   double* qpw;
+  short* jast;    // [ns * ns], or null (jast_lds)
+  double* proj;   // [nproj], or null (proj_lds)
+  unsigned* touch;  // bitmap, or null (touch_words)
 };
 
 __device__ inline SampLds carve_sampler(const EnsView& v, char* base) {
@@ -376,12 +384,15 @@ __device__ inline SampLds carve_sampler(const EnsView& v, char* base) {
   L.pf_new = c.take<double>(v.nqp);
   L.dmisc = c.take<double>(32);
   L.delta = c.take<int>(v.nproj > 0 ? v.nproj : 1);
-  L.terms = c.take<double>(4 * v.ns + 16);
-  L.scan = c.take<int>(blockDim.x + 64);
+  L.terms = c.take<double>(hop_cap(v));
+  L.tidx = c.take<unsigned short>(term_cap(v));
   L.rs = c.take<int>(v.n);
   L.loc_spn = c.take<int>(v.ns);
   L.gutz_idx = c.take<int>(v.ns);
   L.qpw = c.take<double>(v.nqp);
+  L.jast = jast_lds(v) ? c.take<short>(jast_lds(v)) : nullptr;
+  L.proj = proj_lds(v) ? c.take<double>(proj_lds(v)) : nullptr;
+  L.touch = touch_words(v) ? c.take<unsigned>(touch_words(v)) : nullptr;
   L.uni = c.take<double>(union_doubles_sampler(v));
   return L;
 }
@@ -394,37 +405,65 @@ __device__ inline void load_tables(const EnsView& v, SampLds& L) {
     L.gutz_idx[i] = v.gutz_idx[i];
   }
   for (int q = threadIdx.x; q < v.nqp; q += blockDim.x) L.qpw[q] = v.qpw[q];
+  if (L.jast)
+    for (int i = threadIdx.x; i < v.ns * v.ns; i += blockDim.x) L.jast[i] = (short)v.jast_idx[i];
+  if (L.proj)
+    for (int i = threadIdx.x; i < v.nproj; i += blockDim.x) L.proj[i] = v.proj[i];
+  if (L.touch)
+    for (int i = threadIdx.x; i < touch_words(v); i += blockDim.x) L.touch[i] = 0;
 }
 
-// Serial sum_k a[k] * b[k] (k ascending) over LDS arrays, with the operands
-// of DOT_U terms read into registers ahead of their dependent adds.
-constexpr int DOT_U = 16;
-__device__ inline double lds_serial_dot(const double* a, const double* b, int n) {
+// Serial sum_k a[k] * b[k] (k ascending) over LDS arrays: the chain of adds
+// is what it takes, so the operands of the next DOT_U terms are read while
+// the current ones are added (a test per term and a wait per batch took 75
+// cycles a term).
+constexpr int DOT_U = 8;
+__device__ __forceinline__ double lds_serial_dot(const double* a, const double* b, int n) {
   double r = 0.0;
-  for (int k0 = 0; k0 < n; k0 += DOT_U) {
-    double av[DOT_U], bv[DOT_U];
+  int k = 0;
+  if (n >= DOT_U) {
+    double x[DOT_U], y[DOT_U];
 #pragma unroll
-    for (int u = 0; u < DOT_U; ++u)
-      if (k0 + u < n) { av[u] = a[k0 + u]; bv[u] = b[k0 + u]; }
+    for (int u = 0; u < DOT_U; ++u) { x[u] = a[u]; y[u] = b[u]; }
+    for (; k + 2 * DOT_U <= n; k += DOT_U) {
+      double p[DOT_U];
 #pragma unroll
-    for (int u = 0; u < DOT_U; ++u)
-      if (k0 + u < n) r += av[u] * bv[u];
+      for (int u = 0; u < DOT_U; ++u) p[u] = x[u] * y[u];
+#pragma unroll
+      for (int u = 0; u < DOT_U; ++u) { x[u] = a[k + DOT_U + u]; y[u] = b[k + DOT_U + u]; }
+#pragma unroll
+      for (int u = 0; u < DOT_U; ++u) r += p[u];
+    }
+#pragma unroll
+    for (int u = 0; u < DOT_U; ++u) r += x[u] * y[u];
+    k += DOT_U;
   }
+  for (; k < n; ++k) r += a[k] * b[k];
   return r;
 }
 
-// Serial r + sum_{k0 <= k < k1} a[k] (k ascending) over an LDS array, same
-// prefetching; a sum split at any k is the unsplit sum.
-__device__ inline double lds_serial_sum(const double* a, int k0, int k1, double r) {
-  for (int kb = k0; kb < k1; kb += DOT_U) {
-    double av[DOT_U];
+// Serial r + sum_{k0 <= k < k1} a[k] (k ascending) over an LDS array, the
+// same way; a sum split at any k is the unsplit sum.
+__device__ __forceinline__ double lds_serial_sum(const double* a, int k0, int k1, double r) {
+  int k = k0;
+  if (k1 - k0 >= DOT_U) {
+    double x[DOT_U];
 #pragma unroll
-    for (int u = 0; u < DOT_U; ++u)
-      if (kb + u < k1) av[u] = a[kb + u];
+    for (int u = 0; u < DOT_U; ++u) x[u] = a[k + u];
+    for (; k + 2 * DOT_U <= k1; k += DOT_U) {
+      double p[DOT_U];
 #pragma unroll
-    for (int u = 0; u < DOT_U; ++u)
-      if (kb + u < k1) r += av[u];
+      for (int u = 0; u < DOT_U; ++u) p[u] = x[u];
+#pragma unroll
+      for (int u = 0; u < DOT_U; ++u) x[u] = a[k + DOT_U + u];
+#pragma unroll
+      for (int u = 0; u < DOT_U; ++u) r += p[u];
+    }
+#pragma unroll
+    for (int u = 0; u < DOT_U; ++u) r += x[u];
+    k += DOT_U;
   }
+  for (; k < k1; ++k) r += a[k];
   return r;
 }
 
@@ -592,89 +631,141 @@ __global__ void __launch_bounds__(256) k_begin(EnsView v_arg, GroupArgs ga, int 
 }
 
 // ---------------------------------------------------------------------------
-// Projection-count deltas of a hop ri -> rj (post-hop occupations) into
-// LDS `delta` (integer adds commute, so lanes may add concurrently).
+// Projection of a proposal, by wave 0 alone (the other waves stage the rows
+// of the Pfaffian ratio meanwhile): LDS operations of one wave complete in
+// order, so its steps are ordered without barriers.
 // ---------------------------------------------------------------------------
+// The measurement's look-up (row a is contiguous: the table is stored in
+// full, the loader checks its symmetry).
 __device__ inline int jast_of(const EnsView& v, int a, int b) {
-  if (a == b) return -1;
-  // the table is stored in full (the loader checks its symmetry), so row a
-  // is contiguous and lanes over b read it coalesced
-  return v.jast_idx[(size_t)a * v.ns + b];
+  return a == b ? -1 : v.jast_idx[(size_t)a * v.ns + b];
 }
 
-__device__ void hop_deltas(const EnsView& v, SampLds& L, int ri, int rj) {
-  const int ns = v.ns;
+__device__ __forceinline__ void add_delta(SampLds& L, int p, int x) {
+  atomicAdd(&L.delta[p], x);
+  if (L.touch) atomicOr(&L.touch[p >> 5], 1u << (p & 31));
+}
+
+// Projection-count deltas of a hop ri -> rj (post-hop occupations) into LDS
+// `delta` (integer adds commute, so lanes add concurrently).
+__device__ __forceinline__ void hop_deltas(const EnsView& v, SampLds& L, int ri, int rj) {
+  const int ns = v.ns, lane = threadIdx.x;
   const int* n0 = L.ele_num;
   const int* n1 = L.ele_num + ns;
   if (ri == rj) return;
-  if (threadIdx.x == 0 && v.ngutz > 0) {
-    int a = L.gutz_idx[ri], b = L.gutz_idx[rj];
-    if (a >= 0) atomicAdd(&L.delta[a], -(n0[ri] + n1[ri]));
-    if (b >= 0) atomicAdd(&L.delta[b], n0[rj] * n1[rj]);
-  }
   if (v.nproj > v.ngutz) {
     const int off = v.ngutz;
-    if (threadIdx.x == 0) {
-      int idx = jast_of(v, ri, rj);
-      if (idx >= 0) atomicAdd(&L.delta[off + idx], (n0[ri] + n1[ri]) - (n0[rj] + n1[rj]) + 1);
+    auto jast = [&](int a, int b) __attribute__((always_inline)) {
+      return L.jast ? (int)L.jast[a * ns + b] : v.jast_idx[(size_t)a * ns + b];
+    };
+    constexpr int U = 4;  // sites per lane whose table loads go out together
+    for (int k0 = 0; k0 < ns; k0 += 64 * U) {
+      int x[U], a[U], b[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int rk = k0 + 64 * u + lane;
+        const bool on = rk < ns && rk != ri && rk != rj;
+        x[u] = on ? n0[rk] + n1[rk] - 1 : 0;
+        a[u] = x[u] != 0 ? jast(ri, rk) : -1;
+        b[u] = x[u] != 0 ? jast(rj, rk) : -1;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (a[u] >= 0) add_delta(L, off + a[u], -x[u]);
+        if (b[u] >= 0) add_delta(L, off + b[u], x[u]);
+      }
     }
-    for (int rk = threadIdx.x; rk < ns; rk += blockDim.x) {
-      if (rk == ri || rk == rj) continue;
-      int x = n0[rk] + n1[rk] - 1;
-      if (x == 0) continue;
-      int a = jast_of(v, ri, rk);
-      if (a >= 0) atomicAdd(&L.delta[off + a], -x);
-      int b = jast_of(v, rj, rk);
-      if (b >= 0) atomicAdd(&L.delta[off + b], x);
+    if (lane == 0) {
+      const int idx = jast(ri, rj);
+      if (idx >= 0) add_delta(L, off + idx, (n0[ri] + n1[ri]) - (n0[rj] + n1[rj]) + 1);
     }
+  }
+  if (lane == 0 && v.ngutz > 0) {
+    const int a = L.gutz_idx[ri], b = L.gutz_idx[rj];
+    if (a >= 0) add_delta(L, a, -(n0[ri] + n1[ri]));
+    if (b >= 0) add_delta(L, b, n0[rj] * n1[rj]);
   }
 }
 
 // The terms of log_proj_ratio, proj[p] * delta[p] over the changed entries
 // in ascending parameter order (zero terms leave a serial sum unchanged),
-// compacted into L.terms; returns their count (all lanes).  The parameter
-// loads of CB entries are issued together.
-__device__ int proj_terms(const EnsView& v, SampLds& L) {
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int np = v.nproj;
-  const int chunk = (np + nt - 1) / nt;
-  const int p0 = tid * chunk, p1 = min(np, p0 + chunk);
-  int cntl = 0;
-  for (int p = p0; p < p1; ++p) cntl += (L.delta[p] != 0);
-  int total;
-  int off = block_exscan(cntl, L.scan, &total);
-  const int cap = 4 * v.ns + 16;
-  if (total > cap) {
-    if (tid == 0) set_status(v.status, ST_BAD_INPUT);
-    total = cap;
-  }
-  constexpr int CB = 8;
-  for (int b = p0; b < p1; b += CB) {
-    int d[CB];
-    double pv[CB];
-#pragma unroll
-    for (int u = 0; u < CB; ++u) d[u] = b + u < p1 ? L.delta[b + u] : 0;
-#pragma unroll
-    for (int u = 0; u < CB; ++u)
-      if (d[u] != 0) pv[u] = v.proj[b + u];
-#pragma unroll
-    for (int u = 0; u < CB; ++u)
-      if (d[u] != 0) {
-        if (off < cap) L.terms[off] = pv[u] * (double)d[u];
-        ++off;
+// compacted into `terms` (cap entries) with their indices in L.tidx; returns their count.
+__device__ __forceinline__ int proj_terms(const EnsView& v, SampLds& L, double* terms, int cap) {
+  const int lane = threadIdx.x, np = v.nproj;
+  const unsigned long long below = (1ull << lane) - 1;
+  int off = 0;
+  constexpr int U = 4;
+  if (L.touch) {
+    // a word of the bitmap per lane: the entries of its bits that did change
+    // counted, placed behind those of the lanes before, and listed
+    for (int w0 = 0; w0 < (np + 31) / 32; w0 += 64) {
+      const int w = w0 + lane;
+      unsigned bits = w < (np + 31) / 32 ? L.touch[w] : 0u;
+      if (bits) L.touch[w] = 0;
+      unsigned left = 0;
+      for (unsigned b = bits; b; b &= b - 1) {
+        const int k = __ffs(b) - 1;
+        if (L.delta[32 * w + k] != 0) left |= 1u << k;
       }
+      int before = __popc(left);
+      for (int h = 1; h < 64; h <<= 1) {
+        const int y = __shfl_up(before, h, 64);
+        if (lane >= h) before += y;
+      }
+      const int total = __shfl(before, 63, 64);
+      int at = off + before - __popc(left);
+      for (unsigned b = left; b; b &= b - 1, ++at)
+        if (at < cap) L.tidx[at] = 32 * w + __ffs(b) - 1;
+      off += total;
+    }
+  } else {
+    for (int b = 0; b < np; b += 64 * U) {
+      int d[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) d[u] = b + 64 * u + lane < np ? L.delta[b + 64 * u + lane] : 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const unsigned long long hit = __ballot(d[u] != 0);
+        if (hit) {
+          const int at = off + __popcll(hit & below);
+          if (d[u] != 0 && at < cap) L.tidx[at] = b + 64 * u + lane;
+          off += __popcll(hit);
+        }
+      }
+    }
   }
-  __syncthreads();
-  return total;
+  if (off > cap) {
+    if (lane == 0) set_status(v.status, ST_BAD_INPUT);
+    off = cap;
+  }
+  wave_sync();
+  for (int k0 = 0; k0 < off; k0 += 64 * U) {
+    double pv[U];
+    int d[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 64 * u + lane;
+      if (k < off) {
+        const int p = L.tidx[k];
+        d[u] = L.delta[p];
+        pv[u] = L.proj ? L.proj[p] : v.proj[p];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + 64 * u + lane < off) terms[k0 + 64 * u + lane] = pv[u] * (double)d[u];
+  }
+  wave_sync();
+  return off;
 }
 
-__device__ inline void apply_clear_deltas(const EnsView& v, SampLds& L, int* cnt, bool apply) {
-  for (int p = threadIdx.x; p < v.nproj; p += blockDim.x) {
-    int d = L.delta[p];
-    if (d != 0) {
-      if (apply) cnt[p] += d;
-      L.delta[p] = 0;
-    }
+// Clears the deltas of the listed entries, adding them to the walker's
+// counts when the move is accepted.
+__device__ __forceinline__ void apply_clear_deltas(SampLds& L, int* cnt, int total, bool apply) {
+  for (int k = threadIdx.x; k < total; k += 64) {
+    const int p = L.tidx[k];
+    if (apply) cnt[p] += L.delta[p];
+    L.delta[p] = 0;
   }
 }
 
@@ -704,52 +795,49 @@ constexpr int BUF_WORD3 = 0x00020000;  // raw untyped buffer (gfx9 family)
 // slower: the walker's inverse is re-read at its next accepted hop).
 constexpr int BUF_NT = 0;
 
-// Storage of the planes seen as 16-byte vectors of EPV elements: FP64
-// (EPV = 2) or FP32, the mixed-precision form (EPV = 4; the rank-2 updates
-// of the stream in FP32, everything else in FP64).  cnt = elements of the
-// vector inside the row (EPV, or 2 for an FP32 vector at the end of a row
-// whose length is 2 mod 4).
-template <class T>
-struct PlaneIO;
-template <>
-struct PlaneIO<double> {
-  static constexpr int EPV = 2;
-  static __device__ inline u32x4_t load(__amdgpu_buffer_rsrc_t r, int voff, int soff, int) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, BUF_NT);
+// A lane's CPL contiguous elements of one plane row, FP64 or FP32 (the
+// mixed-precision form), as vectors of at most 16 bytes; cnt = elements
+// inside the row (even, or CPL = 1).
+template <class T, int CPL>
+struct PlaneIO {
+  static constexpr int ES = (int)sizeof(T), VB = CPL * ES < 16 ? CPL * ES : 16, EPV = VB / ES, NV = CPL / EPV;
+  static __device__ __forceinline__ void load(T (&x)[CPL], __amdgpu_buffer_rsrc_t r, int voff, int soff, int cnt) {
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      if (cnt <= EPV * m) continue;
+      if constexpr (VB == 16) {
+        u32x4_t w;
+        if (ES == 4 && cnt - EPV * m < EPV) {
+          const u32x2_t h = __builtin_amdgcn_raw_buffer_load_b64(r, voff + 16 * m, soff, BUF_NT);
+          w = u32x4_t{h.x, h.y, 0u, 0u};
+        } else {
+          w = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16 * m, soff, BUF_NT);
+        }
+        __builtin_memcpy(&x[EPV * m], &w, 16);
+      } else {
+        const u32x2_t w = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, BUF_NT);
+        __builtin_memcpy(&x[0], &w, 8);
+      }
+    }
   }
-  static __device__ inline void store(u32x4_t x, __amdgpu_buffer_rsrc_t r, int voff, int soff, int) {
-    __builtin_amdgcn_raw_buffer_store_b128(x, r, voff, soff, BUF_NT);
-  }
-  static __device__ inline double get(u32x4_t x, int h) {
-    const double2 d = __builtin_bit_cast(double2, x);
-    return h == 0 ? d.x : d.y;
-  }
-  static __device__ inline void set(u32x4_t& x, int h, double v) {
-    double2 d = __builtin_bit_cast(double2, x);
-    if (h == 0) d.x = v; else d.y = v;
-    x = __builtin_bit_cast(u32x4_t, d);
-  }
-};
-template <>
-struct PlaneIO<float> {
-  static constexpr int EPV = 4;
-  static __device__ inline u32x4_t load(__amdgpu_buffer_rsrc_t r, int voff, int soff, int cnt) {
-    if (cnt == 4) return __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, BUF_NT);
-    const u32x2_t h = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, BUF_NT);
-    u32x4_t x = {h.x, h.y, 0u, 0u};
-    return x;
-  }
-  static __device__ inline void store(u32x4_t x, __amdgpu_buffer_rsrc_t r, int voff, int soff, int cnt) {
-    if (cnt == 4) __builtin_amdgcn_raw_buffer_store_b128(x, r, voff, soff, BUF_NT);
-    else __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{x.x, x.y}, r, voff, soff, BUF_NT);
-  }
-  static __device__ inline float get(u32x4_t x, int h) {
-    const unsigned u = h == 0 ? x.x : h == 1 ? x.y : h == 2 ? x.z : x.w;
-    return __builtin_bit_cast(float, u);
-  }
-  static __device__ inline void set(u32x4_t& x, int h, float v) {
-    const unsigned u = __builtin_bit_cast(unsigned, v);
-    if (h == 0) x.x = u; else if (h == 1) x.y = u; else if (h == 2) x.z = u; else x.w = u;
+  static __device__ __forceinline__ void store(const T (&x)[CPL], __amdgpu_buffer_rsrc_t r, int voff, int soff,
+                                               int cnt) {
+#pragma unroll
+    for (int m = 0; m < NV; ++m) {
+      if (cnt <= EPV * m) continue;
+      if constexpr (VB == 16) {
+        u32x4_t w;
+        __builtin_memcpy(&w, &x[EPV * m], 16);
+        if (ES == 4 && cnt - EPV * m < EPV)
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{w.x, w.y}, r, voff + 16 * m, soff, BUF_NT);
+        else
+          __builtin_amdgcn_raw_buffer_store_b128(w, r, voff + 16 * m, soff, BUF_NT);
+      } else {
+        u32x2_t w;
+        __builtin_memcpy(&w, &x[0], 8);
+        __builtin_amdgcn_raw_buffer_store_b64(w, r, voff, soff, BUF_NT);
+      }
+    }
   }
 };
 
@@ -783,28 +871,23 @@ struct PendList {
   int pm[PEND_MAX];   // their rows
 };
 
-// One streaming pass over a walker's planes.  A lane owns CPL = 2 * EPV
-// contiguous columns of one plane (q = tid / LP; columns
-// LP*CPL*g + CPL*(tid % LP) + c), read and written as two 16-byte vectors
-// per row, and issues the loads of STREAM_ROWS rows before using any of
-// them: each lane keeps STREAM_ROWS rows of its columns in flight, which is
-// what bounds a pass over HBM at this occupancy (the FP32 form therefore
-// covers twice the columns per round trip).  The pending values of a tile's
-// rows (cache hits) are loaded before the next tile's rows, so waiting for
-// them does not wait for that tile.
+// One streaming pass over a walker's planes.  A lane owns CPL contiguous
+// columns of one plane (q = tid / LP; columns LP*CPL*g + CPL*(tid % LP) + c)
+// and issues the loads of ROWS rows before using any of them, a tile of rows
+// ahead of the one in use: the bytes a workgroup keeps in flight are what
+// bounds a pass.  The pending values of a tile's rows (cache hits) are loaded
+// before the next tile's rows, so waiting for them does not wait for that
+// tile.
 //   P.np > 0 : apply the pending updates, in order, in the storage type's
 //              arithmetic; store = write the result back;
 //   ACC      : out[q][j] = sum_i -X[i][j] * b[q][i] in FP64, serial in i
 //              (the update_one_real vec1 = -(X^T b)), X the current inverse;
 //              rows of b and out are ldb doubles apart.
-constexpr int STREAM_ROWS = 4;
-template <bool ACC, class T>
-__device__ void stream_planes(T* planes, int n, int nqp, const typename PendPair<T>::type* pend, const PendList& P,
-                              bool store,
-                              const double* b, double* out, int ldb = 0) {
-  using IO = PlaneIO<T>;
+template <bool ACC, class T, int CPL, int ROWS>
+__device__ __forceinline__ void stream_tiles(T* planes, int n, int nqp, const typename PendPair<T>::type* pend,
+                                             const PendList& P, bool store, const double* b, double* out, int ldb) {
+  using IO = PlaneIO<T, CPL>;
   using PV = typename PendPair<T>::type;
-  constexpr int EPV = IO::EPV, NV = 2, CPL = NV * EPV;
   constexpr int ES = (int)sizeof(T);
   const int nt = blockDim.x, tid = threadIdx.x;
   const int nn = n * n;
@@ -812,6 +895,8 @@ __device__ void stream_planes(T* planes, int n, int nqp, const typename PendPair
   const int LP = nt / PG;
   const int qo = tid / LP, jl = tid % LP;
   const int span = LP * CPL;  // columns per group
+  // rows past the end of a plane are loaded (from the next plane, or 0 past
+  // the last by the buffer's range) and not used
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(planes, 0, (int)((size_t)nqp * nn * ES), BUF_WORD3);
   const int rowb = n * ES;
@@ -823,95 +908,87 @@ __device__ void stream_planes(T* planes, int n, int nqp, const typename PendPair
     const PV* pq = pend + (size_t)(on ? q : 0) * n * PEND_MAX;
     const double* bq = b + (on ? q : 0) * ldb;
     for (int g0 = 0; g0 < n; g0 += span) {
-      const int jb = g0 + CPL * jl;  // first column of the lane
-      int cnt[NV];                   // elements of vector m inside the row
+      const int jb = g0 + CPL * jl;                             // first column of the lane
+      const int cnt = on ? max(0, min(CPL, n - jb)) : 0;  // its columns inside the row
       double acc[CPL];
       T c1[PEND_MAX][CPL], c2[PEND_MAX][CPL];
 #pragma unroll
-      for (int m = 0; m < NV; ++m) cnt[m] = on ? max(0, min(EPV, n - (jb + EPV * m))) : 0;
-#pragma unroll
       for (int c = 0; c < CPL; ++c) {
-        const bool in = c % EPV < cnt[c / EPV];
         acc[c] = 0.0;
 #pragma unroll
         for (int k = 0; k < PEND_MAX; ++k) {
           PV d = {0, 0};
-          if (k < np && in) d = pq[(jb + c) * PEND_MAX + k];
+          if (k < np && c < cnt) d = pq[(jb + c) * PEND_MAX + k];
           c1[k][c] = (T)d.x;
           c2[k][c] = (T)d.y;
         }
       }
       const int vbase = qoff + jb * ES;
-      // Two tiles of plane rows in flight: the loads of tile i0 +
-      // STREAM_ROWS are issued before tile i0 is updated and stored (a load
-      // after a buffer store could not be moved above it by the compiler).
-      u32x4_t x[STREAM_ROWS][NV], xn[STREAM_ROWS][NV];
-      auto load_tile = [&](int i0, u32x4_t (&tx)[STREAM_ROWS][NV]) {
+      T x[ROWS][CPL], xn[ROWS][CPL];
+      auto load_tile = [&](int i0, T (&tx)[ROWS][CPL]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < STREAM_ROWS; ++r)
-          if (i0 + r < n) {
-#pragma unroll
-            for (int m = 0; m < NV; ++m)
-              if (cnt[m] > 0) tx[r][m] = IO::load(rs, vbase + 16 * m, (i0 + r) * rowb, cnt[m]);
-          }
+        for (int r = 0; r < ROWS; ++r) IO::load(tx[r], rs, vbase, (i0 + r) * rowb, cnt);
       };
       load_tile(0, x);
-      for (int i0 = 0; i0 < n; i0 += STREAM_ROWS) {
-        PV pr[STREAM_ROWS][PEND_MAX];
-        double rsv[STREAM_ROWS];
+      for (int i0 = 0; i0 < n; i0 += ROWS) {
+        PV pr[ROWS][PEND_MAX];
+        double rsv[ROWS];
 #pragma unroll
-        for (int r = 0; r < STREAM_ROWS; ++r)
-          if (i0 + r < n) {
+        for (int r = 0; r < ROWS; ++r) {
+          const int i = min(i0 + r, n - 1);
 #pragma unroll
-            for (int k = 0; k < PEND_MAX; ++k)
-              if (k < np) pr[r][k] = pq[(i0 + r) * PEND_MAX + k];
-            if (ACC) rsv[r] = bq[i0 + r];
-          }
-        if (i0 + STREAM_ROWS < n) load_tile(i0 + STREAM_ROWS, xn);
+          for (int k = 0; k < PEND_MAX; ++k)
+            if (k < np) pr[r][k] = pq[i * PEND_MAX + k];
+          if (ACC) rsv[r] = bq[i];
+        }
+        if (i0 + ROWS < n) load_tile(i0 + ROWS, xn);
 #pragma unroll
-        for (int r = 0; r < STREAM_ROWS; ++r) {
+        for (int r = 0; r < ROWS; ++r) {
           const int i = i0 + r;
           if (i < n) {
-            if (np > 0) {
+            if (np > 0 && cnt > 0) {
 #pragma unroll
-              for (int m = 0; m < NV; ++m)
-                if (cnt[m] > 0) {
+              for (int c = 0; c < CPL; ++c)
 #pragma unroll
-                  for (int h = 0; h < EPV; ++h)
-                    if (h < cnt[m]) {
-                      T e = IO::get(x[r][m], h);
-#pragma unroll
-                      for (int k = 0; k < PEND_MAX; ++k)
-                        if (k < np)
-                          e = apply_pend(e, (T)pr[r][k].x, (T)pr[r][k].y, c1[k][EPV * m + h], c2[k][EPV * m + h], i,
-                                         jb + EPV * m + h, P.pm[k]);
-                      IO::set(x[r][m], h, e);
-                    }
-                  if (store) IO::store(x[r][m], rs, vbase + 16 * m, i * rowb, cnt[m]);
-                }
+                for (int k = 0; k < PEND_MAX; ++k)
+                  if (k < np)
+                    x[r][c] = apply_pend(x[r][c], (T)pr[r][k].x, (T)pr[r][k].y, c1[k][c], c2[k][c], i, jb + c, P.pm[k]);
+              if (store) IO::store(x[r], rs, vbase, i * rowb, cnt);
             }
             if (ACC) {
               const double s0 = rsv[r];
 #pragma unroll
-              for (int m = 0; m < NV; ++m)
-#pragma unroll
-                for (int h = 0; h < EPV; ++h)
-                  if (h < cnt[m]) acc[EPV * m + h] += -(double)IO::get(x[r][m], h) * s0;
+              for (int c = 0; c < CPL; ++c)
+                if (c < cnt) acc[c] += -(double)x[r][c] * s0;
             }
           }
         }
 #pragma unroll
-        for (int r = 0; r < STREAM_ROWS; ++r)
+        for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-          for (int m = 0; m < NV; ++m) x[r][m] = xn[r][m];
+          for (int c = 0; c < CPL; ++c) x[r][c] = xn[r][c];
       }
       if (ACC) {
 #pragma unroll
         for (int c = 0; c < CPL; ++c)
-          if (c % EPV < cnt[c / EPV]) out[q * ldb + jb + c] = acc[c];
+          if (c < cnt) out[q * ldb + jb + c] = acc[c];
       }
     }
   }
+}
+
+// The pass with as few columns per lane as cover a row in one group of
+// lanes: small planes then use every lane, with more rows in flight, instead
+// of a quarter of them with four or eight columns each (8 planes of n = 64 in
+// FP32: 92.8 -> 19 us a pass at 512 workgroups).
+template <bool ACC, class T>
+__device__ void stream_planes(T* planes, int n, int nqp, const typename PendPair<T>::type* pend, const PendList& P,
+                              bool store, const double* b, double* out, int ldb = 0) {
+  const int LP = (int)blockDim.x / min(nqp, (int)blockDim.x);
+  constexpr int W = 8 / (int)sizeof(T);  // columns in 8 bytes
+  if (n <= LP * W) stream_tiles<ACC, T, W, 8>(planes, n, nqp, pend, P, store, b, out, ldb);
+  else if (ACC && n <= LP * 2 * W) stream_tiles<ACC, T, 2 * W, 4>(planes, n, nqp, pend, P, store, b, out, ldb);
+  else stream_tiles<ACC, T, 4 * W, 4>(planes, n, nqp, pend, P, store, b, out, ldb);
 }
 
 // Apply every pending update to the stored planes and empty the list;
@@ -951,8 +1028,88 @@ __device__ inline void flush_pending(T* planes, int n, int nqp, const typename P
   } while (0)
 #endif
 
-enum { M_TYPE = 0, M_REJ, M_MI, M_S, M_RI, M_RJ, M_MJ, M_T, M_ACC, M_NACC, M_NOUT, M_SKIP, M_RES, M_DONE };
+enum { M_TYPE = 0, M_STEP, M_MI, M_S, M_RI, M_RJ, M_MJ, M_T, M_ACC, M_NACC, M_NOUT, M_SKIP, M_RES, M_DONE };
 
+// The next candidate from proposal `step` on (lane 0; candidate.rs:137-385),
+// its move applied to the configuration (the first hop of an exchange); the
+// proposals that find none are passed over.  M_STEP = n_in: none left.
+__device__ __forceinline__ void draw_candidate(const EnsView& v, SampLds& L, int step, int n_in, long long* ctr) {
+  const int ns = v.ns, ne = v.ne;
+  SfmtLds& R = *L.rng;
+  for (; step < n_in; ++step) {
+    int type = v.ex_path == 2 ? 1 : 0;
+    if (v.ex_path == 1) type = sfmt_real2(R) < 0.5 ? 1 : 0;
+    bool none = false;
+    int mi = 0, s = 0, ri = 0, rj = 0, mj = 0, t = 0;
+    if (type == 0) {
+      ctr[0]++;
+      const long long icnt_max = (long long)ns * ns;
+      long long icnt_e = 0;
+      for (;;) {
+        if (icnt_e == icnt_max + 1) {
+          bool any = false;
+          for (int k = 0; k < 2 * ne; ++k) {
+            int r = L.ele_idx[k] < 0 ? 0 : L.ele_idx[k];
+            any = any || !(r >= ns || L.loc_spn[r] == 1);
+          }
+          if (!any) { none = true; break; }
+        }
+        ++icnt_e;
+        mi = (int)sfmt_mod(R, (uint32_t)ne);
+        s = sfmt_real2(R) < 0.5 ? 0 : 1;
+        ri = L.ele_idx[mi + s * ne];
+        if (!(ri < 0 || ri >= ns || L.loc_spn[ri] == 1)) break;
+      }
+      if (!none) {
+        long long icnt = 0;
+        for (;;) {
+          rj = (int)sfmt_mod(R, (uint32_t)ns);
+          if (icnt > icnt_max) { none = true; break; }
+          ++icnt;
+          if (L.ele_cfg[rj + s * ns] == -1 && L.loc_spn[rj] != 1) break;
+        }
+      }
+    } else {
+      ctr[2]++;
+      bool single = false;
+      for (int r = 0; r < ns; ++r)
+        if (L.ele_num[r] + L.ele_num[r + ns] == 1) { single = true; break; }
+      none = !single;
+      if (single) {
+        for (;;) {
+          mi = (int)sfmt_mod(R, (uint32_t)ne);
+          s = sfmt_real2(R) < 0.5 ? 0 : 1;
+          ri = L.ele_idx[mi + s * ne];
+          if (L.ele_cfg[ri + (1 - s) * ns] == -1) break;
+        }
+        t = 1 - s;
+        for (;;) {
+          mj = (int)sfmt_mod(R, (uint32_t)ne);
+          rj = L.ele_idx[mj + t * ne];
+          if (L.ele_cfg[rj + s * ns] == -1) break;
+        }
+      }
+    }
+    if (none) continue;  // the reference's `continue` skips the recompute guard too
+    // update_ele_config (mi: ri -> rj, spin s)
+    L.ele_idx[mi + s * ne] = rj;
+    L.ele_cfg[ri + s * ns] = -1;
+    L.ele_cfg[rj + s * ns] = mi;
+    L.ele_num[ri + s * ns] = 0;
+    L.ele_num[rj + s * ns] = 1;
+    L.misc[M_TYPE] = type;
+    L.misc[M_MI] = mi; L.misc[M_S] = s; L.misc[M_RI] = ri; L.misc[M_RJ] = rj;
+    L.misc[M_MJ] = mj; L.misc[M_T] = t;
+    break;
+  }
+  L.misc[M_STEP] = step;
+}
+
+// A proposal is three barrier intervals (an accepted one adds its pass):
+//   wave 0 forms the projection deltas and terms and half of their serial
+//   sum, the other waves load the inverse and Slater rows | the other half,
+//   the ratio dots (a lane per QP plane) | lane 0 decides, and on a
+//   rejection draws the next candidate at once.
 // Elem: storage type of the sampler's inverse (double; float in the
 // mixed-precision form, whose arithmetic stays FP64).
 // In a group launch (GROUP) the workgroups take entries of the group's
@@ -988,6 +1145,7 @@ __global__ void __launch_bounds__(256, 2) k_block(EnsView v_arg, GroupArgs ga, i
   int* const wpasses = GROUP ? nullptr : v_arg.nflag + 3;
   PHASE_INIT
   __shared__ int next_w;
+  __shared__ long long ctr_l[4];  // the walker's proposal / acceptance counters (lane 0)
   for (;;) {
     // walkers are taken dynamically, so the launch ends when the work does
     // (a walker's results do not depend on the slot that runs it: the
@@ -1034,104 +1192,191 @@ __global__ void __launch_bounds__(256, 2) k_block(EnsView v_arg, GroupArgs ga, i
     for (int q = tid; q < nqp; q += nt) L.pf[q] = v.pf[(size_t)w * nqp + q];
     __syncthreads();
     int stop_at = -1;  // proposal index to resume at after a rebuild
-    for (int step = resume; step < n_in; ++step) {
-      // ---- candidate (lane 0) ----
-      if (tid == 0) {
-        SfmtLds& R = *L.rng;
-        int type;
-        switch (v.ex_path) {
-          case 0: type = 0; break;
-          case 1: type = sfmt_real2(R) < 0.5 ? 1 : 0; break;
-          case 2: type = 1; break;
-          default: type = 3;
-        }
-        int rej = 0, mi = 0, s = 0, ri = 0, rj = 0, mj = 0, t = 0;
-        if (type == 0) {
-          ctr[0]++;
-          const long long icnt_max = (long long)ns * ns;
-          long long icnt_e = 0;
-          for (;;) {
-            if (icnt_e == icnt_max + 1) {
-              bool any = false;
-              for (int k = 0; k < 2 * ne; ++k) {
-                int r = L.ele_idx[k] < 0 ? 0 : L.ele_idx[k];
-                any = any || !(r >= ns || L.loc_spn[r] == 1);
+    if (tid == 0)
+      for (int k = 0; k < 4; ++k) ctr_l[k] = ctr[k];
+    // Each turn decides the proposal of the turn before (open), draws the
+    // next candidate unless it was accepted, and forms its ratio.
+    bool open = false;
+    int next = resume;
+    int type = 0, mi = 0, s = 0, ri = 0, rj = 0, mj = 0, t = 0;
+    int nterms = 0;     // wave 0's: changed projection parameters of the proposal
+    double lsum = 0.0;  // lane 0's: their sum
+    // Rows of the hop staging arrays are hop_ld(n) (odd) doubles apart, so
+    // the ratio dots' lanes (one per QP plane, same k) read distinct LDS
+    // banks.
+    const int ld = hop_ld(n);
+    double* stage = L.uni;              // [nqp][ld]
+    double* slt = L.uni + nqp * ld;     // [nqp][ld]
+    double* vec1 = L.uni + 2 * nqp * ld;
+    for (;;) {
+      if (tid < 64) {
+        int acc = 0;
+        if (open) {
+          // ---- Metropolis (lane 0); wave 0 settles the deltas ----
+          if (tid == 0) {
+            const double lpd = lsum;
+            const double lip_new = ddm::cr_log(fabs(ip_of_l(L.qpw, L.pf_new, nqp)));
+            const double ex = 2.0 * (((lpd + 0.0) + lip_new) - L.dmisc[1]);
+            double wgt = ddm::cr_exp(ex);
+            if (!(wgt - wgt == 0.0)) wgt = -1.0;
+            const double u = sfmt_real2(*L.rng);
+            acc = wgt > u;
+            L.misc[M_ACC] = acc;
+            if (acc) {
+              L.dmisc[1] = lip_new;
+              L.misc[M_NACC] += 1;
+              ctr_l[type == 0 ? 1 : 3]++;
+            } else {
+              if (type == 1) {
+                L.ele_idx[mj + t * ne] = rj;
+                L.ele_cfg[ri + t * ns] = -1;
+                L.ele_cfg[rj + t * ns] = mj;
+                L.ele_num[ri + t * ns] = 0;
+                L.ele_num[rj + t * ns] = 1;
               }
-              if (!any) { rej = 1; break; }
-            }
-            ++icnt_e;
-            mi = (int)sfmt_mod(R, (uint32_t)ne);
-            s = sfmt_real2(R) < 0.5 ? 0 : 1;
-            ri = L.ele_idx[mi + s * ne];
-            if (!(ri < 0 || ri >= ns || L.loc_spn[ri] == 1)) break;
-          }
-          if (!rej) {
-            long long icnt = 0;
-            for (;;) {
-              rj = (int)sfmt_mod(R, (uint32_t)ns);
-              if (icnt > icnt_max) { rej = 1; break; }
-              ++icnt;
-              if (L.ele_cfg[rj + s * ns] == -1 && L.loc_spn[rj] != 1) break;
+              L.ele_idx[mi + s * ne] = ri;
+              L.ele_cfg[ri + s * ns] = mi;
+              L.ele_cfg[rj + s * ns] = -1;
+              L.ele_num[ri + s * ns] = 1;
+              L.ele_num[rj + s * ns] = 0;
             }
           }
-          if (!rej) {
-            // update_ele_config
-            L.ele_idx[mi + s * ne] = rj;
-            L.ele_cfg[ri + s * ns] = -1;
-            L.ele_cfg[rj + s * ns] = mi;
-            L.ele_num[ri + s * ns] = 0;
-            L.ele_num[rj + s * ns] = 1;
-          }
-        } else if (type == 1) {
-          ctr[2]++;
-          bool single = false;
-          for (int r = 0; r < ns; ++r)
-            if (L.ele_num[r] + L.ele_num[r + ns] == 1) { single = true; break; }
-          if (!single) rej = 1;
-          else {
-            for (;;) {
-              mi = (int)sfmt_mod(R, (uint32_t)ne);
-              s = sfmt_real2(R) < 0.5 ? 0 : 1;
-              ri = L.ele_idx[mi + s * ne];
-              if (L.ele_cfg[ri + (1 - s) * ns] == -1) break;
-            }
-            t = 1 - s;
-            for (;;) {
-              mj = (int)sfmt_mod(R, (uint32_t)ne);
-              rj = L.ele_idx[mj + t * ne];
-              if (L.ele_cfg[rj + s * ns] == -1) break;
-            }
-            // first hop (mi: ri -> rj, spin s)
-            L.ele_idx[mi + s * ne] = rj;
-            L.ele_cfg[ri + s * ns] = -1;
-            L.ele_cfg[rj + s * ns] = mi;
-            L.ele_num[ri + s * ns] = 0;
-            L.ele_num[rj + s * ns] = 1;
-          }
-        } else {
-          rej = 2;  // no update: still runs the recompute guard
+          acc = __builtin_amdgcn_readfirstlane(acc);
+          apply_clear_deltas(L, cnt, nterms, acc != 0);
         }
-        L.misc[M_TYPE] = type;
-        L.misc[M_REJ] = rej;
-        L.misc[M_MI] = mi; L.misc[M_S] = s; L.misc[M_RI] = ri; L.misc[M_RJ] = rj;
-        L.misc[M_MJ] = mj; L.misc[M_T] = t;
+        if (tid == 0) {
+          L.misc[M_ACC] = acc;
+          if (!acc) draw_candidate(v, L, next, n_in, ctr_l);
+        }
       }
       __syncthreads();
-      PHASE(0);
-      const int rej = L.misc[M_REJ], type = L.misc[M_TYPE];
-      if (rej == 1) {
-        // `continue` in the reference skips the recompute guard too; the
-        // barrier keeps lane 0 from overwriting the candidate fields before
-        // every wave has read them.
-        __syncthreads();
+      PHASE(open ? 4 : 0);
+      const bool accepted = open && L.misc[M_ACC];
+      open = false;
+      if (accepted) {
+        if (type == 0) {
+          // update_one_real_scalar (updates.rs:1184-1224), delayed: one
+          // pass forms vec1 = -(X^T slt) of this update from the current
+          // inverse (pending updates applied in registers), writing the
+          // planes back only when the pending list is full; this update
+          // joins the list.
+          const int msa = mi + s * ne;
+          const bool full = P.np == PEND_MAX;
+          stream_planes<true>(planes, n, nqp, pend_c, P, full, slt, vec1, ld);
+          if (full && wpasses && tid == 0) atomicAdd(wpasses, 1);
+          __syncthreads();
+          if (full) P.np = 0;
+          const int k = P.np;
+          for (int e = tid; e < nqp * n; e += nt) {
+            const int q = e / n;
+            const int j = e - q * n;
+            const double inv_a = -1.0 / vec1[q * ld + msa];
+            pend[(size_t)e * PEND_MAX + k] = PendPair<Elem>::make(vec1[q * ld + j], stage[q * ld + j] * inv_a);
+          }
+  #pragma unroll
+          for (int kk = 0; kk < PEND_MAX; ++kk)
+            if (kk == k) P.pm[kk] = msa;
+          P.np = k + 1;
+          for (int q = tid; q < nqp; q += nt) L.pf[q] = L.pf_new[q];
+          __syncthreads();
+          PHASE(5);
+        } else {
+          // update_two_real (updates.rs:1429-1503); pf *= ratio recomputed here
+          const int msa = mi + s * ne, msb = mj + t * ne;
+          const int rsa = L.ele_idx[msa] + s * ns, rsb = L.ele_idx[msb] + t * ns;
+          const int rsa_old = ri + s * ns, rsb_old = rj + t * ns;
+          double* P = L.uni;
+          double* Q = L.uni + nqp * n;
+          double* Sv = L.uni + 2 * nqp * n;
+          double* T = L.uni + 3 * nqp * n;
+          double* cf = L.uni + 5 * nqp * n;  // [nqp][16]
+          for (int e = tid; e < nqp * n; e += nt) {
+            const int q = e / n, i = e % n;
+            const int rsi = L.ele_idx[i] + (i < ne ? 0 : ns);
+            const double* S = v.slater + (size_t)q * n2 * n2;
+            Sv[e] = (i == msb) ? S[(size_t)rsa_old * n2 + rsb_old] : S[(size_t)rsa * n2 + rsi];
+            T[e] = S[(size_t)rsb * n2 + rsi];
+          }
+          __syncthreads();
+          for (int e = tid; e < nqp * n; e += nt) {
+            const int q = e / n, i = e % n;
+            const Elem* row = planes + (size_t)q * nn + (size_t)i * n;
+            double p = 0.0, qq = 0.0;
+            for (int j = 0; j < n; ++j) {
+              const double x = row[j];
+              p += x * Sv[q * n + j];
+              qq += x * T[q * n + j];
+            }
+            P[e] = p;
+            Q[e] = qq;
+          }
+          __syncthreads();
+          for (int q = tid; q < nqp; q += nt) {
+            const double* Pq = P + q * n;
+            const double* Qq = Q + q * n;
+            const double* Tq = T + q * n;
+            double bma = 0.0;
+            for (int i = 0; i < n; ++i) bma += Tq[i] * Pq[i];
+            const double iab = planes[(size_t)q * nn + (size_t)msa * n + msb];
+            const double ratio = iab * Tq[msa] + iab * bma + Pq[msa] * Qq[msb] - Pq[msb] * Qq[msa];
+            L.pf[q] *= ratio;
+            const double a = -Pq[msa], b = Pq[msb], c = Qq[msa], d = -Qq[msb];
+            const double ee = -bma - Tq[msa];
+            const double f = iab;
+            const double det = a * d - b * c - ee * f;
+            double* k = cf + q * 16;
+            k[0] = a; k[1] = b; k[2] = c; k[3] = d; k[4] = ee; k[5] = f; k[6] = det; k[7] = 1.0 / det;
+          }
+          __syncthreads();
+          for (int e = tid; e < nqp * n; e += nt) {  // S, T rows of the old inverse, scaled
+            const int q = e / n, i = e % n;
+            const double idet = cf[q * 16 + 7];
+            const double sa = planes[(size_t)q * nn + (size_t)msa * n + i];
+            const double sb = planes[(size_t)q * nn + (size_t)msb * n + i];
+            Sv[e] = idet * sa;
+            T[e] = idet * sb;
+          }
+          __syncthreads();
+          for (size_t e = tid; e < (size_t)nqp * nn; e += nt) {
+            const int q = (int)(e / nn), r = (int)(e % nn);
+            const int i = r / n, j = r % n;
+            const double* k = cf + q * 16;
+            const double a = k[0], b = k[1], c = k[2], d = k[3], ee = k[4], f = k[5], det = k[6], idet = k[7];
+            const double pi = P[q * n + i], qi = Q[q * n + i], si = Sv[q * n + i], ti = T[q * n + i];
+            const double pj = P[q * n + j], qj = Q[q * n + j], sj = Sv[q * n + j], tj = T[q * n + j];
+            double x = planes[e];
+            x += a * (qi * tj - qj * ti) + b * (qi * sj - qj * si) + c * (pi * tj - pj * ti) +
+                 d * (pi * sj - pj * si) + ee * det * (si * tj - sj * ti) + f * idet * (pi * qj - qi * pj);
+            if (j == msa) x += -c * ti - d * si - f * idet * qi;
+            if (j == msb) x += -a * ti - b * si + f * idet * pi;
+            if (i == msa) x += c * tj + d * sj + f * idet * qj;
+            if (i == msb) x += a * tj + b * sj - f * idet * pj;
+            if (i == msa && j == msb) x += f * idet;
+            if (i == msb && j == msa) x -= f * idet;
+            planes[e] = static_cast<Elem>(x);
+          }
+          __syncthreads();
+        }
+        // ---- periodic recompute (engine.rs:454-473): handed to the rebuild ----
+        if (L.misc[M_NACC] > ns) {
+          stop_at = next;
+          break;
+        }
         continue;
       }
-      if (rej == 0) {
-        const int mi = L.misc[M_MI], s = L.misc[M_S], ri = L.misc[M_RI], rj = L.misc[M_RJ];
-        const int mj = L.misc[M_MJ], t = L.misc[M_T];
+      const int step = L.misc[M_STEP];
+      if (step >= n_in) break;
+      next = step + 1;
+      open = true;
+      type = L.misc[M_TYPE];
+      mi = L.misc[M_MI]; s = L.misc[M_S]; ri = L.misc[M_RI]; rj = L.misc[M_RJ];
+      mj = L.misc[M_MJ]; t = L.misc[M_T];
+      nterms = 0;
+      lsum = 0.0;
+      if (tid < 64) {
         hop_deltas(v, L, ri, rj);
-        __syncthreads();
         if (type == 1) {
+          wave_sync();
           if (tid == 0) {  // second hop (mj: rj -> ri, spin t)
             L.ele_idx[mj + t * ne] = ri;
             L.ele_cfg[rj + t * ns] = -1;
@@ -1139,279 +1384,125 @@ __global__ void __launch_bounds__(256, 2) k_block(EnsView v_arg, GroupArgs ga, i
             L.ele_num[rj + t * ns] = 0;
             L.ele_num[ri + t * ns] = 1;
           }
-          __syncthreads();
+          wave_sync();
           hop_deltas(v, L, rj, ri);
-          __syncthreads();
         }
-        const int nterms = proj_terms(v, L);
-        PHASE(1);
-        // ---- Pfaffian ratios ----
-        // The projection sum is one serial chain: on the hop path lane 0 of
-        // wave 0 forms it (in two parts, carried in a register) while the
-        // other waves stage the rows and form the Pfaffian-ratio dots.
-        // Rows of the hop staging arrays are hop_ld(n) (odd) doubles apart,
-        // so the ratio dots' lanes (one per QP plane, same k) read distinct
-        // LDS banks.
-        const int ld = hop_ld(n);
-        double* stage = L.uni;              // [nqp][ld]
-        double* slt = L.uni + nqp * ld;     // [nqp][ld]
-        double* vec1 = L.uni + 2 * nqp * ld;
-        if (type == 0) {
-          const int msa = mi + s * ne;
-          const int rsa = L.ele_idx[msa] + s * ns;
-          const int ksplit = nterms / 2;
-          double lsum = 0.0;
-          if (tid == 0) lsum = lds_serial_sum(L.terms, 0, ksplit, 0.0);
-          // row msa of the current inverse (stored row + pending updates)
-          // and the Slater row (waves 1..), loads of STAGE_U elements per
-          // lane issued together
-          constexpr int STAGE_U = 4;
-          const int st_id = tid - 64, st_n = nt - 64;
-          const int np = P.np;
-          for (int e0 = 0; e0 < nqp * n && tid >= 64; e0 += st_n * STAGE_U) {
-            double xv[STAGE_U], sv[STAGE_U];
-            PV pj[STAGE_U][PEND_MAX];
+        wave_sync();
+        double* terms = type == 0 ? L.terms : L.uni;
+        nterms = proj_terms(v, L, terms, type == 0 ? hop_cap(v) : term_cap(v));
+        if (tid == 0) lsum = lds_serial_sum(terms, 0, type == 0 ? nterms / 2 : nterms, 0.0);
+      } else if (type == 0) {
+        const int msa = mi + s * ne;
+        const int rsa = L.ele_idx[msa] + s * ns;
+        // row msa of the current inverse (stored row + pending updates)
+        // and the Slater row (waves 1..), loads of STAGE_U elements per
+        // lane issued together
+        constexpr int STAGE_U = 2;
+        const int st_id = tid - 64, st_n = nt - 64;
+        const int np = P.np;
+        for (int e0 = 0; e0 < nqp * n; e0 += st_n * STAGE_U) {
+          double xv[STAGE_U], sv[STAGE_U];
+          PV pj[STAGE_U][PEND_MAX], pi[STAGE_U][PEND_MAX];
 #pragma unroll
-            for (int u = 0; u < STAGE_U; ++u) {
-              const int e = e0 + st_id + u * st_n;
-              if (e < nqp * n) {
-                const int q = e / n, j = e % n;
-                xv[u] = planes[(size_t)q * nn + (size_t)msa * n + j];
-                const int rsj = L.ele_idx[j] + (j < ne ? 0 : ns);
-                sv[u] = v.slater[((size_t)q * n2 + rsa) * n2 + rsj];
+          for (int u = 0; u < STAGE_U; ++u) {
+            const int e = e0 + st_id + u * st_n;
+            if (e < nqp * n) {
+              const int q = e / n, j = e % n;
+              xv[u] = planes[(size_t)q * nn + (size_t)msa * n + j];
+              const int rsj = L.ele_idx[j] + (j < ne ? 0 : ns);
+              sv[u] = v.slater[((size_t)q * n2 + rsa) * n2 + rsj];
 #pragma unroll
-                for (int k = 0; k < PEND_MAX; ++k)
-                  if (k < np) pj[u][k] = pend_c[(size_t)e * PEND_MAX + k];
-              }
-            }
-#pragma unroll
-            for (int u = 0; u < STAGE_U; ++u) {
-              const int e = e0 + st_id + u * st_n;
-              if (e < nqp * n) {
-                const int q = e / n, j = e % n;
-                double x = xv[u];
-#pragma unroll
-                for (int k = 0; k < PEND_MAX; ++k)
-                  if (k < np) {
-                    const PV pi = pend_c[((size_t)q * n + msa) * PEND_MAX + k];
-                    x = apply_pend<double>(x, pi.x, pi.y, pj[u][k].x, pj[u][k].y, msa, j, P.pm[k]);
-                  }
-                stage[q * ld + j] = x;
-                slt[q * ld + j] = sv[u];
-              }
+              for (int k = 0; k < PEND_MAX; ++k)
+                if (k < np) {
+                  pj[u][k] = pend_c[(size_t)e * PEND_MAX + k];
+                  pi[u][k] = pend_c[((size_t)q * n + msa) * PEND_MAX + k];
+                }
             }
           }
-          __syncthreads();
-          PHASE(2);
-          if (tid == 0) L.dmisc[0] = lds_serial_sum(L.terms, ksplit, nterms, lsum);
-          for (int q = tid - 64; q < nqp && tid >= 64; q += nt - 64) {
+#pragma unroll
+          for (int u = 0; u < STAGE_U; ++u) {
+            const int e = e0 + st_id + u * st_n;
+            if (e < nqp * n) {
+              const int q = e / n, j = e % n;
+              double x = xv[u];
+#pragma unroll
+              for (int k = 0; k < PEND_MAX; ++k)
+                if (k < np)
+                  x = apply_pend<double>(x, pi[u][k].x, pi[u][k].y, pj[u][k].x, pj[u][k].y, msa, j, P.pm[k]);
+              stage[q * ld + j] = x;
+              slt[q * ld + j] = sv[u];
+            }
+          }
+        }
+      }
+      __syncthreads();
+      PHASE(2);
+      if (type == 0) {
+        if (tid < 64) {
+          if (tid == 0) lsum = lds_serial_sum(L.terms, nterms / 2, nterms, lsum);
+        } else {
+          for (int q = tid - 64; q < nqp; q += nt - 64) {
             const double ratio = lds_serial_dot(stage + q * ld, slt + q * ld, n);
             L.pf_new[q] = -ratio * L.pf[q];
           }
-        } else {
-          if (tid == 0) L.dmisc[0] = lds_serial_sum(L.terms, 0, nterms, 0.0);
-          // two-electron ratio (updates.rs:395-441, 1539-1622) on the
-          // fully updated inverse
-          if (P.np > 0) {
-            flush_pending(planes, n, nqp, pend_c, P, wpasses);
-            __syncthreads();
-          }
-          const int msa = mi + s * ne, msb = mj + t * ne;
-          double* va = L.uni;                 // [nqp][n]
-          double* vb = L.uni + nqp * n;
-          double* ia = L.uni + 2 * nqp * n;   // inv row msa
-          double* ib = L.uni + 3 * nqp * n;   // inv row msb
-          double* tmp = L.uni + 4 * nqp * n;  // row dots of the bilinear form
-          const int rsa = L.ele_idx[msa] + s * ns, rsb = L.ele_idx[msb] + t * ns;
-          for (int e = tid; e < nqp * n; e += nt) {
-            const int q = e / n, i = e % n;
-            const int rsi = L.ele_idx[i] + (i < ne ? 0 : ns);
-            const double* S = v.slater + (size_t)q * n2 * n2;
-            va[e] = S[(size_t)rsa * n2 + rsi];
-            vb[e] = S[(size_t)rsb * n2 + rsi];
-            ia[e] = planes[(size_t)q * nn + (size_t)msa * n + i];
-            ib[e] = planes[(size_t)q * nn + (size_t)msb * n + i];
-          }
+        }
+      } else {
+        // two-electron ratio (updates.rs:395-441, 1539-1622) on the fully
+        // updated inverse
+        if (P.np > 0) {
+          flush_pending(planes, n, nqp, pend_c, P, wpasses);
           __syncthreads();
-          for (int e = tid; e < nqp * n; e += nt) {
-            const int q = e / n, i = e % n;
-            const Elem* row = planes + (size_t)q * nn + (size_t)i * n;
-            const double* a = va + q * n;
-            double acc = 0.0;
-            for (int j = 0; j < n; ++j) acc += row[j] * a[j];
-            tmp[e] = acc;
-          }
-          __syncthreads();
-          for (int q = tid; q < nqp; q += nt) {
-            const double* a = va + q * n;
-            const double* b = vb + q * n;
-            const double* ra = ia + q * n;
-            const double* rb = ib + q * n;
-            double pa = 0.0, pb = 0.0, qa = 0.0, qb = 0.0;
-            for (int i = 0; i < n; ++i) {
-              pa += ra[i] * a[i];
-              pb += rb[i] * a[i];
-              qa += ra[i] * b[i];
-              qb += rb[i] * b[i];
-            }
-            const double iab = ra[msb];
-            double bma = 0.0;
-            for (int i = 0; i < n; ++i) bma += b[i] * tmp[q * n + i];
-            const double ratio = iab * b[msa] + iab * bma + pa * qb - pb * qa;
-            L.pf_new[q] = ratio * L.pf[q];
-          }
+        }
+        const int msa = mi + s * ne, msb = mj + t * ne;
+        double* va = L.uni;                 // [nqp][n]
+        double* vb = L.uni + nqp * n;
+        double* ia = L.uni + 2 * nqp * n;   // inv row msa
+        double* ib = L.uni + 3 * nqp * n;   // inv row msb
+        double* tmp = L.uni + 4 * nqp * n;  // row dots of the bilinear form
+        const int rsa = L.ele_idx[msa] + s * ns, rsb = L.ele_idx[msb] + t * ns;
+        for (int e = tid; e < nqp * n; e += nt) {
+          const int q = e / n, i = e % n;
+          const int rsi = L.ele_idx[i] + (i < ne ? 0 : ns);
+          const double* S = v.slater + (size_t)q * n2 * n2;
+          va[e] = S[(size_t)rsa * n2 + rsi];
+          vb[e] = S[(size_t)rsb * n2 + rsi];
+          ia[e] = planes[(size_t)q * nn + (size_t)msa * n + i];
+          ib[e] = planes[(size_t)q * nn + (size_t)msb * n + i];
         }
         __syncthreads();
-        PHASE(type == 0 ? 3 : 7);
-        // ---- Metropolis (lane 0) ----
-        if (tid == 0) {
-          const double lpd = L.dmisc[0];
-          const double lip_new = ddm::cr_log(fabs(ip_of_l(L.qpw, L.pf_new, nqp)));
-          const double ex = 2.0 * (((lpd + 0.0) + lip_new) - L.dmisc[1]);
-          double wgt = ddm::cr_exp(ex);
-          if (!(wgt - wgt == 0.0)) wgt = -1.0;
-          const double u = sfmt_real2(*L.rng);
-          const int acc = wgt > u;
-          L.misc[M_ACC] = acc;
-          if (acc) {
-            L.dmisc[1] = lip_new;
-            L.misc[M_NACC] += 1;
-            ctr[type == 0 ? 1 : 3]++;
-          } else {
-            if (type == 1) {
-              L.ele_idx[mj + t * ne] = rj;
-              L.ele_cfg[ri + t * ns] = -1;
-              L.ele_cfg[rj + t * ns] = mj;
-              L.ele_num[ri + t * ns] = 0;
-              L.ele_num[rj + t * ns] = 1;
-            }
-            L.ele_idx[mi + s * ne] = ri;
-            L.ele_cfg[ri + s * ns] = mi;
-            L.ele_cfg[rj + s * ns] = -1;
-            L.ele_num[ri + s * ns] = 1;
-            L.ele_num[rj + s * ns] = 0;
-          }
+        for (int e = tid; e < nqp * n; e += nt) {
+          const int q = e / n, i = e % n;
+          const Elem* row = planes + (size_t)q * nn + (size_t)i * n;
+          const double* a = va + q * n;
+          double acc = 0.0;
+          for (int j = 0; j < n; ++j) acc += row[j] * a[j];
+          tmp[e] = acc;
         }
         __syncthreads();
-        PHASE(4);
-        const int acc = L.misc[M_ACC];
-        apply_clear_deltas(v, L, cnt, acc != 0);
-        if (acc) {
-          if (type == 0) {
-            // update_one_real_scalar (updates.rs:1184-1224), delayed: one
-            // pass forms vec1 = -(X^T slt) of this update from the current
-            // inverse (pending updates applied in registers), writing the
-            // planes back only when the pending list is full; this update
-            // joins the list.
-            const int msa = mi + s * ne;
-            const bool full = P.np == PEND_MAX;
-            stream_planes<true>(planes, n, nqp, pend_c, P, full, slt, vec1, ld);
-            if (full && wpasses && tid == 0) atomicAdd(wpasses, 1);
-            __syncthreads();
-            if (full) P.np = 0;
-            const int k = P.np;
-            for (int e = tid; e < nqp * n; e += nt) {
-              const int q = e / n;
-              const int j = e - q * n;
-              const double inv_a = -1.0 / vec1[q * ld + msa];
-              pend[(size_t)e * PEND_MAX + k] = PendPair<Elem>::make(vec1[q * ld + j], stage[q * ld + j] * inv_a);
-            }
-#pragma unroll
-            for (int kk = 0; kk < PEND_MAX; ++kk)
-              if (kk == k) P.pm[kk] = msa;
-            P.np = k + 1;
-            for (int q = tid; q < nqp; q += nt) L.pf[q] = L.pf_new[q];
-            __syncthreads();
-            PHASE(5);
-          } else {
-            // update_two_real (updates.rs:1429-1503); pf *= ratio recomputed here
-            const int msa = mi + s * ne, msb = mj + t * ne;
-            const int rsa = L.ele_idx[msa] + s * ns, rsb = L.ele_idx[msb] + t * ns;
-            const int rsa_old = ri + s * ns, rsb_old = rj + t * ns;
-            double* P = L.uni;
-            double* Q = L.uni + nqp * n;
-            double* Sv = L.uni + 2 * nqp * n;
-            double* T = L.uni + 3 * nqp * n;
-            double* cf = L.uni + 5 * nqp * n;  // [nqp][16]
-            for (int e = tid; e < nqp * n; e += nt) {
-              const int q = e / n, i = e % n;
-              const int rsi = L.ele_idx[i] + (i < ne ? 0 : ns);
-              const double* S = v.slater + (size_t)q * n2 * n2;
-              Sv[e] = (i == msb) ? S[(size_t)rsa_old * n2 + rsb_old] : S[(size_t)rsa * n2 + rsi];
-              T[e] = S[(size_t)rsb * n2 + rsi];
-            }
-            __syncthreads();
-            for (int e = tid; e < nqp * n; e += nt) {
-              const int q = e / n, i = e % n;
-              const Elem* row = planes + (size_t)q * nn + (size_t)i * n;
-              double p = 0.0, qq = 0.0;
-              for (int j = 0; j < n; ++j) {
-                const double x = row[j];
-                p += x * Sv[q * n + j];
-                qq += x * T[q * n + j];
-              }
-              P[e] = p;
-              Q[e] = qq;
-            }
-            __syncthreads();
-            for (int q = tid; q < nqp; q += nt) {
-              const double* Pq = P + q * n;
-              const double* Qq = Q + q * n;
-              const double* Tq = T + q * n;
-              double bma = 0.0;
-              for (int i = 0; i < n; ++i) bma += Tq[i] * Pq[i];
-              const double iab = planes[(size_t)q * nn + (size_t)msa * n + msb];
-              const double ratio = iab * Tq[msa] + iab * bma + Pq[msa] * Qq[msb] - Pq[msb] * Qq[msa];
-              L.pf[q] *= ratio;
-              const double a = -Pq[msa], b = Pq[msb], c = Qq[msa], d = -Qq[msb];
-              const double ee = -bma - Tq[msa];
-              const double f = iab;
-              const double det = a * d - b * c - ee * f;
-              double* k = cf + q * 16;
-              k[0] = a; k[1] = b; k[2] = c; k[3] = d; k[4] = ee; k[5] = f; k[6] = det; k[7] = 1.0 / det;
-            }
-            __syncthreads();
-            for (int e = tid; e < nqp * n; e += nt) {  // S, T rows of the old inverse, scaled
-              const int q = e / n, i = e % n;
-              const double idet = cf[q * 16 + 7];
-              const double sa = planes[(size_t)q * nn + (size_t)msa * n + i];
-              const double sb = planes[(size_t)q * nn + (size_t)msb * n + i];
-              Sv[e] = idet * sa;
-              T[e] = idet * sb;
-            }
-            __syncthreads();
-            for (size_t e = tid; e < (size_t)nqp * nn; e += nt) {
-              const int q = (int)(e / nn), r = (int)(e % nn);
-              const int i = r / n, j = r % n;
-              const double* k = cf + q * 16;
-              const double a = k[0], b = k[1], c = k[2], d = k[3], ee = k[4], f = k[5], det = k[6], idet = k[7];
-              const double pi = P[q * n + i], qi = Q[q * n + i], si = Sv[q * n + i], ti = T[q * n + i];
-              const double pj = P[q * n + j], qj = Q[q * n + j], sj = Sv[q * n + j], tj = T[q * n + j];
-              double x = planes[e];
-              x += a * (qi * tj - qj * ti) + b * (qi * sj - qj * si) + c * (pi * tj - pj * ti) +
-                   d * (pi * sj - pj * si) + ee * det * (si * tj - sj * ti) + f * idet * (pi * qj - qi * pj);
-              if (j == msa) x += -c * ti - d * si - f * idet * qi;
-              if (j == msb) x += -a * ti - b * si + f * idet * pi;
-              if (i == msa) x += c * tj + d * sj + f * idet * qj;
-              if (i == msb) x += a * tj + b * sj - f * idet * pj;
-              if (i == msa && j == msb) x += f * idet;
-              if (i == msb && j == msa) x -= f * idet;
-              planes[e] = static_cast<Elem>(x);
-            }
-            __syncthreads();
+        for (int q = tid; q < nqp; q += nt) {
+          const double* a = va + q * n;
+          const double* b = vb + q * n;
+          const double* ra = ia + q * n;
+          const double* rb = ib + q * n;
+          double pa = 0.0, pb = 0.0, qa = 0.0, qb = 0.0;
+          for (int i = 0; i < n; ++i) {
+            pa += ra[i] * a[i];
+            pb += rb[i] * a[i];
+            qa += ra[i] * b[i];
+            qb += rb[i] * b[i];
           }
-        } else {
-          __syncthreads();
+          const double iab = ra[msb];
+          double bma = 0.0;
+          for (int i = 0; i < n; ++i) bma += b[i] * tmp[q * n + i];
+          const double ratio = iab * b[msa] + iab * bma + pa * qb - pb * qa;
+          L.pf_new[q] = ratio * L.pf[q];
         }
       }
-      // ---- periodic recompute (engine.rs:454-473): handed to k_rebuild ----
-      const int nacc_now = L.misc[M_NACC];
       __syncthreads();
-      if (nacc_now > ns) {
-        stop_at = step + 1;
-        break;
-      }
+      PHASE(type == 0 ? 3 : 7);
     }
+    if (tid == 0)
+      for (int k = 0; k < 4; ++k) ctr[k] = ctr_l[k];
     if (stop_at >= 0) {
       // the planes are rebuilt from the configuration, so the pending
       // updates are dropped; the walker resumes at proposal stop_at
