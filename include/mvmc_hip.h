@@ -147,8 +147,8 @@ int mvmc_ens_sr_cg(mvmc_ens* e, long long* cg_info);
  * the Gram of the packed active samples by the library's MFMA kernel
  * (FP64 MFMA; in the precision form, mvmc_ens_set_precision 1, the samples
  * packed in FP32 and FP32 MFMA with FP32 accumulation), S and g as the
- * reference assembles them, Cholesky by rocSOLVER DPOTRF/DPOTRS, parameter update and
- * gauge sync.  The path NSRCG 0 selects in mvmc_ens_opt_step; skipped gets
+ * reference assembles them, blocked Cholesky solve on the matrix cores, parameter
+ * update and gauge sync.  The path NSRCG 0 selects in mvmc_ens_opt_step; skipped gets
  * 1 when the factorisation fails or the solution is not finite (no update),
  * as the reference's cholesky_solve. */
 int mvmc_ens_sr_direct(mvmc_ens* e, int* skipped);
@@ -293,8 +293,7 @@ int mvmc_group_sample(mvmc_group* g);
 int mvmc_group_timings(mvmc_group* g, double* timings10);
 
 /* The standalone SR entry points below (mvmc_sr_cg_apply, mvmc_sr_gram_real,
- * mvmc_sr_cholesky_solve, mvmc_sr_cg_solve) keep one device workspace or
- * rocBLAS handle per process: calls that overlap from several host threads
+ * mvmc_sr_cholesky_solve, mvmc_sr_cg_solve) keep one device workspace per process: calls that overlap from several host threads
  * race; serialise them (the ensemble's own SR uses per-handle state). */
 
 /* SrStages::cg_local_product (crates/mvmc-core/src/sr_backend.rs:518-598),
@@ -322,7 +321,8 @@ int mvmc_sr_gram_real_f32(int n, int samples, const float* store, double* out, v
 
 /* SrStages::cholesky_solve (sr_backend.rs:243-247, crates/mvmc-core/src/sr.rs:535):
  * solves the symmetric positive-definite S x = rhs in place (rhs becomes x,
- * S is overwritten by its factor) with rocSOLVER DPOTRF/DPOTRS.  *info: 0 ok,
+ * S's upper triangle, column-major, is overwritten by its factor, the lower one is
+ * left alone) by a blocked Cholesky on the matrix cores.  *info: 0 ok,
  * k > 0 the factorisation's info (leading minor k not positive definite),
  * -1 non-finite solution (the reference's Err(())).  Device pointers for s and
  * rhs; synchronises `stream`. */

@@ -43,7 +43,7 @@ def object_command(src, macros, obj):
 
 def link_command(objs, out):
     return [HIPCC, f"--offload-arch={ARCH}", "-fPIC", "-shared", "-o", out] + objs + \
-        ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib"]
+        ["-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib"]
 
 
 def build_library(defines=(), out=None):

@@ -3,8 +3,6 @@
 // kernels of ensemble.hip (crates/mvmc-core/src/run.rs:1294-1475 for the
 // step order; multichain.rs:647-689 for the walker = rank mapping).
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <array>
@@ -28,6 +26,7 @@
 #include "pfinv_lds.h"
 #include "rr_planes.h"
 #include "sr_cg.h"
+#include "sr_chol.h"
 #include "sr_stages.h"
 
 using namespace mvmc_hip;
@@ -47,12 +46,6 @@ struct Fail : std::runtime_error {
     if (e_ != hipSuccess)                                                                         \
       throw Fail(MVMC_E_BACKEND, std::string(#x) + ": " + hipGetErrorString(e_) + " (" + __FILE__ + \
                                      ":" + std::to_string(__LINE__) + ")");                       \
-  } while (0)
-#define BLASCHK(x)                                                                                \
-  do {                                                                                            \
-    rocblas_status s_ = (x);                                                                      \
-    if (s_ != rocblas_status_success)                                                             \
-      throw Fail(MVMC_E_BACKEND, std::string(#x) + ": rocBLAS status " + std::to_string((int)s_));  \
   } while (0)
 
 double now_s() {
@@ -468,14 +461,12 @@ struct mvmc_ens {
   int* d_cfg = nullptr;
   char* d_cfg_out = nullptr;
   double* d_rows = nullptr;  // [W*nsample] cotangents / log|psi| of the saved samples
-  // direct SR (NSRCG 0): rocBLAS handle on the library's stream, S [na][na], Cholesky info
-  rocblas_handle blas = nullptr;
+  // direct SR (NSRCG 0): workspace of the Cholesky solve, then S [na][na]
   double* d_S = nullptr;
   size_t S_cap = 0;
   // precision form: FP32 Gram of the packed samples for the CG product
   void* d_gram = nullptr;
   size_t gram_cap = 0;
-  int* d_info = nullptr;
   double* d_grad = nullptr;  // [size]
   // adjoint VJP: per-slot Slater-table cotangents [adj_slots][nqp][n2^2] and
   // constant + projection sums [adj_slots][1 + nproj]; the orbital map as
@@ -493,7 +484,6 @@ struct mvmc_ens {
     cg.release();
     if (d_S) (void)hipFree(d_S);
     if (d_gram) (void)hipFree(d_gram);
-    if (blas) (void)rocblas_destroy_handle(blas);
     for (void* p : allocs) (void)hipFree(p);
     if (st) (void)hipStreamDestroy(st);
   }
@@ -1153,28 +1143,34 @@ void apply_sr_update(mvmc_ens* E, const std::vector<int>& map, const std::vector
   mvmc::sync_modified_parameter(m, true);
 }
 
+// S x = b in place (sr_chol.h); work: chol_ws_doubles(n), 16-byte aligned.
+void chol_solve(double* S, double* x, int n, double* work, hipStream_t st) {
+  raise_lds_limit((const void*)k_chol_step<false>, 3 * sizeof(double) * CH_B * CH_LD + CH_V);
+  raise_lds_limit((const void*)k_chol_step<true>, 2 * sizeof(double) * CH_B * CH_LD + CH_V);
+  raise_lds_limit((const void*)k_chol_panel, 2 * sizeof(double) * CH_B * CH_LD);
+  chol_launches(S, x, n, work, st);
+  HIPCHK(hipGetLastError());
+}
+
 // Direct SR (sr.rs:60-160 real path; sr_backend.rs:484-516 assembly): the
 // Gram inv_w * P P^T of the packed active samples (P = [na][rows] column
-// major) by rocBLAS DGEMM on the matrix cores, S = Gram - mean mean^T with
-// the diagonal scaled by 1 + DSROptStaDel, then Cholesky (rocSOLVER DPOTRF,
-// DPOTRS, upper) on g in place.  A failed factorisation or a non-finite
+// major) on the matrix cores, S = Gram - mean mean^T with
+// the diagonal scaled by 1 + DSROptStaDel, then the Cholesky solve
+// (sr_chol.h) on g in place.  A failed factorisation or a non-finite
 // solution skips the update (return 1), as the reference's cholesky_solve.
 int direct_sr(mvmc_ens* E, const std::vector<int>& map, int na, size_t rows, double inv_w, double t0,
               long long* info_out, bool f32) {
   mvmc::Model& m = E->m;
   hipStream_t st = E->st;
-  if (!E->blas) {
-    BLASCHK(rocblas_create_handle(&E->blas));
-    E->d_info = dalloc<int>(E->allocs, 4);
-  }
-  BLASCHK(rocblas_set_stream(E->blas, st));
-  const size_t nn = (size_t)na * na;
-  if (E->S_cap < nn) {
+  const size_t nn = (size_t)na * na, nws = (chol_ws_doubles(na) + 1) & ~(size_t)1;
+  if (E->S_cap < nn + nws) {
     if (E->d_S) (void)hipFree(E->d_S);
     E->d_S = nullptr;
-    HIPCHK(hipMalloc(&E->d_S, sizeof(double) * nn));
-    E->S_cap = nn;
+    E->S_cap = 0;
+    HIPCHK(hipMalloc(&E->d_S, sizeof(double) * (nn + nws)));
+    E->S_cap = nn + nws;
   }
+  double* const S = E->d_S + nws;
   hipEvent_t c0, c1;
   HIPCHK(hipEventCreate(&c0));
   HIPCHK(hipEventCreate(&c1));
@@ -1187,23 +1183,23 @@ int direct_sr(mvmc_ens* E, const std::vector<int>& map, int na, size_t rows, dou
   HIPCHK(hipEventCreate(&g1));
   if (f32)
     hipLaunchKernelGGL(k_gram_mfma<float>, dim3(tiles), dim3(256), 0, st, (const float*)E->d_pack, (int)rows, na,
-                       inv_w, E->d_S, 0);
+                       inv_w, S, 0);
   else
     hipLaunchKernelGGL(k_gram_mfma<double>, dim3(tiles), dim3(256), 0, st, (const double*)E->d_pack, (int)rows, na,
-                       inv_w, E->d_S, 0);
+                       inv_w, S, 0);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(g1, st));
   hipLaunchKernelGGL(k_sr_assemble, dim3(nblk((long long)nn)), dim3(256), 0, st, na, E->d_cmean,
-                     1.0 + m.mp.dsr_opt_sta_del, E->d_S);
+                     1.0 + m.mp.dsr_opt_sta_del, S);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(E->d_cx, E->d_cg, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-  BLASCHK(rocsolver_dpotrf(E->blas, rocblas_fill_upper, na, E->d_S, na, E->d_info));
-  int info = 0;
-  HIPCHK(hipMemcpyAsync(&info, E->d_info, sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
-  if (info == 0) BLASCHK(rocsolver_dpotrs(E->blas, rocblas_fill_upper, na, 1, E->d_S, na, E->d_cx, na));
+  chol_solve(S, E->d_cx, na, E->d_S, st);
   HIPCHK(hipEventRecord(c1, st));
-  HIPCHK(hipEventSynchronize(c1));
+  int info = 0;
+  std::vector<double> x(na);
+  HIPCHK(hipMemcpyAsync(&info, chol_ws(E->d_S, na).info, sizeof(int), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipMemcpyAsync(x.data(), E->d_cx, sizeof(double) * na, hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
   float ms = 0, gms = 0;
   HIPCHK(hipEventElapsedTime(&ms, c0, c1));
   HIPCHK(hipEventElapsedTime(&gms, c0, g1));
@@ -1222,8 +1218,6 @@ int direct_sr(mvmc_ens* E, const std::vector<int>& map, int na, size_t rows, dou
     E->t_sr += now_s() - t0;
     return 1;
   }
-  std::vector<double> x(na);
-  E->d2h(x.data(), E->d_cx, sizeof(double) * na);
   E->cg_x = x;
   for (double xv : x)
     if (!std::isfinite(xv)) {
@@ -2235,15 +2229,6 @@ int mvmc_ens_status(mvmc_ens* e) {
   return s;
 }
 
-// One rocBLAS handle for the standalone SR stages, created on first use.
-rocblas_handle sr_blas() {
-  static std::mutex mu;
-  static rocblas_handle h = nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!h) BLASCHK(rocblas_create_handle(&h));
-  return h;
-}
-
 int mvmc_sr_gram_real(int n, int samples, const double* store, double* out, void* stream) {
   return guarded([&] {
     require_gpu();
@@ -2277,23 +2262,24 @@ int mvmc_sr_cholesky_solve(int n, double* s, double* rhs, int* info, void* strea
     if (n == 0) return;
     if (!s || !rhs) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
     hipStream_t st = (hipStream_t)stream;
-    rocblas_handle h = sr_blas();
-    BLASCHK(rocblas_set_stream(h, st));
-    int* d_info = nullptr;
-    HIPCHK(hipMallocAsync((void**)&d_info, sizeof(int), st));
-    BLASCHK(rocsolver_dpotrf(h, rocblas_fill_upper, n, s, n, d_info));
+    double* work = nullptr;
+    HIPCHK(hipMallocAsync((void**)&work, sizeof(double) * chol_ws_doubles(n), st));
     int fi = 0;
-    HIPCHK(hipMemcpyAsync(&fi, d_info, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipFreeAsync(d_info, st));
+    std::vector<double> x(n);
+    try {
+      chol_solve(s, rhs, n, work, st);
+      HIPCHK(hipMemcpyAsync(&fi, chol_ws(work, n).info, sizeof(int), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipMemcpyAsync(x.data(), rhs, sizeof(double) * n, hipMemcpyDeviceToHost, st));
+    } catch (...) {
+      (void)hipFreeAsync(work, st);
+      throw;
+    }
+    HIPCHK(hipFreeAsync(work, st));
     HIPCHK(hipStreamSynchronize(st));
     if (fi != 0) {
       *info = fi;
       return;
     }
-    BLASCHK(rocsolver_dpotrs(h, rocblas_fill_upper, n, 1, s, n, rhs, n));
-    std::vector<double> x(n);
-    HIPCHK(hipMemcpyAsync(x.data(), rhs, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
     for (double v : x)
       if (!std::isfinite(v)) {
         *info = -1;
