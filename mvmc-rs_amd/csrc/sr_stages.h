@@ -105,9 +105,9 @@ __global__ void __launch_bounds__(256) k_gram_complex(const double* store, int n
 // store.  One 256-thread workgroup per 64 x 64 tile of the upper triangle
 // (tiles (ti, tj), ti <= tj, enumerated column by column); each wave owns a
 // 32 x 32 quarter as 2 x 2 blocks of 16 x 16 accumulators; rows stream
-// through LDS GM_KC at a time (double-buffered: the next chunk's global
-// loads are in flight while the current one feeds the MFMAs, one barrier
-// per chunk) and every block consumes them 4 per MFMA
+// through LDS GM_KC at a time (double-buffered, one barrier per chunk; the
+// global loads of the next GM_AHEAD chunks are in flight while the current
+// one feeds the MFMAs) and every block consumes them 4 per MFMA
 // (v_mfma_f64_16x16x4f64, or v_mfma_f32_16x16x4f32 with FP32 accumulation
 // for a float store).  MFMA operand layout (16 x 16 x 4, one block): lane l
 // supplies A[l % 16][l / 16] and B[l / 16][l % 16]; accumulator element e of
@@ -137,6 +137,10 @@ struct GramMfma<float> {
   static __device__ __forceinline__ int row(int lane, int e) { return 4 * (lane >> 4) + e; }
 };
 constexpr int GM_T = 64, GM_KC = 16;
+// Chunks in flight: with one, a tile waited out the latency of every chunk
+// (na = 1111, 4096 rows: 171 tiles, less than one per CU; 292 -> 235 us).
+constexpr int GM_AHEAD = 4;
+static_assert(GM_AHEAD % 2 == 0);
 constexpr int GM_XCDS = 8;  // XCDs of an MI355X (workgroup dispatch order)
 constexpr int GM_LD = 80;  // LDS row stride (elements): the 4 k-rows of one operand fetch fall in two bank halves
 
@@ -151,7 +155,7 @@ __global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int 
   using Op = GramMfma<P>;
   using acc_t = typename Op::acc_t;
   // two LDS buffers: the chunk in use and the next one, stored from the
-  // registers its global loads landed in while the MFMAs ran
+  // registers its global loads landed in
   __shared__ P sA[2][GM_KC][GM_LD];
   __shared__ P sB[2][GM_KC][GM_LD];
   // XCD-aware tile order: workgroups are dealt round-robin over the 8 XCDs
@@ -175,51 +179,63 @@ __global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int 
   for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
-  const int lr = tid >> 4, lc = (tid & 15) * 4;  // loader: row lr of the chunk, 4 columns from lc
-  P ra[4], rb[4];
-  auto load = [&](int r0) {
-    const int r = r0 + lr;
-    const bool rin = r < rows;
-    const P* row = pack + (size_t)(rin ? r : 0) * na;
+  // loader: row lr of a chunk, columns lc, lc + 16, ..; columns past na repeat
+  // the last one (their products are not written), rows past the end are zero
+  const int lr = tid >> 4, lc = tid & 15;
+  int ci[4], cj[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int ci = i0 + lc + u, cj = j0 + lc + u;
-      ra[u] = (rin && ci < na) ? row[ci] : (P)0;
-      rb[u] = (rin && cj < na) ? row[cj] : (P)0;
-    }
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      sA[buf][lr][lc + u] = ra[u];
-      sB[buf][lr][lc + u] = rb[u];
-    }
-  };
-  load(0);
-  store(0);
-  __syncthreads();
-  int buf = 0;
-  for (int r0 = 0; r0 < rows; r0 += GM_KC) {
-    const bool more = r0 + GM_KC < rows;
-    if (more) load(r0 + GM_KC);
-#pragma unroll
-    for (int k0 = 0; k0 < GM_KC; k0 += 4) {
-      const int k = k0 + (lane >> 4), m = lane & 15;
-      P av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a) av[a] = sA[buf][k][32 * wi + 16 * a + m];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) bv[b] = sB[buf][k][32 * wj + 16 * b + m];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = Op::op(av[a], bv[b], acc[a][b]);
-    }
-    // the other buffer was last read before the previous barrier
-    if (more) store(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
+  for (int u = 0; u < 4; ++u) {
+    ci[u] = min(i0 + lc + 16 * u, na - 1);
+    cj[u] = min(j0 + lc + 16 * u, na - 1);
   }
+  P ra[GM_AHEAD][4], rb[GM_AHEAD][4];
+  auto load = [&](int r0, P (&a)[4], P (&b)[4]) __attribute__((always_inline)) {
+    const P* row = pack + (size_t)min(r0 + lr, rows - 1) * na;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[u] = row[ci[u]];
+      b[u] = row[cj[u]];
+    }
+  };
+  auto store = [&](int r0, int buf, const P (&a)[4], const P (&b)[4]) __attribute__((always_inline)) {
+    const bool in = r0 + lr < rows;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      sA[buf][lr][lc + 16 * u] = in ? a[u] : (P)0;
+      sB[buf][lr][lc + 16 * u] = in ? b[u] : (P)0;
+    }
+  };
+  if (rows > 0) {
+#pragma unroll
+    for (int u = 0; u < GM_AHEAD; ++u) load(u * GM_KC, ra[u], rb[u]);
+    store(0, 0, ra[0], rb[0]);
+  }
+  __syncthreads();
+  for (int base = 0; base < rows; base += GM_AHEAD * GM_KC)
+#pragma unroll
+    for (int u = 0; u < GM_AHEAD; ++u) {
+      const int r0 = base + u * GM_KC, buf = u & 1;
+      if (r0 < rows) {
+        if (r0 + GM_AHEAD * GM_KC < rows) load(r0 + GM_AHEAD * GM_KC, ra[u], rb[u]);
+#pragma unroll
+        for (int k0 = 0; k0 < GM_KC; k0 += 4) {
+          const int k = k0 + (lane >> 4), m = lane & 15;
+          P av[2], bv[2];
+#pragma unroll
+          for (int a = 0; a < 2; ++a) av[a] = sA[buf][k][32 * wi + 16 * a + m];
+#pragma unroll
+          for (int b = 0; b < 2; ++b) bv[b] = sB[buf][k][32 * wj + 16 * b + m];
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = Op::op(av[a], bv[b], acc[a][b]);
+        }
+        // the other buffer was last read before the previous barrier
+        const int nx = (u + 1) % GM_AHEAD;
+        if (r0 + GM_KC < rows) store(r0 + GM_KC, buf ^ 1, ra[nx], rb[nx]);
+        __syncthreads();
+      }
+    }
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
