@@ -31,10 +31,56 @@ __host__ __device__ inline size_t cgs_lds_doubles(int na, int rows, bool gram) {
   return 7 * (size_t)na + nch * na + 8;
 }
 
-// Pairwise tree over the 64 lanes (h = 32 .. 1), result in lane 0.
+// Exchanges between the halves of a wave (and between odd and even rows of 16
+// lanes) of two registers, and rotations of a row: a step of a tree without
+// the LDS round trip of a shuffle.
+__device__ __forceinline__ double cg_f64(unsigned lo, unsigned hi) {
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// a + b with a = lanes 0..31 of x, then of y; b = lanes 32..63 of x, then of y
+__device__ __forceinline__ double cg_fold32(double x, double y) {
+  const unsigned long long bx = __builtin_bit_cast(unsigned long long, x), by = __builtin_bit_cast(unsigned long long, y);
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)bx, (unsigned)by, false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(bx >> 32), (unsigned)(by >> 32), false, false);
+  return cg_f64(l[0], h[0]) + cg_f64(l[1], h[1]);
+}
+// the same for the rows 0, 2 and 1, 3 of 16 lanes: x0 + x1, y0 + y1, x2 + x3, y2 + y3
+__device__ __forceinline__ double cg_fold16(double x, double y) {
+  const unsigned long long bx = __builtin_bit_cast(unsigned long long, x), by = __builtin_bit_cast(unsigned long long, y);
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)bx, (unsigned)by, false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(bx >> 32), (unsigned)(by >> 32), false, false);
+  return cg_f64(l[0], h[0]) + cg_f64(l[1], h[1]);
+}
+// x + x rotated by H lanes within every row of 16
+template <int H>
+__device__ __forceinline__ double cg_ror(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + H, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + H, 0xf, 0xf, true);
+  return x + cg_f64(lo, hi);
+}
+__device__ __forceinline__ double cg_tree16(double v) { return cg_ror<1>(cg_ror<2>(cg_ror<4>(cg_ror<8>(v)))); }
+
+// Pairwise tree over the 64 lanes (h = 32 .. 1; sums of two, so the sides may
+// swap), result in every lane.
 __device__ __forceinline__ double cg_tree64(double v) {
-  for (int h = 32; h >= 1; h >>= 1) v += __shfl_down(v, h, 64);
-  return v;
+  v = cg_fold32(v, v);
+  return cg_tree16(cg_fold16(v, v));
+}
+
+// The trees of U = 4 values at once: lanes 0..15 hold the first's, 16..31 the
+// third's, 32..47 the second's, 48..63 the fourth's; of two: a half each.
+template <int U>
+__device__ __forceinline__ double cg_trees(const double (&v)[U]) {
+  static_assert(U == 2 || U == 4);
+  const double a = cg_fold32(v[0], v[1]);
+  return cg_tree16(cg_fold16(a, U == 4 ? cg_fold32(v[U - 2], v[U - 1]) : a));
+}
+
+__device__ __forceinline__ double cg_lane(double x, int lane) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  return cg_f64((unsigned)__builtin_amdgcn_readlane((int)b, lane),
+                (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), lane));
 }
 
 // bdot of the 256 strided lane partials that one wave holds as p[t] = partial
@@ -60,16 +106,22 @@ __device__ void cgs_apply(const P* op, int rows, int na, const double* v, const 
     const double c = cg_tree256_wave(p[0], p[1], p[2], p[3]);
     if (lane == 0) red[0] = c;
   }
-  constexpr int U = M <= 5 ? 4 : 2;  // rows in flight per wave
+  // Four rows at a time (two where four do not fit the registers), the loads of
+  // the next ones ahead of these ones' sums:
+  // with the rows alone in flight a wave waited out an L2 latency per group,
+  // and a shuffle's per step of their trees.
+  constexpr int U = M <= 7 ? 4 : 2;
+  auto load = [&](int r, int r1, P (&o)[U][M]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const P* row = op + (size_t)min(r + u, r1 - 1) * na;
+#pragma unroll
+      for (int m = 0; m < M; ++m) o[u][m] = row[min(lane + 64 * m, na - 1)];
+    }
+  };
   if constexpr (GRAM) {
-    // row i of the symmetric Gram, as k_gram_apply sums it
-    for (int i0 = wave * U; i0 < na; i0 += CGS_WAVES * U) {
-      P o[U][M];
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int m = 0; m < M; ++m)
-          o[u][m] = i0 + u < na && lane + 64 * m < na ? op[(size_t)(i0 + u) * na + lane + 64 * m] : (P)0;
+    // row i of the symmetric Gram, as k_gram_product sums it
+    auto rows4 = [&](int i0, const P (&o)[U][M]) __attribute__((always_inline)) {
       double a[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -78,13 +130,19 @@ __device__ void cgs_apply(const P* op, int rows, int na, const double* v, const 
         for (int m = 0; m < M; ++m)
           if (lane + 64 * m < na) a[u] += (double)o[u][m] * xv[m];
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u) a[u] = cg_tree64(a[u]);
-      if (lane == 0) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (i0 + u < na) cp[i0 + u] = a[u];
-      }
+      const double t = cg_trees<U>(a);
+      const int i = i0 + (U == 4 ? 2 * ((lane >> 4) & 1) : 0) + (lane >> 5);
+      if ((lane & (U == 4 ? 15 : 31)) == 0 && i < na) cp[i] = t;
+    };
+    P o0[U][M], o1[U][M];
+    constexpr int STEP = CGS_WAVES * U;
+    int i0 = wave * U;
+    if (i0 < na) load(i0, na, o0);
+    for (; i0 < na; i0 += 2 * STEP) {
+      if (i0 + STEP < na) load(i0 + STEP, na, o1);
+      rows4(i0, o0);
+      if (i0 + 2 * STEP < na) load(i0 + 2 * STEP, na, o0);
+      if (i0 + STEP < na) rows4(i0 + STEP, o1);
     }
   } else {
     // a wave per chunk of CG_RCH rows: the row's dot, then its axpy from the
@@ -95,28 +153,32 @@ __device__ void cgs_apply(const P* op, int rows, int na, const double* v, const 
       double acc[M];
 #pragma unroll
       for (int m = 0; m < M; ++m) acc[m] = 0.0;
-      for (int r = r0; r < r1; r += U) {
-        double o[U][M], y[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int m = 0; m < M; ++m)
-            o[u][m] = r + u < r1 && lane + 64 * m < na ? (double)op[(size_t)(r + u) * na + lane + 64 * m] : 0.0;
+      auto rows4 = [&](int r, const P (&o)[U][M]) __attribute__((always_inline)) {
+        double y[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           double p[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
           for (int m = 0; m < M; ++m)
-            if (lane + 64 * m < na) p[m & 3] += o[u][m] * xv[m];
-          y[u] = cg_tree256_wave(p[0], p[1], p[2], p[3]);
+            if (lane + 64 * m < na) p[m & 3] += (double)o[u][m] * xv[m];
+          y[u] = (p[0] + p[2]) + (p[1] + p[3]);
         }
+        const double t = cg_trees<U>(y);
 #pragma unroll
         for (int u = 0; u < U; ++u)
           if (r + u < r1) {
-            const double yu = __shfl(y[u], 0, 64);
+            const double yu = cg_lane(t, u == 0 ? 0 : u == 1 ? 32 : u == 2 ? 16 : 48);
 #pragma unroll
-            for (int m = 0; m < M; ++m) acc[m] += o[u][m] * yu;
+            for (int m = 0; m < M; ++m) acc[m] += (double)o[u][m] * yu;
           }
+      };
+      P o0[U][M], o1[U][M];
+      load(r0, r1, o0);
+      for (int r = r0; r < r1; r += 2 * U) {
+        if (r + U < r1) load(r + U, r1, o1);
+        rows4(r, o0);
+        if (r + 2 * U < r1) load(r + 2 * U, r1, o0);
+        if (r + U < r1) rows4(r + U, o1);
       }
 #pragma unroll
       for (int m = 0; m < M; ++m)
