@@ -13,6 +13,7 @@
 #include <cstring>
 #include <filesystem>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <set>
 #include <stdexcept>
@@ -195,6 +196,38 @@ void cg_small(const P* op, int rows, int na, const double* mean, const double* d
   HIPCHK(hipGetLastError());
 }
 
+// {threshold, preconditioner factor} of a solve.
+inline std::array<double, 2> cg_limits(int na, double tol, double shift) {
+  return {tol * tol * (double)na * (double)na, 1.0 + shift};
+}
+
+long long cg_status(CgWork& wk, hipStream_t st) {
+  int ctl[4];
+  HIPCHK(hipMemcpyAsync(ctl, wk.ctl, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  return (long long)(((unsigned long long)(unsigned)ctl[2] << 32) | (unsigned)ctl[1]);
+}
+
+// Issues the solve if one launch does it (x_out and wk.ctl hold its result
+// when the stream gets there); false otherwise.
+template <class P>
+bool cg_issue_small(int na, int rows, const P* pack, const double* mean, const double* diag, const double* g,
+                    double inv_w, double shift, double tol, int max_it, bool diag_scale, double* x_out, CgWork& wk,
+                    hipStream_t st, const float* gram) {
+  const long long elems = (long long)na * (gram ? na : rows);
+  if (na > 64 * CGS_M || rows <= 0 || elems > CGS_ELEMS) return false;
+  wk.ensure(na, rows);
+  const auto [threshold, pfac] = cg_limits(na, tol, shift);
+  if (gram)
+    cg_small<true>(gram, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
+                   wk.ctl, st);
+  else
+    cg_small<false>(pack, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
+                    wk.ctl, st);
+  HIPCHK(hipMemcpyAsync(x_out, wk.x, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
+  return true;
+}
+
 // C 1.4.0 StochasticOptCG_Main / PreconCG_DiagScale (sr_cg.rs:700-880).
 // Operators that one CU streams fast enough (CGS_ELEMS) are solved by one
 // launch.  Otherwise an iteration is its product (chunk partials and their
@@ -208,9 +241,10 @@ long long cg_solve_dev(int na, int W, int NS, const P* pack, const double* mean,
                        const double* g, double inv_w, double shift, double tol, int max_it, bool diag_scale,
                        double* x_out, CgWork& wk, hipStream_t st, const float* gram = nullptr) {
   const int rows = W * NS;
+  if (cg_issue_small(na, rows, pack, mean, diag, g, inv_w, shift, tol, max_it, diag_scale, x_out, wk, st, gram))
+    return cg_status(wk, st);
   wk.ensure(na, rows);
-  const double threshold = tol * tol * (double)na * (double)na;
-  const double pfac = 1.0 + shift;
+  const auto [threshold, pfac] = cg_limits(na, tol, shift);
   const dim3 blk(256);
   auto read_ctl = [&](int (&ctl)[4]) {
     HIPCHK(hipMemcpyAsync(ctl, wk.ctl, sizeof(int) * 4, hipMemcpyDeviceToHost, st));
@@ -218,17 +252,6 @@ long long cg_solve_dev(int na, int W, int NS, const P* pack, const double* mean,
     return (long long)(((unsigned long long)(unsigned)ctl[2] << 32) | (unsigned)ctl[1]);
   };
   int ctl[4];
-  const long long elems = (long long)na * (gram ? na : rows);
-  if (na <= 64 * CGS_M && rows > 0 && elems <= CGS_ELEMS) {
-    if (gram)
-      cg_small<true>(gram, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
-                     wk.ctl, st);
-    else
-      cg_small<false>(pack, rows, na, mean, diag, g, inv_w, shift, threshold, pfac, max_it, diag_scale ? 1 : 0, wk.x,
-                      wk.ctl, st);
-    HIPCHK(hipMemcpyAsync(x_out, wk.x, sizeof(double) * na, hipMemcpyDeviceToDevice, st));
-    return read_ctl(ctl);
-  }
   auto product = [&](const double* xv) {
     if (!gram) return cg_product(na, rows, pack, mean, xv, wk, st);
     hipLaunchKernelGGL(k_gram_product, dim3((na + 3) / 4 + 1), blk, 0, st, gram, na, xv, mean, wk.spart, wk.sc + 5,
@@ -392,6 +415,20 @@ T* dupload(std::vector<void*>& list, const std::vector<T>& h, hipStream_t st) {
   return p;
 }
 
+// The operands of one SR solve, on their way to the device (their
+// host copies stay until the copies are done).
+struct SrJob {
+  std::vector<int> map;
+  std::vector<double> mean, diag, g;
+  const float* gram = nullptr;
+  hipEvent_t c0 = nullptr, c1 = nullptr;  // around the solve
+  bool issued = false;
+  ~SrJob() {
+    if (c0) (void)hipEventDestroy(c0);
+    if (c1) (void)hipEventDestroy(c1);
+  }
+};
+
 }  // namespace
 
 struct mvmc_ens {
@@ -464,6 +501,7 @@ struct mvmc_ens {
   // direct SR (NSRCG 0): workspace of the Cholesky solve, then S [na][na]
   double* d_S = nullptr;
   size_t S_cap = 0;
+  std::shared_ptr<SrJob> job;  // an SR solve issued ahead of sr_impl
   // precision form: FP32 Gram of the packed samples for the CG product
   void* d_gram = nullptr;
   size_t gram_cap = 0;
@@ -1229,12 +1267,10 @@ int direct_sr(mvmc_ens* E, const std::vector<int>& map, int na, size_t rows, dou
   return 0;
 }
 
-// sr_cg.rs:201-484 (real parameters, offset 1, no RescaleSmat); NSRCG 0
-// takes the direct path above.
-int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
+std::shared_ptr<SrJob> sr_prepare(mvmc_ens* E, bool force_direct) {
+  auto job = std::make_shared<SrJob>();
   mvmc::Model& m = E->m;
   EnsView& v = E->v;
-  const double t0 = now_s();
   const int np = m.n_para(), size = m.sr_opt_size();
   if (m.mp.rescale_smat) throw Fail(MVMC_E_INPUT, "RescaleSmat is not supported");
   std::vector<double> var(np);
@@ -1249,16 +1285,18 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
   else
     for (double x : var) vmax = std::fmax(vmax, x);
   const double thr = vmax * m.mp.dsr_opt_red_cut;
-  std::vector<int> map;
+  std::vector<int>& map = job->map;
   for (int pi = 0; pi < np; ++pi) {
     if (m.opt_flags[2 * pi] != 1) continue;
     if (var[pi] < thr) continue;
     map.push_back(pi);
   }
-  E->cg_x.clear();
-  if (map.empty()) { *info_out = 0; E->cg_info = 0; E->t_sr += now_s() - t0; return 0; }
+  if (map.empty()) return job;
   const int na = (int)map.size();
-  std::vector<double> mean(na), diag(na), g(na);
+  std::vector<double>&mean = job->mean, &diag = job->diag, &g = job->g;
+  mean.resize(na);
+  diag.resize(na);
+  g.resize(na);
   const double dt = 2.0 * m.mp.dsr_opt_step_dt;
   for (int si = 0; si < na; ++si) {
     const int idx = map[si] + 1;
@@ -1291,17 +1329,13 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
     hipLaunchKernelGGL(k_cg_pack<double>, dim3(nblk((long long)(rows * na))), dim3(256), 0, st, v, E->d_map, na,
                        (double*)E->d_pack);
   HIPCHK(hipGetLastError());
-  const double inv_w = 1.0 / E->wc;
-  if (direct) return direct_sr(E, map, na, rows, inv_w, t0, info_out, f32);
-  const int max_it = m.mp.nsr_opt_cg_max_iter > 0 ? m.mp.nsr_opt_cg_max_iter : na;
-  hipEvent_t c0, c1;
-  HIPCHK(hipEventCreate(&c0));
-  HIPCHK(hipEventCreate(&c1));
-  HIPCHK(hipEventRecord(c0, st));
+  if (direct) return job;
+  HIPCHK(hipEventCreate(&job->c0));
+  HIPCHK(hipEventCreate(&job->c1));
+  HIPCHK(hipEventRecord(job->c0, st));
   // precision form: the CG product from the FP32-MFMA Gram of the FP32
   // samples (one MFMA pass, then na^2 per product instead of rows * na),
   // when the Gram fits in 2 GiB
-  const float* gram = nullptr;
   if (f32 && (size_t)na * na * sizeof(float) <= ((size_t)2 << 30)) {
     const size_t gb = (size_t)na * na * sizeof(float);
     if (E->gram_cap < gb) {
@@ -1313,16 +1347,64 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
     hipLaunchKernelGGL((k_gram_mfma<float, float>), dim3((unsigned)gm_tiles(na)), dim3(256), 0, st,
                        (const float*)E->d_pack, (int)rows, na, 1.0, (float*)E->d_gram, 1);
     HIPCHK(hipGetLastError());
-    gram = (const float*)E->d_gram;
+    job->gram = (const float*)E->d_gram;
   }
+  return job;
+}
+
+int sr_max_it(const mvmc_ens* E, int na) {
+  return E->m.mp.nsr_opt_cg_max_iter > 0 ? E->m.mp.nsr_opt_cg_max_iter : na;
+}
+
+// The SR-CG solve of a run that one launch does, issued ahead of sr_impl: the
+// runs of a group have a stream each, and their one-workgroup solves run side
+// by side (4 runs of 2.3 .. 14.7 ms: 28 -> 15 ms).
+void sr_issue(mvmc_ens* E) {
+  const mvmc::Model& m = E->m;
+  if (m.mp.nsrcg == 0) return;
+  auto job = sr_prepare(E, false);
+  if (!job->map.empty()) {
+    const int na = (int)job->map.size();
+    const double inv_w = 1.0 / E->wc;
+    auto issue = [&](auto* pack) {
+      return cg_issue_small(na, E->v.W * E->v.nsample, pack, E->d_cmean, E->d_cdiag, E->d_cg, inv_w,
+                            m.mp.dsr_opt_sta_del, m.mp.dsr_opt_cg_tol, sr_max_it(E, na), m.mp.use_diag_scale != 0,
+                            E->d_cx, E->cg, E->st, job->gram);
+    };
+    job->issued = E->precision == 1 ? issue((const float*)E->d_pack) : issue((const double*)E->d_pack);
+    if (job->issued) HIPCHK(hipEventRecord(job->c1, E->st));
+  }
+  E->job = job;
+}
+
+// sr_cg.rs:201-484 (real parameters, offset 1, no RescaleSmat); NSRCG 0
+// takes the direct path above.
+int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
+  mvmc::Model& m = E->m;
+  EnsView& v = E->v;
+  const double t0 = now_s();
+  std::shared_ptr<SrJob> job = std::move(E->job);
+  if (!job) job = sr_prepare(E, force_direct);
+  const std::vector<int>& map = job->map;
+  E->cg_x.clear();
+  if (map.empty()) { *info_out = 0; E->cg_info = 0; E->t_sr += now_s() - t0; return 0; }
+  hipStream_t st = E->st;
+  const int na = (int)map.size();
+  const size_t rows = (size_t)v.W * v.nsample;
+  const bool f32 = E->precision == 1;
+  const double inv_w = 1.0 / E->wc;
+  if (m.mp.nsrcg == 0 || force_direct) return direct_sr(E, map, na, rows, inv_w, t0, info_out, f32);
+  const int max_it = sr_max_it(E, na);
+  const float* gram = job->gram;
+  hipEvent_t c0 = job->c0, c1 = job->c1;
   auto solve = [&](bool dscale) {
     return f32 ? cg_solve_dev(na, v.W, v.nsample, (const float*)E->d_pack, E->d_cmean, E->d_cdiag, E->d_cg, inv_w,
                               m.mp.dsr_opt_sta_del, m.mp.dsr_opt_cg_tol, max_it, dscale, E->d_cx, E->cg, st, gram)
                : cg_solve_dev(na, v.W, v.nsample, (const double*)E->d_pack, E->d_cmean, E->d_cdiag, E->d_cg, inv_w,
                               m.mp.dsr_opt_sta_del, m.mp.dsr_opt_cg_tol, max_it, dscale, E->d_cx, E->cg, st);
   };
-  long long status = solve(m.mp.use_diag_scale != 0);
-  HIPCHK(hipEventRecord(c1, st));
+  long long status = job->issued ? cg_status(E->cg, st) : solve(m.mp.use_diag_scale != 0);
+  if (!job->issued) HIPCHK(hipEventRecord(c1, st));
   HIPCHK(hipEventSynchronize(c1));
   {
     float ms = 0;
@@ -1332,8 +1414,6 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
     E->cg_na = na;
     E->cg_rows = (double)rows;
   }
-  (void)hipEventDestroy(c0);
-  (void)hipEventDestroy(c1);
   long long info = status;
   if (status < 0) {
     if (m.mp.nsrcg_fallback) {
@@ -2406,6 +2486,25 @@ int mvmc_group_opt_step(mvmc_group* g, double* rows) {
     group_sample(g);
     group_measure(g);
     const double t0 = now_s();
+    // no issued solve outlives the step (finish_opt_step of an earlier run may throw)
+    struct Jobs {
+      std::vector<mvmc_ens*>& runs;
+      ~Jobs() {
+        for (mvmc_ens* e : runs)
+          if (e->job) {
+            (void)hipStreamSynchronize(e->st);
+            e->job.reset();
+          }
+      }
+    } jobs{g->runs};
+    for (mvmc_ens* e : g->runs) {
+      // what a run's preparation throws is thrown in its own turn, below
+      try {
+        sr_issue(e);
+      } catch (const Fail&) {
+        e->job.reset();
+      }
+    }
     for (size_t r = 0; r < g->runs.size(); ++r) finish_opt_step(g->runs[r], rows ? rows + 6 * r : nullptr);
     g->t_sr = now_s() - t0;
     if (g->autotune) {
