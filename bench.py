@@ -447,7 +447,7 @@ def main():
                                     "achieved_GBs": cb / (tl["cg_ms"] / 1e3) / 1e9,
                                     "frac_hbm": cb / (tl["cg_ms"] / 1e3) / 1e9 / HBM_PEAK_GBS}
     variants = ["3 workgroups/CU, 8-column close batches", "2 workgroups/CU, 16-column close batches",
-                "register-resident, one 1024-thread workgroup per CU"]
+                "plane by plane, one wave (n <= 104) or four waves each"]
     rv = int(tl["rebuild_variant"])
     out["autotuned"] = {"rebuild_variant": variants[rv] if 0 <= rv < len(variants) else "not decided",
                         "rebuild_ms_per_walker_measured": list(tl["rebuild_ms_per_walker"])}
@@ -499,9 +499,9 @@ def main():
         skipped["derivative_form"] = "budget"
     if not args.no_direct:
         if time.time() + 30 + margin < deadline:
-            # direct SR (NSRCG 0 path) on the same measured operands: Gram by
-            # DGEMM on the matrix cores + Cholesky
-            ens.sr_direct()   # first call: rocSOLVER initialisation
+            # direct SR (NSRCG 0 path) on the same measured operands: Gram on the
+            # matrix cores + Cholesky
+            ens.sr_direct()   # first call: allocates the matrix
             ens.sr_direct()
             td = ens.timings()
             na_, rows_ = td["cg_na"], td["cg_rows"]
