@@ -1216,15 +1216,12 @@ int direct_sr(mvmc_ens* E, const std::vector<int>& map, int na, size_t rows, dou
   // upper triangle of the Gram inv_w P P^T on the matrix cores (FP64 MFMA;
   // FP32 MFMA with FP32 accumulation in the precision form)
   if (rows > (size_t)INT32_MAX) throw Fail(MVMC_E_INVALID_SHAPE, "too many sample rows for the Gram kernel");
-  const unsigned tiles = (unsigned)gm_tiles(na);
   hipEvent_t g1;
   HIPCHK(hipEventCreate(&g1));
   if (f32)
-    hipLaunchKernelGGL(k_gram_mfma<float>, dim3(tiles), dim3(256), 0, st, (const float*)E->d_pack, (int)rows, na,
-                       inv_w, S, 0);
+    gram_launch((const float*)E->d_pack, (int)rows, na, inv_w, S, 0, st);
   else
-    hipLaunchKernelGGL(k_gram_mfma<double>, dim3(tiles), dim3(256), 0, st, (const double*)E->d_pack, (int)rows, na,
-                       inv_w, S, 0);
+    gram_launch((const double*)E->d_pack, (int)rows, na, inv_w, S, 0, st);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(g1, st));
   hipLaunchKernelGGL(k_sr_assemble, dim3(nblk((long long)nn)), dim3(256), 0, st, na, E->d_cmean,
@@ -1344,8 +1341,7 @@ std::shared_ptr<SrJob> sr_prepare(mvmc_ens* E, bool force_direct) {
       HIPCHK(hipMalloc(&E->d_gram, gb));
       E->gram_cap = gb;
     }
-    hipLaunchKernelGGL((k_gram_mfma<float, float>), dim3((unsigned)gm_tiles(na)), dim3(256), 0, st,
-                       (const float*)E->d_pack, (int)rows, na, 1.0, (float*)E->d_gram, 1);
+    gram_launch((const float*)E->d_pack, (int)rows, na, 1.0, (float*)E->d_gram, 1, st);
     HIPCHK(hipGetLastError());
     job->gram = (const float*)E->d_gram;
   }
@@ -2315,8 +2311,7 @@ int mvmc_sr_gram_real(int n, int samples, const double* store, double* out, void
     if (n < 0 || samples < 0) throw Fail(MVMC_E_INVALID_SHAPE, "bad Gram dimensions");
     if (n == 0) return;
     if (!out || (!store && samples > 0)) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
-    hipLaunchKernelGGL(k_gram_mfma<double>, dim3((unsigned)gm_tiles(n)), dim3(256), 0, (hipStream_t)stream,
-                       store, samples, n, 1.0, out, 1);
+    gram_launch(store, samples, n, 1.0, out, 1, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
   });
 }
@@ -2327,8 +2322,7 @@ int mvmc_sr_gram_real_f32(int n, int samples, const float* store, double* out, v
     if (n < 0 || samples < 0) throw Fail(MVMC_E_INVALID_SHAPE, "bad Gram dimensions");
     if (n == 0) return;
     if (!out || (!store && samples > 0)) throw Fail(MVMC_E_INVALID_SHAPE, "null buffer");
-    hipLaunchKernelGGL(k_gram_mfma<float>, dim3((unsigned)gm_tiles(n)), dim3(256), 0, (hipStream_t)stream,
-                       store, samples, n, 1.0, out, 1);
+    gram_launch(store, samples, n, 1.0, out, 1, (hipStream_t)stream);
     HIPCHK(hipGetLastError());
   });
 }

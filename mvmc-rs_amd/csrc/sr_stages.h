@@ -102,9 +102,9 @@ __global__ void __launch_bounds__(256) k_gram_complex(const double* store, int n
 // Gram of the stored samples on the matrix cores (COrderSr::gram_real,
 // sr_backend.rs:312-333, and the Gram of the direct solve, sr.rs:60-160):
 // G[i + j na] = scale * sum_r P[r][i] P[r][j] over a row-major [rows][na]
-// store.  One 256-thread workgroup per 64 x 64 tile of the upper triangle
-// (tiles (ti, tj), ti <= tj, enumerated column by column); each wave owns a
-// 32 x 32 quarter as 2 x 2 blocks of 16 x 16 accumulators; rows stream
+// store.  One 512-thread workgroup per 64 x 64 tile of the upper triangle
+// (tiles (ti, tj), ti <= tj, enumerated column by column); each wave owns
+// 16 x 32 as two blocks of 16 x 16 accumulators; rows stream
 // through LDS GM_KC at a time (double-buffered, one barrier per chunk; the
 // global loads of the next GM_AHEAD chunks are in flight while the current
 // one feeds the MFMAs) and every block consumes them 4 per MFMA
@@ -138,8 +138,12 @@ struct GramMfma<float> {
 };
 constexpr int GM_T = 64, GM_KC = 16;
 // Chunks in flight: with one, a tile waited out the latency of every chunk
-// (na = 1111, 4096 rows: 171 tiles, less than one per CU; 292 -> 235 us).
+// (na = 1111, 4096 rows: 171 tiles, less than one per CU; 292 -> 230 us).
 constexpr int GM_AHEAD = 4;
+// Waves of a workgroup: two a SIMD cover each other's LDS reads and barriers
+// (4096 rows, FP64: 230 us with four waves, 198 with eight at na = 1111; 858
+// and 840 at na = 2900, where a CU has other tiles too).
+constexpr int GM_W = 8;
 static_assert(GM_AHEAD % 2 == 0);
 constexpr int GM_XCDS = 8;  // XCDs of an MI355X (workgroup dispatch order)
 constexpr int GM_LD = 80;  // LDS row stride (elements): the 4 k-rows of one operand fetch fall in two bank halves
@@ -150,7 +154,7 @@ __host__ __device__ inline long long gm_tiles(int na) {
 }
 
 template <class P, class OutT = double>
-__global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int na, double scale, OutT* G,
+__global__ void __launch_bounds__(64 * GM_W) k_gram_mfma(const P* pack, int rows, int na, double scale, OutT* G,
                                                    int full) {
   using Op = GramMfma<P>;
   using acc_t = typename Op::acc_t;
@@ -173,36 +177,35 @@ __global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int 
   const int ti = (int)(t - (long long)tj * (tj + 1) / 2);
   const int i0 = ti * GM_T, j0 = tj * GM_T;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wi = wave >> 1, wj = wave & 1;
-  acc_t acc[2][2];
+  const int wi = (wave >> 1) * 16, wj = wave & 1;
+  acc_t acc[2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
-  // loader: row lr of a chunk, columns lc, lc + 16, ..; columns past na repeat
+  for (int b = 0; b < 2; ++b) acc[b] = acc_t{0, 0, 0, 0};
+  // loader: row lr of a chunk, columns lc, lc + LW, ..; columns past na repeat
   // the last one (their products are not written), rows past the end are zero
-  const int lr = tid >> 4, lc = tid & 15;
-  int ci[4], cj[4];
+  constexpr int LW = 4 * GM_W, NL = GM_T / LW;
+  const int lr = tid / LW, lc = tid % LW;
+  int ci[NL], cj[NL];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    ci[u] = min(i0 + lc + 16 * u, na - 1);
-    cj[u] = min(j0 + lc + 16 * u, na - 1);
+  for (int u = 0; u < NL; ++u) {
+    ci[u] = min(i0 + lc + LW * u, na - 1);
+    cj[u] = min(j0 + lc + LW * u, na - 1);
   }
-  P ra[GM_AHEAD][4], rb[GM_AHEAD][4];
-  auto load = [&](int r0, P (&a)[4], P (&b)[4]) __attribute__((always_inline)) {
+  P ra[GM_AHEAD][NL], rb[GM_AHEAD][NL];
+  auto load = [&](int r0, P (&a)[NL], P (&b)[NL]) __attribute__((always_inline)) {
     const P* row = pack + (size_t)min(r0 + lr, rows - 1) * na;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < NL; ++u) {
       a[u] = row[ci[u]];
       b[u] = row[cj[u]];
     }
   };
-  auto store = [&](int r0, int buf, const P (&a)[4], const P (&b)[4]) __attribute__((always_inline)) {
+  auto store = [&](int r0, int buf, const P (&a)[NL], const P (&b)[NL]) __attribute__((always_inline)) {
     const bool in = r0 + lr < rows;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      sA[buf][lr][lc + 16 * u] = in ? a[u] : (P)0;
-      sB[buf][lr][lc + 16 * u] = in ? b[u] : (P)0;
+    for (int u = 0; u < NL; ++u) {
+      sA[buf][lr][lc + LW * u] = in ? a[u] : (P)0;
+      sB[buf][lr][lc + LW * u] = in ? b[u] : (P)0;
     }
   };
   if (rows > 0) {
@@ -220,15 +223,12 @@ __global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int 
 #pragma unroll
         for (int k0 = 0; k0 < GM_KC; k0 += 4) {
           const int k = k0 + (lane >> 4), m = lane & 15;
-          P av[2], bv[2];
-#pragma unroll
-          for (int a = 0; a < 2; ++a) av[a] = sA[buf][k][32 * wi + 16 * a + m];
+          const P av = sA[buf][k][wi + m];
+          P bv[2];
 #pragma unroll
           for (int b = 0; b < 2; ++b) bv[b] = sB[buf][k][32 * wj + 16 * b + m];
 #pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = Op::op(av[a], bv[b], acc[a][b]);
+          for (int b = 0; b < 2; ++b) acc[b] = Op::op(av, bv[b], acc[b]);
         }
         // the other buffer was last read before the previous barrier
         const int nx = (u + 1) % GM_AHEAD;
@@ -237,19 +237,23 @@ __global__ void __launch_bounds__(256) k_gram_mfma(const P* pack, int rows, int 
       }
     }
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int b = 0; b < 2; ++b)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = i0 + 32 * wi + 16 * a + Op::row(lane, e);
-        const int j = j0 + 32 * wj + 16 * b + (lane & 15);
-        if (i < na && j < na) {
-          const OutT x = (OutT)(scale * (double)acc[a][b][e]);
-          G[i + (size_t)j * na] = x;
-          if (full && ti != tj) G[j + (size_t)i * na] = x;
-        }
+    for (int e = 0; e < 4; ++e) {
+      const int i = i0 + wi + Op::row(lane, e);
+      const int j = j0 + 32 * wj + 16 * b + (lane & 15);
+      if (i < na && j < na) {
+        const OutT x = (OutT)(scale * (double)acc[b][e]);
+        G[i + (size_t)j * na] = x;
+        if (full && ti != tj) G[j + (size_t)i * na] = x;
       }
+    }
+}
+
+template <class P, class OutT>
+inline void gram_launch(const P* pack, int rows, int na, double scale, OutT* G, int full, hipStream_t st) {
+  hipLaunchKernelGGL((k_gram_mfma<P, OutT>), dim3((unsigned)gm_tiles(na)), dim3(64 * GM_W), 0, st, pack, rows, na,
+                     scale, G, full);
 }
 
 // sr_s_g, centered() (stage_backend.rs:167-184): thread p < np forms the
