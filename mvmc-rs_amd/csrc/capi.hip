@@ -275,6 +275,12 @@ long long cg_solve_dev(int na, int W, int NS, const P* pack, const double* mean,
   const size_t lds = na <= CGT_NMAX ? sizeof(double) * na : 0;
   raise_lds_limit((const void*)k_cg_tail, sizeof(double) * CGT_NMAX);
   auto tail = [&](int stage, int j, int nsup) {
+    if (!gram && (long long)nsup * na >= CG_FOLD_MIN) {
+      hipLaunchKernelGGL(k_cg_fold2, dim3(nblk(na)), blk, 0, st, wk.spart, nsup, na, stage == 2 ? wk.x : wk.d, mean,
+                         diag, wk.sc + 5, inv_w, shift, stage == 2 ? wk.g : nullptr, stage == 2 ? wk.r : wk.q,
+                         wk.ctl);
+      nsup = -1;
+    }
     hipLaunchKernelGGL(k_cg_tail, dim3(1), dim3(CGT_NT), lds, st, stage, j, na, nsup, wk.spart, mean, diag, wk.g,
                        wk.sc + 5, inv_w, shift, pfac, diag_scale ? 1 : 0, max_it, threshold, wk.x, wk.r, wk.d, wk.q,
                        wk.prod, wk.sc, CG_PERIOD, wk.ctl);

@@ -2357,11 +2357,16 @@ __device__ inline void block_tree256x2(double& p0, double& p1, double* red) {
 // C = columns per lane (na <= 256*C).  P: element type of the packed samples
 // (double; float in the precision form, accumulated in FP64).  Bound by HBM
 // (the samples once per product), if the rows' dot chain does not hold the
-// loads up: two rows share a tree, and the next two rows' loads are in
-// flight meanwhile (8192 rows x 2099: 36 -> 27 us).
+// loads up.  Up to C = 16 two rows share a tree, and the next two rows' loads
+// are in flight meanwhile (8192 rows x 2099: 36 -> 27 us a product).  Above,
+// those rows take the registers of a second workgroup on the CU, and two
+// workgroups of one row each cover each other's chains better than one of two
+// rows does (an iteration at 16384 rows: 193 -> 180 us at na = 5000, 262 ->
+// 237 at 6500, 300 -> 268 at 7784; at 4090, C = 16, 146 against 148).
 template <int C, class P>
-__global__ void __launch_bounds__(256, C <= 16 ? 2 : 1) k_cg_chunk(const P* pack, int rows, int na, const double* x,
+__global__ void __launch_bounds__(256, 2) k_cg_chunk(const P* pack, int rows, int na, const double* x,
                                                   const double* mean, double* cpart, double* coef, const int* ctl) {
+  constexpr int U = C <= 16 ? 2 : 1;  // rows at a time
   if (ctl[CTL_DONE]) return;
   __shared__ double red[514];
   const int tid = threadIdx.x;
@@ -2375,16 +2380,16 @@ __global__ void __launch_bounds__(256, C <= 16 ? 2 : 1) k_cg_chunk(const P* pack
   const int r0 = b * CG_RCH, r1 = min(rows, r0 + CG_RCH);
   // one buffer resource per row: element i >= na reads 0 in hardware, so the
   // loads carry no branch and are all in flight before the first use
-  P raw[2][C];
+  P raw[U][C];
   auto load = [&](int r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       const RowBuf<P> row(pack + (size_t)min(r + u, r1 - 1) * na, na);
 #pragma unroll
       for (int k = 0; k < C; ++k) raw[u][k] = row.load(tid + 256 * k);
     }
   };
-  load(r0);
+  if (U == 2) load(r0);
   double xv[C], acc[C];
 #pragma unroll
   for (int k = 0; k < C; ++k) {
@@ -2392,25 +2397,27 @@ __global__ void __launch_bounds__(256, C <= 16 ? 2 : 1) k_cg_chunk(const P* pack
     xv[k] = i < na ? x[i] : 0.0;
     acc[k] = 0.0;
   }
-  for (int r = r0; r < r1; r += 2) {
-    double o[2][C];
+  for (int r = r0; r < r1; r += U) {
+    if (U == 1) load(r);
+    double o[U][C];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int k = 0; k < C; ++k) o[u][k] = (double)raw[u][k];
-    load(min(r + 2, r1 - 1));
-    double p[2] = {0.0, 0.0};
+    if (U == 2) load(min(r + 2, r1 - 1));
+    double p[U] = {};
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int k = 0; k < C; ++k)
         if (tid + 256 * k < na) p[u] += o[u][k] * xv[k];
-    block_tree256x2(p[0], p[1], red);
+    if constexpr (U == 2) block_tree256x2(p[0], p[1], red);
+    else p[0] = block_tree256(p[0], red);
 #pragma unroll
     for (int k = 0; k < C; ++k)
       if (tid + 256 * k < na) {
         acc[k] += o[0][k] * p[0];
-        if (r + 1 < r1) acc[k] += o[1][k] * p[1];
+        if (U == 2 && r + 1 < r1) acc[k] += o[U - 1][k] * p[U - 1];
       }
   }
 #pragma unroll

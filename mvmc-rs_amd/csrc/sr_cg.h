@@ -23,6 +23,13 @@ constexpr int CGS_M = 10;                 // columns per lane of k_cg_small: na 
 constexpr long long CGS_ELEMS = 160 * 1024;
 constexpr int CGT_NT = 1024;              // threads of k_cg_tail
 constexpr int CGT_NMAX = 8000;            // na up to which k_cg_tail keeps products in LDS
+// Superchunk partials from which their fold is a launch over all CUs instead
+// of k_cg_tail's one: a launch costs 1 us more than the fold it replaces at
+// 4000 partials (na = 1000, 2048 rows: 33.4 us an iteration in the tail, 34.5
+// apart), as much at 8000 (4000 x 600: 59.0 and 58.8), and the tail's CU
+// reads the rest at its own rate (7784 x 512: 99.8 and 96.6, 4000 x 8192: 81
+// and 75, 7784 x 16384: 268 and 239).
+constexpr long long CG_FOLD_MIN = 8000;
 
 // LDS doubles of k_cg_small: x, r, d, q, mean, diag, g, the chunk partials
 // and the reduction buffers.
@@ -360,10 +367,12 @@ __global__ void __launch_bounds__(256) k_gram_product(const float* G, int na, co
 //      the head of the next iteration
 //   1  (before a residual refresh) q = z, alpha, x += alpha d
 //   2  (after it) r = g - z, beta, d, the next head
-// (a Gram product is one superchunk).  The products of a dot are formed by
-// all threads and summed in its order by 256 (in LDS, or in `prod` past
-// CGT_NMAX).  The guards and their statuses are those of k_cg_alpha / k_cg_beta /
-// k_cg_head; ctl[CTL_ITER] + j is the iteration.
+// (a Gram product is one superchunk).  nsup < 0: the fold went before, in a
+// launch of its own, with z in q (stage 2: g - z in r).  The products of a dot
+// are formed by all threads and summed in its order by 256 (in LDS, or in
+// `prod` past CGT_NMAX).  Guards: a d.q or r.src that is not finite, a d.q or
+// delta below 1e-20 in magnitude, an alpha or beta that is not finite end the
+// solve with status -(iteration + 1); ctl[CTL_ITER] + j is the iteration.
 __global__ void __launch_bounds__(CGT_NT) k_cg_tail(int stage, int j, int na, int nsup, const double* spart,
                                                     const double* mean, const double* diag, const double* g,
                                                     double* coef, double inv_w, double shift, double pfac,
@@ -377,18 +386,23 @@ __global__ void __launch_bounds__(CGT_NT) k_cg_tail(int stage, int j, int na, in
   const int tid = threadIdx.x;
   const int iter = ctl[CTL_ITER] + j;
   const double* v = stage == 2 ? x : d;
-  const double cf = coef[0];
-  for (int i = tid; i < na; i += CGT_NT) {
-    double tot = nsup > 0 ? spart[i] : 0.0;
+  if (nsup >= 0) {
+    const double cf = coef[0];
+    for (int i = tid; i < na; i += CGT_NT) {
+      double tot = nsup > 0 ? spart[i] : 0.0;
 #pragma unroll 4
-    for (int s = 1; s < nsup; ++s) tot += spart[(size_t)s * na + i];
-    const double z = inv_w * tot - cf * mean[i] + shift * diag[i] * v[i];
-    if (stage == 2) {
-      r[i] = g[i] - z;
-    } else {
-      q[i] = z;
-      cgt_prod[i] = d[i] * z;
+      for (int s = 1; s < nsup; ++s) tot += spart[(size_t)s * na + i];
+      const double z = inv_w * tot - cf * mean[i] + shift * diag[i] * v[i];
+      if (stage == 2) {
+        r[i] = g[i] - z;
+      } else {
+        q[i] = z;
+        cgt_prod[i] = d[i] * z;
+      }
     }
+  } else if (stage != 2) {
+#pragma unroll 4
+    for (int i = tid; i < na; i += CGT_NT) cgt_prod[i] = d[i] * q[i];
   }
   __syncthreads();
   if (stage != 2) {
