@@ -186,13 +186,15 @@ void cg_small(const P* op, int rows, int na, const double* mean, const double* d
     hipLaunchKernelGGL((k_cg_small<M, GRAM, P>), dim3(1), dim3(CGS_NT), lds, st, op, rows, na, mean, diag, g, inv_w,
                        shift, threshold, pfac, max_it, diag_scale, x, ctl);
   };
-  const int m = (na + 63) / 64;
-  if (m <= 1) go.template operator()<1>();
-  else if (m <= 2) go.template operator()<2>();
-  else if (m <= 3) go.template operator()<3>();
-  else if (m <= 5) go.template operator()<5>();
-  else if (m <= 7) go.template operator()<7>();
-  else go.template operator()<CGS_M>();
+  switch (cgs_columns(na)) {
+    case 1: go.template operator()<1>(); break;
+    case 2: go.template operator()<2>(); break;
+    case 3: go.template operator()<3>(); break;
+    case 5: go.template operator()<5>(); break;
+    case 7: go.template operator()<7>(); break;
+    default:  // samples only: a Gram of that order is past CGS_ELEMS
+      if constexpr (!GRAM) go.template operator()<CGS_M>();
+  }
   HIPCHK(hipGetLastError());
 }
 
@@ -209,13 +211,12 @@ long long cg_status(CgWork& wk, hipStream_t st) {
 }
 
 // Issues the solve if one launch does it (x_out and wk.ctl hold its result
-// when the stream gets there); false otherwise.
+// when the stream gets there), beside `side` - 1 others; false otherwise.
 template <class P>
 bool cg_issue_small(int na, int rows, const P* pack, const double* mean, const double* diag, const double* g,
                     double inv_w, double shift, double tol, int max_it, bool diag_scale, double* x_out, CgWork& wk,
-                    hipStream_t st, const float* gram) {
-  const long long elems = (long long)na * (gram ? na : rows);
-  if (na > 64 * CGS_M || rows <= 0 || elems > CGS_ELEMS) return false;
+                    hipStream_t st, const float* gram, int side = 1) {
+  if (!cgs_takes(na, rows, gram != nullptr, side)) return false;
   wk.ensure(na, rows);
   const auto [threshold, pfac] = cg_limits(na, tol, shift);
   if (gram)
@@ -229,7 +230,7 @@ bool cg_issue_small(int na, int rows, const P* pack, const double* mean, const d
 }
 
 // C 1.4.0 StochasticOptCG_Main / PreconCG_DiagScale (sr_cg.rs:700-880).
-// Operators that one CU streams fast enough (CGS_ELEMS) are solved by one
+// Operators that one CU streams fast enough (cgs_takes) are solved by one
 // launch.  Otherwise an iteration is its product (chunk partials and their
 // first fold, or the Gram's rows) and k_cg_tail, issued a residual-refresh
 // period at a time; a done flag set by the guards turns the rest into
@@ -1361,7 +1362,7 @@ int sr_max_it(const mvmc_ens* E, int na) {
 // The SR-CG solve of a run that one launch does, issued ahead of sr_impl: the
 // runs of a group have a stream each, and their one-workgroup solves run side
 // by side (4 runs of 2.3 .. 14.7 ms: 28 -> 15 ms).
-void sr_issue(mvmc_ens* E) {
+void sr_issue(mvmc_ens* E, int runs) {
   const mvmc::Model& m = E->m;
   if (m.mp.nsrcg == 0) return;
   auto job = sr_prepare(E, false);
@@ -1371,7 +1372,7 @@ void sr_issue(mvmc_ens* E) {
     auto issue = [&](auto* pack) {
       return cg_issue_small(na, E->v.W * E->v.nsample, pack, E->d_cmean, E->d_cdiag, E->d_cg, inv_w,
                             m.mp.dsr_opt_sta_del, m.mp.dsr_opt_cg_tol, sr_max_it(E, na), m.mp.use_diag_scale != 0,
-                            E->d_cx, E->cg, E->st, job->gram);
+                            E->d_cx, E->cg, E->st, job->gram, runs);
     };
     job->issued = E->precision == 1 ? issue((const float*)E->d_pack) : issue((const double*)E->d_pack);
     if (job->issued) HIPCHK(hipEventRecord(job->c1, E->st));
@@ -2500,7 +2501,7 @@ int mvmc_group_opt_step(mvmc_group* g, double* rows) {
     for (mvmc_ens* e : g->runs) {
       // what a run's preparation throws is thrown in its own turn, below
       try {
-        sr_issue(e);
+        sr_issue(e, (int)g->runs.size());
       } catch (const Fail&) {
         e->job.reset();
       }

@@ -2,7 +2,7 @@
 // arithmetic and the reduction order of the k_cg_* kernels of ensemble.hip,
 // element by element):
 //   k_cg_small   the whole solve in one workgroup, for operators that its CU
-//                streams from L2 faster than a launch takes
+//                streams from L2 faster than an iteration's launches take
 //   k_cg_tail    everything of an iteration after the chunk partials' first
 //                fold, in one workgroup
 // What bounds the solver is not arithmetic: an iteration is 8 dependent
@@ -17,10 +17,26 @@ namespace mvmc_hip {
 constexpr int CGS_WAVES = 8;              // waves of k_cg_small
 constexpr int CGS_NT = 64 * CGS_WAVES;
 constexpr int CGS_M = 10;                 // columns per lane of k_cg_small: na <= 640
-// Elements of the operator (samples or Gram) k_cg_small takes: its CU streams
-// 64 bytes a cycle, so 160 k doubles are about 10 us an iteration, what the
-// launches of one iteration take otherwise.
+// Operators that k_cg_small takes.  A wave takes a chunk of 32 rows at a time
+// (CGS_WAVES chunks a round), at a cost per round of about a fixed part and a
+// part per column of the lane, while an iteration of launches takes 23 .. 30 us
+// whatever the size in this range.  So the line lies at rounds x (columns per
+// lane + 2) = CGS_COST (us an iteration, one launch / launches):
+//   columns   up to the line          behind it
+//        64   1280 rows 22.2 / 26.1   2560 rows 41.9 / 26.8
+//       100    800 rows 19.7 / 26.4   1600 rows 35.7 / 26.8
+//       200    400 rows 19.8 / 25.7    800 rows 36.2 / 26.7
+//       400    200 rows 15.8 / 25.2    400 rows 27.1 / 26.6
+//       500    160 rows 19.0 / 24.5    320 rows 29.9 / 26.2
+//       595    256 rows 24.7 / 30.5
+// (20 x 8192 in one launch took 73 us, in launches 25).  Solves that run side
+// by side cost the longest of them in one launch each and their sum in
+// launches, which moves the line by their number.
+// A Gram of FP32 has half the bytes and no second pass: 271 columns 8.7 us
+// against 15.0, 421 columns 15.3 against 13.8.  CGS_ELEMS is its line (404
+// columns) and, for samples, what keeps the chunk partials in LDS.
 constexpr long long CGS_ELEMS = 160 * 1024;
+constexpr long long CGS_COST = 16;
 constexpr int CGT_NT = 1024;              // threads of k_cg_tail
 constexpr int CGT_NMAX = 8000;            // na up to which k_cg_tail keeps products in LDS
 // Superchunk partials from which their fold is a launch over all CUs instead
@@ -36,6 +52,19 @@ constexpr long long CG_FOLD_MIN = 8000;
 __host__ __device__ inline size_t cgs_lds_doubles(int na, int rows, bool gram) {
   const size_t nch = gram ? 0 : (size_t)(rows + CG_RCH - 1) / CG_RCH;
   return 7 * (size_t)na + nch * na + 8;
+}
+
+// Columns per lane of the k_cg_small instance for na columns.
+__host__ __device__ constexpr int cgs_columns(int na) {
+  const int m = (na + 63) / 64;
+  return m <= 3 ? m : m <= 5 ? 5 : m <= 7 ? 7 : CGS_M;
+}
+
+// Whether one launch solves it, beside `side` - 1 other solves.
+inline bool cgs_takes(int na, int rows, bool gram, int side) {
+  if (na > 64 * CGS_M || rows <= 0 || (long long)na * (gram ? na : rows) > CGS_ELEMS) return false;
+  const long long rounds = ((rows + CG_RCH - 1) / CG_RCH + CGS_WAVES - 1) / CGS_WAVES;
+  return gram || rounds * (cgs_columns(na) + 2) <= CGS_COST * side;
 }
 
 // Exchanges between the halves of a wave (and between odd and even rows of 16

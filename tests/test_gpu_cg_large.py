@@ -1,5 +1,5 @@
 """SR-CG of operators past one launch, whole solves against the oracle bit for
-bit: several superchunks of rows, their fold in the tail (up to 8000 partials)
+bit: the first sizes past that line, several superchunks of rows, their fold in the tail (up to 8000 partials)
 and apart, the column counts per lane of the chunk pass (two rows at a time up
 to 4096 columns, one above, the wide form past 8192), the dot products past
 the tail's LDS (8000); iteration limits on both sides of a residual refresh."""
@@ -21,7 +21,8 @@ def M():
 
 
 @pytest.mark.parametrize("variant", [0, 1])
-@pytest.mark.parametrize("na,rows", [(642, 40), (700, 1100), (1999, 2048), (2000, 2048), (2500, 600), (4096, 545),
+@pytest.mark.parametrize("na,rows", [(20, 8192), (64, 1281), (128, 1025), (192, 769), (320, 513), (448, 257),
+                                     (640, 257), (642, 40), (700, 1100), (1999, 2048), (2000, 2048), (2500, 600), (4096, 545),
                                      (4097, 513), (6144, 70), (6145, 33), (8000, 40), (8001, 70), (8193, 35)])
 def test_solve_matches_oracle(M, na, rows, variant):
     import torch
