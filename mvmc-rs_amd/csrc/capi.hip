@@ -216,7 +216,8 @@ template <class P>
 bool cg_issue_small(int na, int rows, const P* pack, const double* mean, const double* diag, const double* g,
                     double inv_w, double shift, double tol, int max_it, bool diag_scale, double* x_out, CgWork& wk,
                     hipStream_t st, const float* gram, int side = 1) {
-  if (!cgs_takes(na, rows, gram != nullptr, side)) return false;
+  // (a negative limit is refused by the general form, which no period of iterations ends)
+  if (max_it < 0 || !cgs_takes(na, rows, gram != nullptr, side)) return false;
   wk.ensure(na, rows);
   const auto [threshold, pfac] = cg_limits(na, tol, shift);
   if (gram)

@@ -39,3 +39,13 @@ def test_solve_matches_oracle(M, na, rows, variant):
         sto, xo, _, _ = O.cg_solve(mean, diag, o, g, 1.0 / rows, 1e-2, 1e-9, limit, bool(variant))
         assert st == sto
         assert np.array_equal(x.cpu().numpy(), xo)
+
+
+@pytest.mark.parametrize("na,rows", [(8, 32), (700, 64)])
+def test_negative_iteration_limit_is_refused(M, na, rows):
+    import torch
+    print(f"cg na={na} rows={rows} limit -1", flush=True)
+    o = torch.randn(rows, na, dtype=torch.float64, device="cuda")
+    v = torch.ones(na, dtype=torch.float64, device="cuda")
+    with pytest.raises(M.BackendError):
+        M.sr_cg_solve(o, v, v, v, torch.zeros_like(v), na, 1, rows, 1.0 / rows, 1e-2, 1e-9, -1, 0)
