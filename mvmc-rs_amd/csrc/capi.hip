@@ -1388,6 +1388,7 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
   EnsView& v = E->v;
   const double t0 = now_s();
   std::shared_ptr<SrJob> job = std::move(E->job);
+  const bool ahead = job != nullptr;
   if (!job) job = sr_prepare(E, force_direct);
   const std::vector<int>& map = job->map;
   E->cg_x.clear();
@@ -1407,6 +1408,8 @@ int sr_impl(mvmc_ens* E, long long* info_out, bool force_direct = false) {
                : cg_solve_dev(na, v.W, v.nsample, (const double*)E->d_pack, E->d_cmean, E->d_cdiag, E->d_cg, inv_w,
                               m.mp.dsr_opt_sta_del, m.mp.dsr_opt_cg_tol, max_it, dscale, E->d_cx, E->cg, st);
   };
+  // prepared ahead, but solved now: other runs' solves may lie between
+  if (ahead && !job->issued) HIPCHK(hipEventRecord(c0, st));
   long long status = job->issued ? cg_status(E->cg, st) : solve(m.mp.use_diag_scale != 0);
   if (!job->issued) HIPCHK(hipEventRecord(c1, st));
   HIPCHK(hipEventSynchronize(c1));
