@@ -215,6 +215,12 @@ __device__ __forceinline__ void rr_pfinv(const Ar& ar, Src src, int n, typename 
   constexpr int NS = FULL ? R * R : R * (R + 1) / 2;
   constexpr int NT = T * T, VL = rr_vl(T, R), LDB = rr_ldb(T, R), SETS = rr_sets(T), Q = VL / 64;
   constexpr int JC = (T * R + NT - 1) / NT;  // columns per thread where a thread owns whole columns
+  // Complex planes of 10 blocks a side fill 220 of a thread's 512 registers
+  // with slots; with a step's x and y of all rows beside them the kernel
+  // spilled 513 (n = 152, 256 planes: 2064 us, where 1024 threads a plane had
+  // taken 1480).  There the update goes by groups of RG block rows: 1385 us.
+  constexpr bool TIGHT = sizeof(S) == 16 && R >= 10;
+  constexpr int RG = 4;
   const int tid = threadIdx.x, lane = tid & 63;
   const int a0 = tid % T, b0 = tid / T;
   // copies of (a, b) the compiler cannot prove loop-invariant: the index
@@ -405,6 +411,7 @@ RR_FOR(cj, P, R) {
     }
     RR_PHASE(3);
     rr_case<0, R>(K0, [&]<int K>() RR_INLINE {
+      if constexpr (!TIGHT) {
       S xi[K + 1], yi[K + 1];
 RR_FOR(ri, 0, K + 1) {
         xi[ri] = xs[a + T * ri];
@@ -446,6 +453,52 @@ RR_FOR(ri, 0, K + 1) {
             if (ri < K || a < kb) RC(ri, K + 1) = ar.scale(xi[ri], alpha);
           };
         }
+      }
+      } else {
+        // the same by groups of RG block rows
+        RR_FOR(h, 0, (K + RG) / RG) {
+          constexpr int R0 = h * RG, R1 = R0 + RG < K + 1 ? R0 + RG : K + 1;
+          S xi[R1 - R0], yi[R1 - R0];
+          RR_FOR(ri, R0, R1) {
+            xi[ri - R0] = xs[a + T * ri];
+            yi[ri - R0] = yn[a + T * ri];
+          };
+          if (kpc != kk0) {
+            if (b == kb) {
+              RR_FOR(ri, R0, R1) {
+                if (ri < K || a < kb) RC(ri, K) = yi[ri - R0];
+              };
+            }
+            if (R1 == K + 1 && a == kb) {
+              RR_FOR(cj, K, R) {
+                if (cj > K || b > kb) RC(K, cj) = r1[b + T * cj];
+              };
+            }
+          }
+          RR_FOR(cj, R0, K + 1) {
+            const S yj = yn[b + T * cj], xj = xs[b + T * cj];
+            const S t1 = Ar::mul(alpha, yj), t2 = Ar::mul(alpha, xj);
+            if (cj < K || b < kb) {
+              RR_FOR(ri, R0, (cj + 1 < R1 ? cj + 1 : R1)) {
+                RC(ri, cj) = Ar::update(RC(ri, cj), xi[ri - R0], yi[ri - R0], t1, t2);
+              };
+            }
+          };
+          if (kb + 1 < T) {
+            if (b == kb + 1) {
+              RR_FOR(ri, R0, R1) {
+                if (ri < K || a < kb) RC(ri, K) = ar.scale(xi[ri - R0], alpha);
+              };
+            }
+            RR_APART(K + 100 + 1000 * h);
+          } else if constexpr (K + 1 < R) {
+            if (b == 0) {
+              RR_FOR(ri, R0, R1) {
+                if (ri < K || a < kb) RC(ri, K + 1) = ar.scale(xi[ri - R0], alpha);
+              };
+            }
+          }
+        };
       }
     });
     RR_PHASE(4);
