@@ -355,8 +355,7 @@ __device__ __forceinline__ void wg_pfinv(double* planes, double* work, int n, in
       }
     }
     PF_FRESH();
-    if (tid < np) {
-      const int p = tid;
+    for (int p = tid; p < np; p += nthr) {
       if (sh.colmax[p] == 0.0) {
         if (sh.info[p] == 0) sh.info[p] = kk0 + 1;
         sh.P(p, kk0) = kk0 + 1;
@@ -512,8 +511,7 @@ __device__ __forceinline__ void wg_pfinv(double* planes, double* work, int n, in
   __syncthreads();
   PF_FRESH();
   // ---------------- Pfaffian (utu2pfa) ----------------
-  if (tid < np) {
-    const int p = tid;
+  for (int p = tid; p < np; p += nthr) {
     if (sh.info[p] == 0) {
       const double* a = planes + (size_t)p * nn;
       double v = 1.0;
@@ -783,8 +781,7 @@ __device__ __forceinline__ void wg_pfinv(double* planes, double* work, int n, in
   // j ascending) compose into one index map g, applied to rows and columns
   // as a gather (pure data movement), then the sign (calc_m_all's final
   // DSCAL by -1).  g lives in ks, the gather goes through `work`.
-  if (tid < np) {
-    const int p = tid;
+  for (int p = tid; p < np; p += nthr) {
     int* g = &sh.KS(p, 0);
     for (int k = 0; k < n; ++k) g[k] = k;
     for (int j = 0; j < n; ++j) {
