@@ -365,8 +365,8 @@ RrPlan rr_plan(int n, bool cplx) {
     q.threads = 256;
     q.kernel = cplx ? rr_kernel_c128_large(r16) : r16 <= 10 ? rr_kernel_large(r16) : rr_kernel_huge(r16);
     q.lds = rnd16((size_t)n * 4) +
-            (cplx ? rr_lds_bytes<cz, true>(16, r16, false, n) : rr_lds_bytes<double, false>(16, r16, false, n));
-    q.scratch = rr_scratch_len(false, n) * (cplx ? sizeof(cz) : sizeof(double));
+            (cplx ? rr_lds_bytes<cz, true>(16, r16, n) : rr_lds_bytes<double, false>(16, r16, n));
+    q.scratch = rr_scratch_len(n) * (cplx ? sizeof(cz) : sizeof(double));
   }
   if (!q.kernel) throw Fail(MVMC_E_INVALID_SHAPE, "no Pfaffian kernel for n = " + std::to_string(n));
   int ncu = 0, occ = 0;

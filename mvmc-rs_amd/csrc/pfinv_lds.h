@@ -440,7 +440,7 @@ __device__ __forceinline__ void lp_pfinv(const Ar& ar, Src src, int n, typename 
   RR_FOR(g, 0, G) {
     constexpr int C0 = g * HC, C1 = C0 + HC < R ? C0 + HC : R;
     S c[FULL ? R * HC : R * (R + 1) / 2];
-#define RC(ri, cj) c[FULL ? (ri) * HC + (cj) - C0 : rr_slot<R, false>(ri, cj)]
+#define RC(ri, cj) c[FULL ? (ri) * HC + (cj) - C0 : rr_slot<R>(ri, cj)]
     RR_FRESH();
     RR_FOR(ri, 0, R) {
       RR_FOR(cj, FULL ? C0 : ri, C1) {

@@ -33,11 +33,11 @@
 namespace mvmc_hip {
 
 constexpr int RR_NMAX = 224;  // largest n
-constexpr int RR_NFULL = 64;  // largest n of the full form (utu2inv's small-matrix path)
+constexpr int RR_NFULL = 64;  // largest n of utu2inv's small-matrix path (pfinv_lds.h)
 
 // Orders the LDS traffic of the T x T workgroup: a barrier, or for the
-// single wave of T = 8, whose LDS operations complete in order, only a fence
-// for the compiler.
+// single wave of T = 8 (pfinv_lds.h), whose LDS operations complete in order,
+// only a fence for the compiler.
 template <int T>
 __device__ __forceinline__ void rr_sync() {
   if constexpr (T == 8) {
@@ -100,29 +100,24 @@ __device__ __forceinline__ double rr_wave_max(double x) {
                           __builtin_amdgcn_readlane(__double2loint(x), 63));
 }
 
-// LDS of one plane.  `vec`: the step vectors (two sets by step parity when
-// several waves share the plane: a fast wave may write the next step's while
-// a slow one still reads this step's), reused as the row blocks of the solve
-// (full form), of the product and of the output.
+// LDS of one plane.  `vec`: the step vectors (two sets by step parity: a fast
+// wave may write the next step's while a slow one still reads this step's),
+// reused as the row blocks of the product and of the output.
 constexpr int rr_vl(int T, int R) { return (T * R + 63) / 64 * 64; }  // padded vector length
-constexpr int rr_sets(int T) { return T == 8 ? 1 : 2; }
 // row stride of the T-row blocks: T lanes of a row beside the next row's
 constexpr int rr_ldb(int T, int R) { return rr_vl(T, R) + T; }
 // scalars of `vec`: 2 y columns, then per set x, u, r1, r2
-constexpr int rr_vec_len(int T, int R, bool FULL) {
-  const int step = (2 + 4 * rr_sets(T)) * rr_vl(T, R);
-  const int blocks = (FULL ? 1 : 2) * T * rr_ldb(T, R);
+constexpr int rr_vec_len(int T, int R) {
+  const int step = 10 * rr_vl(T, R);
+  const int blocks = 2 * T * rr_ldb(T, R);
   return step > blocks ? step : blocks;
 }
-// packed strict upper triangle of M, columns up to n - 2 (full form)
-__host__ __device__ constexpr int rr_m_len(int n) { return n > 2 ? (n - 1) * (n - 2) / 2 : 0; }
 
 template <class S>
 struct RrLdsT {
   S* vec;
   S* sup;          // the superdiagonal A(i, i+1) after the LTL
   S *rneg, *rpos;  // complex solve: reciprocals of -vt[i] and vt[i]
-  S* m;            // full form: M packed
   S* sa;           // [1] the Pfaffian
   int* finv;       // inverse of the output permutation
   double* sd;      // [16] max |a|^2 per wave
@@ -130,35 +125,32 @@ struct RrLdsT {
 using RrLds = RrLdsT<double>;
 
 template <class S, bool RECIP>
-__host__ __device__ inline size_t rr_lds_bytes(int T, int R, bool full, int n) {
+__host__ __device__ inline size_t rr_lds_bytes(int T, int R, int n) {
   const int nw = T * T / 64;
-  return rnd16((size_t)rr_vec_len(T, R, full) * sizeof(S)) + rnd16((size_t)n * sizeof(S)) * (RECIP ? 3 : 1) +
-         (full ? rnd16((size_t)rr_m_len(n) * sizeof(S)) : 0) + 16 + rnd16((size_t)n * 4) + rnd16((size_t)nw * 8);
+  return rnd16((size_t)rr_vec_len(T, R) * sizeof(S)) + rnd16((size_t)n * sizeof(S)) * (RECIP ? 3 : 1) + 16 +
+         rnd16((size_t)n * 4) + rnd16((size_t)nw * 8);
 }
 
-template <class S, bool RECIP, int T, int R, bool FULL, class Carver>
+template <class S, bool RECIP, int T, int R, class Carver>
 __device__ inline RrLdsT<S> carve_rr(Carver& c, int n) {
   RrLdsT<S> L;
-  L.vec = c.template take<S>(rr_vec_len(T, R, FULL));
+  L.vec = c.template take<S>(rr_vec_len(T, R));
   L.sup = c.template take<S>(n);
   L.rneg = RECIP ? c.template take<S>(n) : nullptr;
   L.rpos = RECIP ? c.template take<S>(n) : nullptr;
-  L.m = FULL ? c.template take<S>(rr_m_len(n)) : nullptr;
   L.sa = c.template take<S>(1);
   L.finv = c.template take<int>(n);
   L.sd = c.template take<double>(T * T / 64);
   return L;
 }
 
-// Scratch in global memory per workgroup, in scalars: M and C of the panel
-// form; the full form needs none.
-__host__ __device__ inline size_t rr_scratch_len(bool full, int n) { return full ? 0 : (size_t)2 * n * n; }
+// Scratch in global memory per workgroup, in scalars: M and C.
+__host__ __device__ inline size_t rr_scratch_len(int n) { return (size_t)2 * n * n; }
 
-// Slot of block (ri, cj): packed upper block triangle (cj >= ri) in the
-// panel form, row-major R x R in the full form.
-template <int R, bool FULL>
+// Slot of block (ri, cj) of the packed upper block triangle (cj >= ri).
+template <int R>
 __host__ __device__ constexpr int rr_slot(int ri, int cj) {
-  return FULL ? ri * R + cj : ri * R - ri * (ri - 1) / 2 + (cj - ri);
+  return ri * R - ri * (ri - 1) / 2 + (cj - ri);
 }
 
 // C IDAMAX order of the pivot search: first index of the largest |x|; a NaN
@@ -205,15 +197,14 @@ struct RrReal {
 // max |a|^2 < 1e-28 over the whole plane, in which case nothing else is
 // done.  gs: rr_scratch_len scalars of global scratch.  Every thread of the
 // T x T workgroup (blockDim.x == T * T) calls it; the results are uniform.
-// FULL: the full form (n <= 64), else the panel form (n > 64).
 // T (R - 1) < n <= T R.
-template <int T, int R, bool FULL, class Ar, class Src>
+template <int T, int R, class Ar, class Src>
 __device__ __forceinline__ void rr_pfinv(const Ar& ar, Src src, int n, typename Ar::S* out, float* out32, double sign,
                                          typename Ar::S* gs, RrLdsT<typename Ar::S>& L, typename Ar::S& pf, int& info,
                                          bool check_zero, bool& allzero) {
   using S = typename Ar::S;
-  constexpr int NS = FULL ? R * R : R * (R + 1) / 2;
-  constexpr int NT = T * T, VL = rr_vl(T, R), LDB = rr_ldb(T, R), SETS = rr_sets(T), Q = VL / 64;
+  constexpr int NS = R * (R + 1) / 2;
+  constexpr int NT = T * T, VL = rr_vl(T, R), LDB = rr_ldb(T, R), Q = VL / 64;
   constexpr int JC = (T * R + NT - 1) / NT;  // columns per thread where a thread owns whole columns
   // Complex planes of 10 blocks a side fill 220 of a thread's 512 registers
   // with slots; with a step's x and y of all rows beside them the kernel
@@ -234,7 +225,7 @@ __device__ __forceinline__ void rr_pfinv(const Ar& ar, Src src, int n, typename 
     asm volatile("" : "+v"(a), "+v"(b)); \
   } while (0)
   S c[NS];
-#define RC(ri, cj) c[rr_slot<R, FULL>(ri, cj)]
+#define RC(ri, cj) c[rr_slot<R>(ri, cj)]
 #ifdef MVMC_PHASE_CLOCKS
   long long rr_t0 = __builtin_readcyclecounter(), rr_ph[12] = {};
 #define RR_PHASE(k)                                         \
@@ -251,10 +242,10 @@ __device__ __forceinline__ void rr_pfinv(const Ar& ar, Src src, int n, typename 
   // ---- gather (and the all-zero guard, pfaffian.rs:884-890: the plane is skew, so the upper half decides) ----
   double mx = 0.0;
 RR_FOR(ri, 0, R) {
-RR_FOR(cj, FULL ? 0 : ri, R) {
+RR_FOR(cj, ri, R) {
       const int i = a + T * ri, j = b + T * cj;
       S x = Ar::zero();
-      if (cj >= ri && i < n && j < n && i <= j) {
+      if (i < n && j < n && i <= j) {
         x = src(i, j);
         mx = fmax(mx, Ar::mag2(x));
       }
@@ -274,7 +265,7 @@ RR_FOR(cj, FULL ? 0 : ri, R) {
     allzero = false;
   }
   S* const y0 = L.vec;
-  auto setv = [&](int par, int k) { return L.vec + (2 + (SETS == 2 ? 4 * par : 0) + k) * VL; };
+  auto setv = [&](int par, int k) { return L.vec + (2 + 4 * par + k) * VL; };
 
   RR_PHASE(0);
   // ---- dsktf2: k0 = n-1 .. 1 ----
@@ -542,8 +533,7 @@ RR_FOR(ri, 0, K + 1) {
     if (tid + NT * u < n) L.finv[f[u]] = tid + NT * u;
 
   RR_PHASE(5);
-  // ---- utu2inv (panel path for n > 64; the full form differs from the
-  // solve on) ----
+  // ---- utu2inv (its panel path, n > 64) ----
   // trtri('U','U') on B(i, j) = A(i, j+1), 0 <= i < j <= n-2: at step k the
   // column k of the inverse is final (Bn(i, k) = -acc(i, k), i < k) and
   // every acc(i, j), i < k < j, adds Bn(i, k) B(k, j) with row k of B still
@@ -596,8 +586,7 @@ RR_FOR(ri, 0, K) { RC(ri, cj) = Ar::add(RC(ri, cj), Ar::mul(ui[ri], bj));
   }
   RR_PHASE(6);
   // M (unit upper, M(i, j) = Bn(i, j) for i < j <= n-2, M(i, n-1) = 0 for
-  // i < n-1): packed in LDS (full form) or row-major in gs
-  auto mrow = [&](int i) { return i * (n - 2) - i * (i - 1) / 2 - i - 1; };  // packed: element (i, m) at mrow(i) + m
+  // i < n-1), row-major in gs
   S* gm = gs;
   S* gc = gs + (size_t)n * n;
   RR_FRESH();
@@ -605,8 +594,7 @@ RR_FOR(ri, 0, R) {
 RR_FOR(cj, ri, R) {
       const int i = a + T * ri, jj = b + T * cj;
       if (i + 1 < jj && jj < n) {
-        if constexpr (FULL) L.m[mrow(i) + jj - 1] = RC(ri, cj);
-        else gm[(size_t)i * n + (jj - 1)] = RC(ri, cj);
+        gm[(size_t)i * n + (jj - 1)] = RC(ri, cj);
       }
     };
   };
@@ -614,8 +602,7 @@ RR_FOR(cj, ri, R) {
   auto mval = [&](int i, int j) RR_INLINE -> S {  // M(i, j), j < n
     if (j <= i) return j == i ? Ar::one() : Ar::zero();
     if (j == n - 1) return Ar::zero();
-    if constexpr (FULL) return L.m[mrow(i) + j];
-    else return gm[(size_t)i * n + j];
+    return gm[(size_t)i * n + j];
   };
   RR_PHASE(7);
   // skew-tridiagonal solve T C = M (vt[i] = -A(i, i+1) = -sup[i]), a thread
@@ -623,214 +610,118 @@ RR_FOR(cj, ri, R) {
   //   forward   C(1) = M(0) / -vt[0]; C(i+1) = (M(i) - C(i-1) vt[i-1]) / -vt[i], i even
   //   backward  C(n-2) = M(n-1) / vt[n-2]; C(i-1) = (M(i) + C(i+1) vt[i]) / vt[i-1], i odd descending
   // The forward chain fills the odd rows of C, the backward one the even
-  // rows.  Full form: through a T-row LDS block into the registers (M is in
-  // LDS).  Panel form: the upper part to gc row-major, M read ahead.
-  if constexpr (FULL) {
-    S* cb = L.vec;
-    const int j = tid;
-    S prev = Ar::zero();
+  // rows: the upper part to gc row-major, M read ahead.
 #pragma unroll 1
-    for (int blk = 0; blk < R; ++blk) {
-      if (j < n) {
-#pragma unroll 4
-        for (int i = T * blk; i < T * blk + T; i += 2)
-          if (i < n) {
-            const S vti = Ar::neg(L.sup[i]);
-            S num = mval(i, j);
-            if (i > 0) num = Ar::sub(num, Ar::mul(prev, Ar::neg(L.sup[i - 1])));
-            prev = Ar::div_negvt(num, vti, Ar::kRecip ? L.rneg[i] : vti);
-            cb[(i + 1 - T * blk) * LDB + j] = prev;
-          }
-      }
-      rr_sync<T>();
-      RR_FRESH();
-      if (a & 1)
-        rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
-RR_FOR(cj, 0, R) { RC(K, cj) = cb[a * LDB + b + T * cj];
-          };
-        });
-      rr_sync<T>();
-    }
-#pragma unroll 1
-    for (int blk = R - 1; blk >= 0; --blk) {
-      if (j < n) {
-#pragma unroll 4
-        for (int i = T * blk + T - 1; i > T * blk; i -= 2)
-          if (i < n) {
-            const S vtm = Ar::neg(L.sup[i - 1]);
-            S num = mval(i, j);
-            if (i < n - 1) num = Ar::add(num, Ar::mul(prev, Ar::neg(L.sup[i])));
-            prev = Ar::div_vt(num, vtm, Ar::kRecip ? L.rpos[i - 1] : vtm);
-            cb[(i - 1 - T * blk) * LDB + j] = prev;
-          }
-      }
-      rr_sync<T>();
-      RR_FRESH();
-      if (!(a & 1))
-        rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
-RR_FOR(cj, 0, R) { RC(K, cj) = cb[a * LDB + b + T * cj];
-          };
-        });
-      rr_sync<T>();
-    }
-  } else {
-#pragma unroll 1
-    for (int u = 0; u < JC; ++u) {
-      const int j = tid + NT * u;
-      if (j < n) {
-        // step s of the chains: forward row 2 s + 1 from M row 2 s,
-        // backward row n - 2 - 2 s from M row n - 1 - 2 s; M of MB steps
-        // loaded together, a batch ahead
-        constexpr int MB = 4;
-        const int steps = n / 2;
-        S mf[MB], mb[MB], pfw = Ar::zero(), pbw = Ar::zero();
-        auto fetch = [&](int s0, S (&vf)[MB], S (&vb)[MB]) RR_INLINE {
+  for (int u = 0; u < JC; ++u) {
+    const int j = tid + NT * u;
+    if (j < n) {
+      // step s of the chains: forward row 2 s + 1 from M row 2 s,
+      // backward row n - 2 - 2 s from M row n - 1 - 2 s; M of MB steps
+      // loaded together, a batch ahead
+      constexpr int MB = 4;
+      const int steps = n / 2;
+      S mf[MB], mb[MB], pfw = Ar::zero(), pbw = Ar::zero();
+      auto fetch = [&](int s0, S (&vf)[MB], S (&vb)[MB]) RR_INLINE {
 #pragma unroll
-          for (int t = 0; t < MB; ++t) {
-            vf[t] = s0 + t < steps ? mval(2 * (s0 + t), j) : Ar::zero();
-            vb[t] = s0 + t < steps ? mval(n - 1 - 2 * (s0 + t), j) : Ar::zero();
-          }
-        };
-        fetch(0, mf, mb);
+        for (int t = 0; t < MB; ++t) {
+          vf[t] = s0 + t < steps ? mval(2 * (s0 + t), j) : Ar::zero();
+          vb[t] = s0 + t < steps ? mval(n - 1 - 2 * (s0 + t), j) : Ar::zero();
+        }
+      };
+      fetch(0, mf, mb);
 #pragma unroll 1
-        for (int s0 = 0; s0 < steps; s0 += MB) {
-          S nf[MB], nb[MB];
-          fetch(s0 + MB, nf, nb);
+      for (int s0 = 0; s0 < steps; s0 += MB) {
+        S nf[MB], nb[MB];
+        fetch(s0 + MB, nf, nb);
 #pragma unroll
-          for (int t = 0; t < MB; ++t) {
-            const int s = s0 + t;
-            if (s < steps) {
-              const int i = 2 * s, k = n - 1 - 2 * s;
-              const S vti = Ar::neg(L.sup[i]), vtm = Ar::neg(L.sup[k - 1]);
-              S nu = mf[t], nv = mb[t];
-              if (s > 0) {
-                nu = Ar::sub(nu, Ar::mul(pfw, Ar::neg(L.sup[i - 1])));
-                nv = Ar::add(nv, Ar::mul(pbw, Ar::neg(L.sup[k])));
-              }
-              pfw = Ar::div_negvt(nu, vti, Ar::kRecip ? L.rneg[i] : vti);
-              pbw = Ar::div_vt(nv, vtm, Ar::kRecip ? L.rpos[k - 1] : vtm);
-              if (i + 1 < j) gc[(size_t)(i + 1) * n + j] = pfw;
-              if (k - 1 < j) gc[(size_t)(k - 1) * n + j] = pbw;
+        for (int t = 0; t < MB; ++t) {
+          const int s = s0 + t;
+          if (s < steps) {
+            const int i = 2 * s, k = n - 1 - 2 * s;
+            const S vti = Ar::neg(L.sup[i]), vtm = Ar::neg(L.sup[k - 1]);
+            S nu = mf[t], nv = mb[t];
+            if (s > 0) {
+              nu = Ar::sub(nu, Ar::mul(pfw, Ar::neg(L.sup[i - 1])));
+              nv = Ar::add(nv, Ar::mul(pbw, Ar::neg(L.sup[k])));
             }
+            pfw = Ar::div_negvt(nu, vti, Ar::kRecip ? L.rneg[i] : vti);
+            pbw = Ar::div_vt(nv, vtm, Ar::kRecip ? L.rpos[k - 1] : vtm);
+            if (i + 1 < j) gc[(size_t)(i + 1) * n + j] = pfw;
+            if (k - 1 < j) gc[(size_t)(k - 1) * n + j] = pbw;
           }
+        }
 #pragma unroll
-          for (int t = 0; t < MB; ++t) {
-            mf[t] = nf[t];
-            mb[t] = nb[t];
-          }
+        for (int t = 0; t < MB; ++t) {
+          mf[t] = nf[t];
+          mb[t] = nb[t];
         }
       }
     }
-    __syncthreads();
-    RR_FRESH();
+  }
+  __syncthreads();
+  RR_FRESH();
 RR_FOR(ri, 0, R) {
 RR_FOR(cj, ri, R) {
-        const int i = a + T * ri, j = b + T * cj;
-        RC(ri, cj) = (i < j && j < n) ? gc[(size_t)i * n + j] : Ar::zero();
-      };
+      const int i = a + T * ri, j = b + T * cj;
+      RC(ri, cj) = (i < j && j < n) ? gc[(size_t)i * n + j] : Ar::zero();
     };
-  }
+  };
   RR_PHASE(8);
   // product C'(i, j) = C(i, j) + sum_{k < i} M(k, i) C(k, j), k ascending,
-  // C as solved.  Full form, every element (the small-matrix path multiplies
-  // the column-permuted C; a column's result depends on that column alone,
-  // so the permutation moves to the output): row block by row block from the
-  // last, its sums beside the registers' C, the row blocks of C broadcast
-  // through LDS.  Panel form, the upper part (the lower follows by skew
+  // C as solved, of the upper part (the lower follows by skew
   // symmetry): k block by k block, T rows of M and C from gs through LDS.
-  if constexpr (FULL) {
-    S* cb = L.vec;
+  S* mb = L.vec;
+  S* cb = L.vec + T * LDB;
 #pragma unroll 1
-    for (int ib = R - 1; ib >= 0; --ib) {
-      RR_FRESH();
-      S acc[R];
-      rr_case<0, R>(ib, [&]<int K>() RR_INLINE {
-RR_FOR(cj, 0, R) { acc[cj] = RC(K, cj);
-        };
-      });
-      const int i = a + T * ib;
+  for (int kb = 0; kb < R; ++kb) {
+    RR_FRESH();
+    // rows kb T + b of M and C, columns a + T cj
+    const int k = kb * T + b;
 #pragma unroll 1
-      for (int kb = 0; kb <= ib; ++kb) {
-        rr_case<0, R>(kb, [&]<int K>() RR_INLINE {
-RR_FOR(cj, 0, R) { cb[a * LDB + b + T * cj] = RC(K, cj);
-          };
-        });
-        rr_sync<T>();
-#pragma unroll 4
-        for (int kk = 0; kk < T; ++kk) {
-          const int k = kb * T + kk;
-          if (k < i && i < n) {
-            const S m = mval(k, i);
-RR_FOR(cj, 0, R) { acc[cj] = Ar::add(acc[cj], Ar::mul(m, cb[kk * LDB + b + T * cj]));
-            };
-          }
-        }
-        rr_sync<T>();
-      }
-      rr_case<0, R>(ib, [&]<int K>() RR_INLINE {
-RR_FOR(cj, 0, R) { RC(K, cj) = acc[cj];
-        };
-      });
+    for (int cj = kb; cj < R; ++cj) {
+      const int j = a + T * cj;
+      const bool in = k < j && j < n;
+      mb[b * LDB + j] = in ? mval(k, j) : Ar::zero();
+      cb[b * LDB + j] = in ? gc[(size_t)k * n + j] : Ar::zero();
     }
-  } else {
-    S* mb = L.vec;
-    S* cb = L.vec + T * LDB;
+    __syncthreads();
+    rr_case<0, R>(kb, [&]<int K>() RR_INLINE {
 #pragma unroll 1
-    for (int kb = 0; kb < R; ++kb) {
-      RR_FRESH();
-      // rows kb T + b of M and C, columns a + T cj
-      const int k = kb * T + b;
-#pragma unroll 1
-      for (int cj = kb; cj < R; ++cj) {
-        const int j = a + T * cj;
-        const bool in = k < j && j < n;
-        mb[b * LDB + j] = in ? mval(k, j) : Ar::zero();
-        cb[b * LDB + j] = in ? gc[(size_t)k * n + j] : Ar::zero();
-      }
-      __syncthreads();
-      rr_case<0, R>(kb, [&]<int K>() RR_INLINE {
-#pragma unroll 1
-        for (int kk = 0; kk < T; ++kk) {
-          S mi[R], cjv[R];
+      for (int kk = 0; kk < T; ++kk) {
+        S mi[R], cjv[R];
 RR_FOR(r, K, R) {
-            mi[r] = mb[kk * LDB + a + T * r];
-            cjv[r] = cb[kk * LDB + b + T * r];
-          };
+          mi[r] = mb[kk * LDB + a + T * r];
+          cjv[r] = cb[kk * LDB + b + T * r];
+        };
 RR_FOR(cj, K, R) {
 RR_FOR(ri, K + 1, cj + 1) { RC(ri, cj) = Ar::add(RC(ri, cj), Ar::mul(mi[ri], cjv[cj]));
-            };
-            if (kk < a) RC(K, cj) = Ar::add(RC(K, cj), Ar::mul(mi[K], cjv[cj]));
           };
-        }
-      });
-      __syncthreads();
-    }
+          if (kk < a) RC(K, cj) = Ar::add(RC(K, cj), Ar::mul(mi[K], cjv[cj]));
+        };
+      }
+    });
+    __syncthreads();
   }
   RR_PHASE(9);
-  // output: out(r, c) = sign * F(f(r), f(c)), F = C' (full form) or the skew
-  // completion of C' (panel form, 0 on the diagonal).  T columns of F at a
-  // time through LDS, each written as one permuted column of out.
+  // output: out(r, c) = sign * F(f(r), f(c)), F = the skew completion of C' (0
+  // on the diagonal).  T columns of F at a time through LDS, each written as
+  // one permuted column of out.
   {
     S* ob = L.vec;
 #pragma unroll 1
     for (int blk = 0; blk < R; ++blk) {
       RR_FRESH();
       rr_case<0, R>(blk, [&]<int K>() RR_INLINE {
-        if constexpr (FULL) {
-RR_FOR(ri, 0, R) { ob[b * LDB + a + T * ri] = RC(ri, K);
-          };
-        } else {
 RR_FOR(ri, 0, K) { ob[b * LDB + a + T * ri] = RC(ri, K);
-          };
-          if (a < b) {
-            ob[b * LDB + a + T * K] = RC(K, K);
-            ob[a * LDB + b + T * K] = Ar::neg(RC(K, K));
-          } else if (a == b) {
-            ob[a * LDB + a + T * K] = Ar::zero();
-          }
-RR_FOR(cj, K + 1, R) { ob[a * LDB + b + T * cj] = Ar::neg(RC(K, cj));
-          };
+        };
+        if (a < b) {
+          ob[b * LDB + a + T * K] = RC(K, K);
+          ob[a * LDB + b + T * K] = Ar::neg(RC(K, K));
+        } else if (a == b) {
+          ob[a * LDB + a + T * K] = Ar::zero();
         }
+RR_FOR(cj, K + 1, R) { ob[a * LDB + b + T * cj] = Ar::neg(RC(K, cj));
+        };
       });
       rr_sync<T>();
       const int v1 = min(T, n - T * blk);

@@ -122,11 +122,11 @@ __global__ void __launch_bounds__(256, R <= 10 ? 2 : 1) k_rr_planes(RrJob job) {
   extern __shared__ __align__(16) char lds[];
   Carver c{lds};
   int* rs = c.take<int>(job.n);
-  RrLds L = carve_rr<double, false, 16, R, false>(c, job.n);
-  double* gs = (double*)job.gs + (size_t)blockIdx.x * rr_scratch_len(false, job.n);
+  RrLds L = carve_rr<double, false, 16, R>(c, job.n);
+  double* gs = (double*)job.gs + (size_t)blockIdx.x * rr_scratch_len(job.n);
   rr_items<256>(job, rs, [&](auto src, double* out, float* out32, double sign, double& pf, int& info, bool chk,
                              bool& az) RR_INLINE {
-    rr_pfinv<16, R, false>(RrReal{}, src, job.n, out, out32, sign, gs, L, pf, info, chk, az);
+    rr_pfinv<16, R>(RrReal{}, src, job.n, out, out32, sign, gs, L, pf, info, chk, az);
   });
 }
 

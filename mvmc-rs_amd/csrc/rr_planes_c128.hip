@@ -97,10 +97,10 @@ template <int R>
 __global__ void __launch_bounds__(256, R <= 6 ? 2 : 1) k_rr_planes_c128(RrJob job) {
   extern __shared__ __align__(16) char lds[];
   Carver c{lds};
-  RrLdsT<cz> L = carve_rr<cz, true, 16, R, false>(c, job.n);
-  cz* gs = (cz*)job.gs + (size_t)blockIdx.x * rr_scratch_len(false, job.n);
+  RrLdsT<cz> L = carve_rr<cz, true, 16, R>(c, job.n);
+  cz* gs = (cz*)job.gs + (size_t)blockIdx.x * rr_scratch_len(job.n);
   rr_planes_c128<256>(job, [&](auto src, cz* out, cz& pf, int& info, bool& az) RR_INLINE {
-    rr_pfinv<16, R, false>(RrCplx{job.order}, src, job.n, out, nullptr, 1.0, gs, L, pf, info, false, az);
+    rr_pfinv<16, R>(RrCplx{job.order}, src, job.n, out, nullptr, 1.0, gs, L, pf, info, false, az);
   });
 }
 
