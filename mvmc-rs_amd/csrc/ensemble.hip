@@ -104,15 +104,22 @@ __host__ __device__ inline int hop_cap(const EnsView& v) { return 2 * v.ns + 16;
 __host__ __device__ inline bool lds_tables(const EnsView& v) { return v.nqp * v.n <= 2048 && v.nproj <= 8192; }
 // Entries of the Jastrow index table (16 bits each) and of the projection
 // parameters that the sampler keeps in LDS: those of the smaller models,
-// whose proposals wait for little else than these loads (L2: 0.3 us each).
+// whose proposals wait for little else than these loads (L2: 0.3 us each;
+// without the table a sweep of 16 to 64 sites takes 0.5 to 1.7 % longer,
+// without the parameters 0.4 to 1.3 %).  The lines are what they take: 8 KiB
+// and 2 KiB.
 __host__ __device__ inline int jast_lds(const EnsView& v) {
   return v.ns <= 64 && v.nproj > v.ngutz && lds_tables(v) ? v.ns * v.ns : 0;
 }
 __host__ __device__ inline int proj_lds(const EnsView& v) { return v.nproj <= 256 && lds_tables(v) ? v.nproj : 0; }
-// Words of the bitmap of projection parameters a proposal touches; few
-// parameters are scanned directly instead (0).
+// Words of the bitmap of projection parameters a proposal touches; fewer
+// parameters are scanned directly instead (0).  A sweep with the bitmap against
+// one without: 1.16 / 1.07 times as long (few / many electrons) at 64 sites
+// and 793 parameters, 1.15 / 1.07 at 100 and 921, 1.13 / 1.05 at 144 and
+// 1171, 1.03 / 0.96 at 64 and 1521, 0.99 / 0.97 at 100 and 1926, 0.90 / 0.89
+// at 100 and 3726.
 __host__ __device__ inline int touch_words(const EnsView& v) {
-  return v.nproj > 512 && lds_tables(v) ? (v.nproj + 31) / 32 : 0;
+  return v.nproj > 1536 && lds_tables(v) ? (v.nproj + 31) / 32 : 0;
 }
 
 __host__ __device__ inline size_t lds_bytes_sampler(const EnsView& v) {
