@@ -292,9 +292,11 @@ int mvmc_group_sample(mvmc_group* g);
  * sweep, rebuild and measurement launches, sampler LDS bytes. */
 int mvmc_group_timings(mvmc_group* g, double* timings10);
 
-/* The standalone SR entry points below (mvmc_sr_cg_apply, mvmc_sr_gram_real,
- * mvmc_sr_cholesky_solve, mvmc_sr_cg_solve) keep one device workspace per process: calls that overlap from several host threads
- * race; serialise them (the ensemble's own SR uses per-handle state). */
+/* Of the standalone SR entry points below, mvmc_sr_cg_apply and
+ * mvmc_sr_cg_solve keep a device workspace per process each: calls of one of
+ * them that overlap from several host threads race; serialise them (the
+ * ensemble's own SR uses per-handle state).  mvmc_sr_cg_solve refuses
+ * max_it < 0. */
 
 /* SrStages::cg_local_product (crates/mvmc-core/src/sr_backend.rs:518-598),
  * one product of the sampled operator on device operands:

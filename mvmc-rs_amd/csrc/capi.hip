@@ -456,7 +456,8 @@ struct mvmc_ens {
   hipStream_t st = nullptr;
   int grid_samp = 0, grid_meas = 0, grid_rebuild = 0, slots = 0;
   // rebuild-kernel variants: 2, plane by plane (rr_planes.hip), wherever it
-  // covers n (it measured 2-4 times faster than the others); beyond, walker
+  // covers n (4096 planes: 4.5 times the panel-delayed kernel's rate at n = 64,
+  // 2.2 to 2.5 from 98 to 160, 1.7 at 192, 1.6 at 224); beyond, walker
   // by walker (0: 3 workgroups per CU, 8-column close batches; 1: 2 per CU,
   // 16 columns), tuned on the first well-filled launches: rb_variant -1
   // while measuring, then the faster one

@@ -233,7 +233,8 @@ __device__ inline double ip_of_l(const double* qpw, const double* pf, int nqp) {
 // the bus: the 16 x 16 lattice's Slater table is 16.8 MB).
 // ---------------------------------------------------------------------------
 // Slater table (update_slater_elm, slater_update.rs:17-126), a thread per
-// (plane, site, site): its four spin blocks.
+// (plane, site, site): its four spin blocks.  Every site of tsite is one of
+// the model's (create_impl refuses a map with holes).
 __global__ void k_slater_table(EnsView v, const double* orb, double* table) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const int ns = v.ns, n2 = v.n2;
@@ -903,7 +904,8 @@ __device__ __forceinline__ void stream_tiles(T* planes, int n, int nqp, const ty
   const int qo = tid / LP, jl = tid % LP;
   const int span = LP * CPL;  // columns per group
   // rows past the end of a plane are loaded (from the next plane, or 0 past
-  // the last by the buffer's range) and not used
+  // the last: the buffer's range check counts the scalar offset too) and not
+  // used
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(planes, 0, (int)((size_t)nqp * nn * ES), BUF_WORD3);
   const int rowb = n * ES;

@@ -21,9 +21,10 @@
 //     save: n = 224 0.6x; 4 waves, T = 16, it is);
 //   - the block of the step's column picks one of R code bodies whose slots
 //     and bounds are compile-time constants (no per-element tests inside).
-// Measured: 2048 planes of n = 144 7470 -> 4000 us, 1024 of n = 224
-// 8580 -> 7200 us (before: 1024 threads a plane, two barriers a step),
-// complex 768 of n = 144 4080 -> 3190 us.
+// Measured: 2048 planes of n = 144 7470 -> 3320 us (before: the panel-delayed
+// kernel), 1024 of n = 224 8580 -> 7200 us, complex 768 of n = 144 4080 ->
+// 3190 us and of n = 160 4720 -> 4260 us (before: 1024 threads a plane, two
+// barriers a step).
 #pragma once
 #include "common.h"
 

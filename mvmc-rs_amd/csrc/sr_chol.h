@@ -20,7 +20,7 @@
 //  - L y = b rides along with the diagonal tiles; L^T x = y takes a launch
 //    per 256 columns, every workgroup solving that block itself and taking
 //    it from its own 64 columns.
-// n = 1111: 0.56 ms (25 launches; 20 us a panel, 10 of them the 64 pivots)
+// n = 1111: 0.56 ms (24 launches; 20 us a panel, 10 of them the 64 pivots)
 // where a factorisation and two triangular solves by the vendor's solver took
 // 3.4; n = 5000: 4.4 ms.  Residuals are 0.6 of the vendor's.
 // From CH_PRE trailing tile rows on, forming L_I per tile costs more than a

@@ -217,7 +217,7 @@ class Ensemble:
         return info.value
 
     def sr_direct(self):
-        """Direct SR (DSYRK + Cholesky) on the last measurement; 1 if skipped."""
+        """Direct SR (Gram on the matrix cores + Cholesky) on the last measurement; 1 if skipped."""
         sk = ctypes.c_int(0)
         _check(lib().mvmc_ens_sr_direct(self.h, ctypes.byref(sk)))
         return sk.value
